@@ -1358,9 +1358,13 @@ static void mark_nprev_valid(ibpm_batch* B) {
     B->old_saved = true;
     for (int i = 0; i < B->nsub; ++i) {
         for (auto& o : B->h_fops[i]) o.nprev_valid = o.sfd_valid = 1;
-        (void)hipMemcpy(B->d_fops[i], B->h_fops[i].data(), sizeof(FlowOps) * B->h_fops[i].size(),
-                        hipMemcpyHostToDevice);
+        // on the batch's own stream: a copy on the legacy stream would reach into
+        // every other blocking stream, and a batch on another context may be
+        // capturing its step there
+        (void)hipMemcpyAsync(B->d_fops[i], B->h_fops[i].data(), sizeof(FlowOps) * B->h_fops[i].size(),
+                             hipMemcpyHostToDevice, B->ctx->c.stream);
     }
+    (void)hipStreamSynchronize(B->ctx->c.stream);
 }
 
 // The local Helmholtz path of substep i's M applications (k_fs_helm).  The
