@@ -12,7 +12,9 @@ OBJ = os.path.join(HERE, "_build")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("IBPM_OFFLOAD_ARCH", "gfx950")
 
-DEVICE_SOURCES = ["elliptic.hip", "ops.hip", "learn.hip", "scratch.hip"]
+# dst_f64.hip compiles in parts (IBPM_DST_PART), a share of the transform lengths each.
+DST_PARTS = ["dst_f64.hip:%d" % k for k in range(8)]
+DEVICE_SOURCES = DST_PARTS + ["elliptic.hip", "ops.hip", "learn.hip", "scratch.hip"]
 HOST_SOURCES = ["engine.cpp", "geometry.cpp", "restart.cpp"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]
 # Packed FP32 instructions are kept out of every code object.
@@ -21,7 +23,9 @@ DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang
 
 def _compile(src, defines=(), obj_dir=OBJ):
     os.makedirs(obj_dir, exist_ok=True)
-    obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
+    src, _, part = src.partition(":")
+    obj = os.path.join(obj_dir, os.path.splitext(src)[0] + part + ".o")
+    defines = list(defines) + (["-DIBPM_DST_PART=" + part] if part else [])
     path = os.path.join(CSRC, src)
     if src.endswith(".hip"):
         cmd = [HIPCC] + COMMON + DEVICE_FLAGS + list(defines) + ["-c", path, "-o", obj]
@@ -38,7 +42,7 @@ def _compile(src, defines=(), obj_dir=OBJ):
 def build(verbose=False, defines=(), out=OUT, obj_dir=OBJ):
     """Compiles every source (always) and links libibpm_gpu.so (or `out`,
     with extra -D `defines`, for a tuning variant)."""
-    with concurrent.futures.ThreadPoolExecutor(max_workers=4) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=8) as ex:
         results = list(ex.map(lambda s: _compile(s, defines, obj_dir), DEVICE_SOURCES + HOST_SOURCES))
     objs = [o for o, _ in results]
     for _, msgs in results:

@@ -39,6 +39,10 @@ struct FftPlan {
     int nst;        // number of Stockham stages
     int rad[kMaxStages];
     const double2* tw;   // tw[k] = exp(-2 pi i k / M), k < M
+    // tables of n = N + 1 cells: cos(pi i / n) and 2 sin(pi i / n), i = 1..n-1
+    // (then zeros to t1_ld(N)), and 2 sin(pi l j / n) at j = n/4 and n/4 + n/2,
+    // the columns of a coarse level that the finer level's edge runs along
+    const double *cosn, *sin1, *ring;
     const double2* tw16; // M = 1024, 2048: the second radix-16 stage's w^((M/256) jm r) at 16 r + jm (r, jm < 16)
 };
 
@@ -46,7 +50,7 @@ struct FftPlan {
 struct EllJob {
     int nx, ny;              // cells; rows i=1..nx-1, columns j=1..ny-1
     int lev, ngrid;
-    int kind;                // 0 Poisson, 1 Helmholtz
+    int kind;                // 0 Poisson, 1 Helmholtz, 2 forward transform alone (passes 1 and 2, to u)
     int epilogue;            // 0: u = v ; 1: u = W - v
     double in_scale;         // multiplies the right-hand side (+1 or -1)
     double bc_coef;          // 1/dx^2 (Poisson) or alpha/dx^2 (Helmholtz)
@@ -55,39 +59,35 @@ struct EllJob {
     const double* R;         // level slice of the coarsified rhs (central region), lev >= 1
     const double* uc;        // level slice lev+1 of the solution (BC source), lev < ngrid-1
     const double* bcring;    // explicit BC ring 2(nx+ny) instead of uc (single-level API)
-    double* T1;              // scratch (ny-1) rows of nx-1 values, row stride ld1
-    double* T2;              // scratch (nx-1) rows of ny-1 values, row stride ld2
-    int ld1, ld2;            // >= nx-1, ny-1; padded (t1_ld) where the scratch is the library's own
+    double* T1;              // scratch T: (nx-1) rows of ny-1 values, row stride ld1 = t1_ld(ny-1)
+    double* T2;              // the GEMM-DST's second pair of planes (null where it does not run)
+    int ld1;
     double* u;               // level slice of the solution
     double* u2;              // null, or a second output of the same values (pass 3)
     const double* W;         // epilogue 1 operand (level slice)
     double* vside;           // epilogue solves, levels >= 1: v (before the epilogue) stored at
-                             // the points the next finer level's getBC reads (level slice)
-    const double* cosx;      // cos(pi i / nx), i = 1..nx-1
-    const double* cosy;      // cos(pi j / ny), j = 1..ny-1
+                             // the points the next finer level's getBC reads (level slice; FP32
+                             // and GEMM transforms, whose finer levels read u itself)
     FftPlan pj;              // transform along j (length ny-1)
     FftPlan pi;              // transform along i (length nx-1)
     const double* skip;      // null, or the flow's solver flags (see skipped())
-    // Pass 3 over part of the level (the register-held pass 3 only): row pairs
-    // in [full_lo, full_hi] and pairs fq0, fq1 are transformed; of the other
-    // rows, those in [ring_lo, ring_hi] (1-based) get u at columns rj0 and rj1
-    // alone, by direct sums against ringsin (2 sin(pi l j / ny), l = 1..ny-1,
-    // for j = rj0 then rj1); the rest is not written.
-    int full_lo, full_hi, fq0, fq1, ring_lo, ring_hi, rj0, rj1;
-    const double* ringsin;
-    // Pass 1 (register-held): rows i outside [sup_lo, sup_hi] (1-based) have
-    // no interior right-hand side; a workgroup whose rows are all such rows,
-    // none of them 1 or nx-1, writes their transform in closed form from the
-    // two boundary terms, sin1[k - 1] = 2 sin(pi k / ny) (null: never).
+    // Boundary values in pass 2's space (null: zero), with c = bc_coef of this
+    // level: 2 (nx-1) doubles, for i = 1..nx-1 the pair c (bottom_i + top_i),
+    // c (bottom_i - top_i), padded to 2 t1_ld(nx-1); then c times the DST-I of
+    // left, and of right, t1_ld(ny-1) doubles each (a pad column holds 0).
+    const double* bcv;
+    double* bc_out;          // the next finer level's bcv (its own for bcring), null on level 0
+    double bc_out_coef;      // that level's bc_coef
+    // Passes over part of the level.  Pass 1 runs, and pass 2 reads, rows i in
+    // [sup_lo, sup_hi] (1-based): the right-hand side is zero on the others.
+    // In the central region R is read inside the box rb_* only and taken as 0
+    // outside it, where the solve's coarsify chain, run over the box alone,
+    // left other solves' values.  Pass 2 writes rows [t2_lo, t2_hi] (0-based),
+    // those read afterwards; pass 3 runs row pairs [full_lo, full_hi].
     int sup_lo, sup_hi;
-    const double* sin1;
-    // Pass 1 (register-held): in the central region R is read inside this box
-    // only and taken as 0 outside it, where the solve's coarsify chain, run
-    // over the box alone, left other solves' values.
     int rb_i0, rb_i1, rb_j0, rb_j1;
-    // Pass 2 (register-held): rows of T2 (0-based i) that pass 3 reads; the
-    // others are not written.
     int t2_lo, t2_hi;
+    int full_lo, full_hi;
 };
 
 // Local solve of A u = r, A = 1 + alpha Lap (the force solve's A^-1 of one
@@ -136,10 +136,11 @@ __device__ inline bool skipped(const double* flags) {
 
 __host__ __device__ inline int nx_ext(int nx) { return nx / 4; }   // Grid.h:89-91, zero shift
 
-// Row stride of the transposed scratch rows of n values: a multiple of 8
-// doubles, so the 64-byte pieces that the register-held pass 1 writes per
-// column start on 64-byte boundaries (one write request each, not two).
-inline int t1_ld(int n) { return (n + 7) & ~7; }
+// Row stride of the scratch T with rows of n values: a multiple of 8 doubles,
+// so the 64-byte pieces (4 column pairs of a row) that the register-held pass 2
+// reads and writes start on 64-byte boundaries, and the last pair of an odd n
+// has a pad column to read.
+__host__ __device__ constexpr int t1_ld(int n) { return (n + 7) & ~7; }
 
 __device__ inline long sidx(int nx, int ny, int i, int j) {   // within a level slice
     return (long)(i - 1) * (ny - 1) + (j - 1);

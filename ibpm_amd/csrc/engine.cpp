@@ -163,10 +163,13 @@ static int plan_shape(int N, FftPlan* P) {
 // Whether a plan of FFT length M has the second-stage table tw16.
 static bool plan_has_tw16(int M) { return M == 1024 || M == 2048; }
 
-// Host values of a plan's twiddle tables: tw (M entries) and, where
-// plan_has_tw16, t16 (256 entries).
-static void plan_tables(int M, double2* tw, double2* t16) {
-    const double twopi = 8.0 * std::atan(1.0);
+// Host values of a plan's tables: tw (M entries), t16 (256 entries, where
+// plan_has_tw16), and the real tables cosn, sin1 (t1_ld(N) each) and ring
+// (2 N) one after another (plan_reals(N) doubles); see FftPlan.
+static size_t plan_reals(int N) { return 2 * (size_t)t1_ld(N) + 2 * (size_t)N; }
+
+static void plan_tables(int M, double2* tw, double2* t16, double* reals) {
+    const double twopi = 8.0 * std::atan(1.0), pi = 4. * std::atan(1.0);
     for (int k = 0; k < M; ++k) {
         const double a = -twopi * (double)k / (double)M;
         tw[k] = make_double2(std::cos(a), std::sin(a));
@@ -176,6 +179,23 @@ static void plan_tables(int M, double2* tw, double2* t16) {
         for (int r = 0; r < 16; ++r)
             for (int jm = 0; jm < 16; ++jm) t16[16 * r + jm] = tw[(tstep * jm * r) % M];
     }
+    const int n = M / 2, N = n - 1, e = nx_ext(n);
+    double *cosn = reals, *sin1 = cosn + t1_ld(N), *ring = sin1 + t1_ld(N);
+    for (int i = N; i < t1_ld(N); ++i) cosn[i] = sin1[i] = 0.0;
+    for (int i = 1; i < n; ++i) {
+        cosn[i - 1] = std::cos((pi * i) / n);   // EllipticSolver2d.cc:47-48
+        sin1[i - 1] = 2. * std::sin(pi * i / n);
+        ring[i - 1] = 2. * std::sin(pi * i * e / n);
+        ring[N + i - 1] = 2. * std::sin(pi * i * (e + n / 2) / n);
+    }
+}
+
+static void plan_pointers(FftPlan& P, const double2* tw, const double2* t16, const double* reals) {
+    P.tw = tw;
+    P.tw16 = plan_has_tw16(P.M) ? t16 : nullptr;
+    P.cosn = reals;
+    P.sin1 = reals + t1_ld(P.N);
+    P.ring = P.sin1 + t1_ld(P.N);
 }
 
 static int get_plan(Ctx* c, int N, FftPlan* out) {
@@ -183,25 +203,27 @@ static int get_plan(Ctx* c, int N, FftPlan* out) {
     if (it != c->plans.end()) { *out = it->second; return 0; }
     FftPlan P{};
     CKR(plan_shape(N, &P));
-    std::vector<double2> tw(P.M), t16(256);
-    plan_tables(P.M, tw.data(), t16.data());
-    double2* d = nullptr;
-    CKR(c->mem.alloc(&d, P.M));
-    CK(hipMemcpy(d, tw.data(), sizeof(double2) * P.M, hipMemcpyHostToDevice));
-    P.tw = d;
-    P.tw16 = nullptr;
-    if (plan_has_tw16(P.M)) {
-        double2* d16 = nullptr;
-        CKR(c->mem.alloc(&d16, 256));
-        CK(hipMemcpy(d16, t16.data(), sizeof(double2) * 256, hipMemcpyHostToDevice));
-        P.tw16 = d16;
-    }
+    // tw, t16 and the reals in one upload
+    std::vector<double> h(2 * (size_t)P.M + 512 + plan_reals(N));
+    double2 *tw = (double2*)h.data(), *t16 = tw + P.M;
+    plan_tables(P.M, tw, t16, (double*)(t16 + 256));
+    double* d = nullptr;
+    CKR(c->mem.alloc(&d, h.size()));
+    CK(hipMemcpy(d, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
+    plan_pointers(P, (double2*)d, (double2*)d + P.M, d + 2 * (size_t)P.M + 512);
     c->plans[N] = P;
     *out = P;
     return 0;
 }
 
 // ------------------------------------------------------------ solve plans
+// Most bytes of T, summed over the levels of every flow of a batch, for which
+// T of every level is kept and passes 1 and 3 run over all levels at once:
+// half of the 256 MB Infinity Cache, so that pass 2 still finds T there.  Past
+// it the launches are long enough by themselves, and one level's T, reused
+// level after level, stays in the cache.
+constexpr double kAllLevelBytes = 128e6;
+
 // One multi-domain solve of one flow.
 struct SolveSpec {
     int nx, ny, L;
@@ -211,13 +233,13 @@ struct SolveSpec {
     const double* f;
     double* u;
     double* R;             // coarsify buffer (L levels)
-    double* T1;
+    double* T1;            // scratch rows of one level, or of every level, tstride apart
+    long tstride;          // 0: one level's
     double* T2;
+    double* bcv;           // boundary values of levels 0..L-2 (bcv_size each; of level 0 with bcring)
     double in_scale;
     int epilogue;
     const double* W;
-    const double* cosx;
-    const double* cosy;
     const double* bcring;  // single-level explicit boundary values (L == 1 only)
     const double* skip;    // null, or the flow's force-solve flags
     double* vside;         // epilogue solves: side buffer (L levels) for the BC values of v
@@ -232,13 +254,13 @@ struct SolveSpec {
 enum KClass { K_PASS1, K_PASS2, K_PASS3, K_COARSIFY, K_VEL, K_CROSS, K_RHS, K_CURLQ, K_INTERP,
               K_SMEAR, K_MINV, K_CG, K_FORCES, K_CLEAR, K_FSPASS1, K_FSPASS2, K_FSPASS3, K_FSCOARSIFY,
               K_FSHELM, K_HELM, K_PASS32_1, K_PASS32_2, K_PASS32_3, K_FSPASS32_1, K_FSPASS32_2,
-              K_FSPASS32_3, K_GEMM, K_PCASM, K_PCNS, K_NCLASS };
+              K_FSPASS32_3, K_GEMM, K_PCASM, K_PCNS, K_BC, K_FSBC, K_NCLASS };
 static const char* kclass_names[K_NCLASS] = {"ell_pass1", "ell_pass2", "ell_pass3", "coarsify", "vel",
                                              "cross", "rhs", "curl_q", "interp", "smear_curl", "minv",
                                              "cg", "forces", "clear_nodes", "fs_pass1", "fs_pass2",
                                              "fs_pass3", "fs_coarsify", "fs_helm", "helm", "ell32_pass1",
                                              "ell32_pass2", "ell32_pass3", "fs32_pass1", "fs32_pass2",
-                                             "fs32_pass3", "ell_gemm", "pc_assemble", "pc_refresh"};
+                                             "fs32_pass3", "ell_gemm", "pc_assemble", "pc_refresh", "ell_bc", "fs_bc"};
 struct Probe {
     struct Rec { int cls; hipEvent_t a, b; double bytes; };
     std::vector<Rec> recs;
@@ -265,23 +287,23 @@ static void timed(Probe* pr, int cls, double bytes, hipStream_t s, Fn fn) {
     pr->recs.push_back(r);
 }
 
-// The jobs of one level step that share their transform lengths (one launch
-// per pass).
-// Passes 1 and 3 over the whole level (EllJob's partial-pass fields off).
+// The whole level in every pass (EllJob's partial-pass fields off).
 static void whole_level(EllJob& J) {
-    J.full_lo = 0; J.full_hi = INT_MAX; J.fq0 = J.fq1 = -1;
-    J.ring_lo = 1; J.ring_hi = 0; J.rj0 = J.rj1 = 1; J.ringsin = nullptr;
-    J.sup_lo = 1; J.sup_hi = INT_MAX; J.sin1 = nullptr;
+    J.full_lo = 0; J.full_hi = INT_MAX;
+    J.sup_lo = 1; J.sup_hi = J.nx - 1;
     J.rb_i0 = 0; J.rb_i1 = INT_MAX; J.rb_j0 = 0; J.rb_j1 = INT_MAX;
     J.t2_lo = 0; J.t2_hi = INT_MAX;
 }
+
+// Doubles of one level's boundary values (EllJob::bcv).
+static size_t bcv_size(int nx, int ny) { return 2 * (size_t)(t1_ld(nx - 1) + t1_ld(ny - 1)); }
 
 // The job of level lev of one solve (every field but the two FFT plans).
 static void fill_ell_job(const SolveSpec& s, int lev, EllJob& J) {
     const long ns = (long)(s.nx - 1) * (s.ny - 1);
     const double dxl = s.dx * (1 << lev);
-    whole_level(J);
     J.nx = s.nx; J.ny = s.ny; J.lev = lev; J.ngrid = s.L;
+    whole_level(J);
     J.kind = s.kind; J.epilogue = s.epilogue; J.in_scale = s.in_scale;
     J.alpha = s.alpha;
     J.bydx2 = 1. / (dxl * dxl);                                  // EllipticSolver2d.cc:44
@@ -295,48 +317,57 @@ static void fill_ell_job(const SolveSpec& s, int lev, EllJob& J) {
     J.uc = (lev < s.L - 1) ? bcsrc + (lev + 1) * ns : nullptr;
     J.vside = (s.vside && lev >= 1) ? s.vside + lev * ns : nullptr;
     J.bcring = (s.L == 1) ? s.bcring : nullptr;
-    J.T1 = s.T1; J.T2 = s.T2;
-    J.ld1 = t1_ld(s.nx - 1); J.ld2 = t1_ld(s.ny - 1);   // the scratch is sized for the padding
+    J.T1 = s.T1 + lev * s.tstride; J.T2 = s.T2;
+    const size_t nbc = bcv_size(s.nx, s.ny);
+    if (J.bcring) {
+        J.bcv = J.bc_out = s.bcv;
+        J.bc_out_coef = J.bc_coef;
+    } else {
+        J.bcv = lev < s.L - 1 ? s.bcv + lev * nbc : nullptr;
+        J.bc_out = lev >= 1 ? s.bcv + (lev - 1) * nbc : nullptr;
+        J.bc_out_coef = 4 * J.bc_coef;   // of the next finer level: dx halves
+    }
+    J.ld1 = t1_ld(s.ny - 1);   // the scratch is sized for the padding
     J.u = s.u + lev * ns;
     J.u2 = s.u2 ? s.u2 + lev * ns : nullptr;
     J.W = s.W ? s.W + lev * ns : nullptr;
-    J.cosx = s.cosx; J.cosy = s.cosy;
     J.skip = s.skip;
 }
 
-// Launch shape of the three passes of a single-job group: registers or LDS,
-// workgroups and dynamic LDS bytes per pass (as build_solve_plan sizes them).
-static void pass_shape(const EllJob& J, bool regs[3], int maxb[3], int lds[3]) {
-    for (int k = 0; k < 3; ++k) {
-        const long pairs = (k == 1 ? J.ny : J.nx) / 2;
-        regs[k] = pass_in_registers(k == 1 ? J.pi.M : J.pj.M, pairs);
-        maxb[k] = blocks_for_pass(J, k + 1, regs[k]);
-        lds[k] = lds_for_pass(J, k + 1, regs[k]);
-    }
-}
-
+// The jobs of one level step that share their transform lengths (one launch
+// per pass).
 struct PassGroup {
     EllJob* d = nullptr;
     int n = 0;
     int mj = 0, mi = 0;                             // FFT lengths along j (passes 1, 3) and i (pass 2)
-    int maxb[3] = {0, 0, 0}, lds[3] = {0, 0, 0};
+    int maxb[4] = {0, 0, 0, 0};                     // workgroups of passes 1..3 and bc
     bool regs[3] = {false, false, false};           // pass_in_registers per pass
-    bool fp32 = false;                              // FP32 transforms (LDS passes, k32_*)
+    bool p3 = true, bc = false;                     // any job runs pass 3 / makes boundary values
+    int maxb32[3] = {0, 0, 0}, lds32[3] = {0, 0, 0};   // the FP32 passes' launch shape
     bool gemm = false;                              // split-BF16 GEMM-DST on MFMA (launch_gemm_dst)
     const __bf16 *Sh = nullptr, *Sl = nullptr;      // its sine matrix
     int gemm_n = 0;                                 // its N (square levels only)
     double t_radix_us = 0, t_gemm_us = 0;           // autotuner timings of the group (0: not timed)
-    int maxb64[3] = {0, 0, 0}, lds64[3] = {0, 0, 0};   // the FP64 launch shape, kept for switching back
-    bool regs64[3] = {false, false, false};
     std::vector<int> jflow;                         // flow of each job
     std::vector<double> jbytes[3];                  // per pass: 16 B per point (one read + one write),
     double bytes[3] = {0, 0, 0};                    // less where a pass is restricted (pass_bytes)
     std::vector<EllJob> h;                          // host copy of the jobs
 };
 
+// The groups of every step with the same lengths, their jobs one array: a
+// pass over all levels is one launch per entry.
+struct LenGroup {
+    EllJob* d = nullptr;
+    int n = 0, mj = 0, mi = 0;
+    std::vector<std::pair<int, int>> member;        // (step, group)
+};
+
 struct SolvePlan {
     bool force_solve = false;                       // M application (k_fs_* kernels)
     bool fp32 = false;                              // every group's transforms in FP32 (set_plan_fp32)
+    bool all_levels = false;                        // T of every level: passes 1 and 3 over all levels at once
+    bool given_bc = false;                          // explicit boundary values (one level)
+    std::vector<LenGroup> lens;
     int nlev = 0;                                   // max L over flows
     std::vector<std::vector<int>> cflow;            // flow of each coarsify job, per level
     std::vector<std::vector<double>> cjbytes;
@@ -354,6 +385,7 @@ static int build_solve_plan(Ctx* c, DevMem& mem, const std::vector<SolveSpec>& s
     P.cj_rows.assign(P.nlev, 0);
     P.cflow.assign(P.nlev, {});
     P.cjbytes.assign(P.nlev, {});
+    P.lens.clear();
     for (int lev = 1; lev < P.nlev; ++lev) {
         std::vector<CoarsifyJob> jobs;
         int pts = 0;
@@ -409,64 +441,69 @@ static int build_solve_plan(Ctx* c, DevMem& mem, const std::vector<SolveSpec>& s
                 long pairs = 0;
                 for (auto& J : jobs) pairs += (k == 1 ? J.ny : J.nx) / 2;   // ceil(rows / 2)
                 G.regs[k] = pass_in_registers(k == 1 ? G.mi : G.mj, pairs);
-                for (auto& J : jobs) {
-                    G.maxb[k] = std::max(G.maxb[k], blocks_for_pass(J, k + 1, G.regs[k]));
-                    G.lds[k] = std::max(G.lds[k], lds_for_pass(J, k + 1, G.regs[k]));
+            }
+            for (auto& J : jobs) {
+                for (int k = 0; k < 4; ++k)
+                    G.maxb[k] = std::max(G.maxb[k], blocks_for_pass(J, k + 1, k < 3 && G.regs[k]));
+                for (int k = 0; k < 3; ++k) {
+                    G.maxb32[k] = std::max(G.maxb32[k], blocks_for_pass32(J, k + 1));
+                    G.lds32[k] = std::max(G.lds32[k], lds_for_pass32(J, k + 1));
                 }
+                G.bc = G.bc || J.bc_out;
             }
-            for (int k = 0; k < 3; ++k) {
-                G.regs64[k] = G.regs[k];
-                G.maxb64[k] = G.maxb[k];
-                G.lds64[k] = G.lds[k];
-            }
-            CKR(mem.alloc(&G.d, jobs.size()));
-            CK(hipMemcpy(G.d, jobs.data(), sizeof(EllJob) * jobs.size(), hipMemcpyHostToDevice));
             G.n = (int)jobs.size();
             G.h = jobs;
+            size_t q = 0;
+            while (q < P.lens.size() && !(P.lens[q].mj == G.mj && P.lens[q].mi == G.mi)) ++q;
+            if (q == P.lens.size()) {
+                P.lens.emplace_back();
+                P.lens[q].mj = G.mj;
+                P.lens[q].mi = G.mi;
+            }
+            P.lens[q].n += G.n;
+            P.lens[q].member.push_back({st, (int)g});
         }
+    }
+    for (LenGroup& Q : P.lens) {
+        CKR(mem.alloc(&Q.d, Q.n));
+        std::vector<EllJob> jobs;
+        for (auto& m : Q.member) {
+            PassGroup& G = P.steps[m.first][m.second];
+            G.d = Q.d + jobs.size();
+            jobs.insert(jobs.end(), G.h.begin(), G.h.end());
+        }
+        CK(hipMemcpy(Q.d, jobs.data(), sizeof(EllJob) * jobs.size(), hipMemcpyHostToDevice));
+    }
+    P.all_levels = true;
+    for (auto& s : specs) {
+        P.all_levels = P.all_levels && s.tstride > 0;
+        P.given_bc = P.given_bc || s.bcring;
     }
     return 0;
 }
 
-static void group_bytes(PassGroup& G);
+static void group_bytes(PassGroup& G, bool fp32);
 
-// Switches a plan's transforms between FP64 (the register-held or LDS
-// passes chosen at build) and FP32 (LDS passes over every row: the partial-
-// pass restrictions of register-held passes do not apply, so an FP32 pass
-// computes a superset of what the FP64 one writes).
+// Switches a plan's transforms between FP64 and FP32 (LDS passes over every
+// row: the partial-pass restrictions do not apply, so an FP32 pass computes a
+// superset of what the FP64 one writes).
 static void set_plan_fp32(SolvePlan& P, bool on) {
     P.fp32 = on;
     for (auto& step : P.steps)
         for (auto& G : step) {
-            G.fp32 = on;
             G.gemm = false;
-            for (int k = 0; k < 3; ++k) {
-                if (!on) {
-                    G.regs[k] = G.regs64[k];
-                    G.maxb[k] = G.maxb64[k];
-                    G.lds[k] = G.lds64[k];
-                    continue;
-                }
-                G.regs[k] = false;
-                G.maxb[k] = 0;
-                G.lds[k] = 0;
-                for (auto& J : G.h) {
-                    G.maxb[k] = std::max(G.maxb[k], blocks_for_pass(J, k + 1, false));
-                    G.lds[k] = std::max(G.lds[k], lds_for_pass32(J, k + 1));
-                }
-            }
-            if (!G.jbytes[0].empty()) group_bytes(G);
+            if (!G.jbytes[0].empty()) group_bytes(G, on);
         }
 }
 
 // Whether a group can take the GEMM-DST: square levels of N <= 511 whose
-// transposed scratch holds the two bf16 plane pairs (2 Np^2 each).
+// scratch T holds the two bf16 plane pairs (2 Np^2 each).
 static bool gemm_eligible(const PassGroup& G) {
     if (G.h.empty()) return false;
     for (const EllJob& J : G.h) {
         const int N = J.nx - 1, Np = gemm_np_host(N);
         if (J.nx != J.ny || N > 511 || N != G.h[0].nx - 1) return false;
-        if (4.0 * Np * Np > 8.0 * (double)(J.ny - 1) * t1_ld(J.nx - 1)) return false;
+        if (4.0 * Np * Np > 8.0 * (double)(J.nx - 1) * t1_ld(J.ny - 1)) return false;
     }
     return true;
 }
@@ -499,7 +536,7 @@ static int tune_plan_gemm(Ctx* c, DevMem& mem, SolvePlan& P, int mode) {
             CK(hipMemcpy(d, jobs.data(), sizeof(EllJob) * jobs.size(), hipMemcpyHostToDevice));
             auto radix = [&] {
                 for (int pass = 1; pass <= 3; ++pass)
-                    launch_ell_pass32(pass, d, G.n, G.maxb[pass - 1], G.lds[pass - 1], s, P.force_solve,
+                    launch_ell_pass32(pass, d, G.n, G.maxb32[pass - 1], G.lds32[pass - 1], s, P.force_solve,
                                       pass == 2 ? G.mi : G.mj);
             };
             auto gemm = [&] { launch_gemm_dst(d, G.n, N, G.Sh, G.Sl, s); };
@@ -546,56 +583,86 @@ static void run_coarsify(const SolvePlan& P, hipStream_t s, Probe* pr, const std
               [&] { launch_coarsify(P.cj[lev], P.cj_n[lev], P.cj_rows[lev], s, fs); });
 }
 
-// active (probe only): flows whose jobs do work; the others are skipped by
-// their flags, so their bytes are not counted.
-// coarsify = false: the caller has built the coarse right-hand sides.
-static void run_solve(const SolvePlan& P, hipStream_t s, Probe* pr = nullptr,
-                      const std::vector<char>* active = nullptr, bool coarsify = true) {
-    auto sum = [&](const std::vector<int>& fl, const std::vector<double>& by, double all) {
-        if (!active) return all;
-        double b = 0;
-        for (size_t j = 0; j < fl.size(); ++j)
-            if ((*active)[fl[j]]) b += by[j];
-        return b;
-    };
+// The solve in reduced precision: level by level, every pass over the whole
+// level, the finer level's boundary values read from u (or vside).
+static void run_solve_reduced(const SolvePlan& P, hipStream_t s, Probe* pr, const std::vector<char>* active) {
     const bool fs = P.force_solve;
-    if (coarsify) run_coarsify(P, s, pr, active);
     for (int st = 0; st < P.nlev; ++st)
         for (const PassGroup& G : P.steps[st]) {
+            double by[4] = {0, 0, 0, 0};
+            if (pr)
+                for (size_t j = 0; j < G.jflow.size(); ++j)
+                    if (!active || (*active)[G.jflow[j]]) {
+                        for (int q = 0; q < 3; ++q) by[q] += G.jbytes[q][j];
+                        by[3] += 48.0 * (G.h[j].nx - 1) * (G.h[j].ny - 1);
+                    }
             if (G.gemm) {
-                double by = 0;
-                if (pr)
-                    for (size_t j = 0; j < G.jflow.size(); ++j)
-                        if (!active || (*active)[G.jflow[j]]) by += 48.0 * (G.h[j].nx - 1) * (G.h[j].ny - 1);
-                timed(pr, K_GEMM, by, s, [&] { launch_gemm_dst(G.d, G.n, G.gemm_n, G.Sh, G.Sl, s); });
+                timed(pr, K_GEMM, by[3], s, [&] { launch_gemm_dst(G.d, G.n, G.gemm_n, G.Sh, G.Sl, s); });
                 continue;
             }
-            for (int pass = 1; pass <= 3; ++pass) {
-                const int cls = G.fp32 ? (fs ? K_FSPASS32_1 : K_PASS32_1) : (fs ? K_FSPASS1 : K_PASS1);
-                timed(pr, cls + pass - 1, pr ? sum(G.jflow, G.jbytes[pass - 1], G.bytes[pass - 1]) : 0, s, [&] {
-                    if (G.fp32)
-                        launch_ell_pass32(pass, G.d, G.n, G.maxb[pass - 1], G.lds[pass - 1], s, fs,
-                                          pass == 2 ? G.mi : G.mj);
-                    else
-                        launch_ell_pass(pass, G.d, G.n, G.maxb[pass - 1], G.lds[pass - 1], s, fs,
-                                        pass == 2 ? G.mi : G.mj, G.regs[pass - 1]);
+            for (int pass = 1; pass <= 3; ++pass)
+                timed(pr, (fs ? K_FSPASS32_1 : K_PASS32_1) + pass - 1, by[pass - 1], s, [&] {
+                    launch_ell_pass32(pass, G.d, G.n, G.maxb32[pass - 1], G.lds32[pass - 1], s, fs,
+                                      pass == 2 ? G.mi : G.mj);
                 });
-            }
         }
 }
 
-// cos(pi i / n), i = 1..n-1 (EllipticSolver2d.cc:47-48) into t[0..n-2].
-static void cos_fill(int n, double* t) {
-    const double pi = 4. * std::atan(1.0);
-    for (int i = 1; i < n; ++i) t[i - 1] = std::cos((pi * i) / n);
-}
-
-static int cos_tables(DevMem& mem, int n, double** out) {
-    std::vector<double> t(n - 1);
-    cos_fill(n, t.data());
-    CKR(mem.alloc(out, n - 1));
-    CK(hipMemcpy(*out, t.data(), sizeof(double) * (n - 1), hipMemcpyHostToDevice));
-    return 0;
+// One solve over all levels (dst_passes.h).  active (probe only): flows whose
+// jobs do work; the others are skipped by their flags, so their bytes are not
+// counted.  coarsify = false: the caller has built the coarse right-hand sides.
+static void run_solve(const SolvePlan& P, hipStream_t s, Probe* pr = nullptr,
+                      const std::vector<char>* active = nullptr, bool coarsify = true) {
+    const bool fs = P.force_solve;
+    if (coarsify) run_coarsify(P, s, pr, active);
+    if (P.fp32) {
+        run_solve_reduced(P, s, pr, active);
+        return;
+    }
+    auto bytes = [&](const PassGroup& G, int pass) {
+        if (!pr) return 0.0;
+        if (!active) return G.bytes[pass - 1];
+        double b = 0;
+        for (size_t j = 0; j < G.jflow.size(); ++j)
+            if ((*active)[G.jflow[j]]) b += G.jbytes[pass - 1][j];
+        return b;
+    };
+    auto one = [&](const PassGroup& G, int pass) {
+        timed(pr, (fs ? K_FSPASS1 : K_PASS1) + pass - 1, bytes(G, pass), s, [&] {
+            launch_ell_pass(pass, G.d, G.n, G.maxb[pass - 1], s, pass == 2 ? G.mi : G.mj, G.regs[pass - 1]);
+        });
+    };
+    auto boundary = [&](const PassGroup& G) {
+        timed(pr, fs ? K_FSBC : K_BC, 0, s, [&] { launch_ell_pass(4, G.d, G.n, G.maxb[3], s, G.mj, false); });
+    };
+    auto every_level = [&](const LenGroup& Q, int pass) {
+        double by = 0;
+        int blocks = 0;
+        bool regs = true, any = pass == 1;
+        for (auto& m : Q.member) {
+            const PassGroup& G = P.steps[m.first][m.second];
+            by += bytes(G, pass);
+            blocks = std::max(blocks, G.maxb[pass - 1]);
+            regs = regs && G.regs[pass - 1];
+            any = any || G.p3;
+        }
+        if (!any) return;
+        timed(pr, (fs ? K_FSPASS1 : K_PASS1) + pass - 1, by, s,
+              [&] { launch_ell_pass(pass, Q.d, Q.n, blocks, s, Q.mj, regs); });
+    };
+    if (P.given_bc)
+        for (const PassGroup& G : P.steps[0]) boundary(G);
+    if (P.all_levels)
+        for (const LenGroup& Q : P.lens) every_level(Q, 1);
+    for (int st = 0; st < P.nlev; ++st)
+        for (const PassGroup& G : P.steps[st]) {
+            if (!P.all_levels) one(G, 1);
+            one(G, 2);
+            if (G.bc && !P.given_bc) boundary(G);
+            if (!P.all_levels && G.p3) one(G, 3);
+        }
+    if (P.all_levels)
+        for (const LenGroup& Q : P.lens) every_level(Q, 3);
 }
 
 // ---------------------------------------------------------------- batch
@@ -608,13 +675,14 @@ struct Flow {
     long ns, nf;
     bool cg = false;
     // device fields
-    double *omega, *q, *nprev, *a, *wstar, *psi, *c, *U, *V, *cross, *R, *T1, *T2, *mt, *cosx, *cosy;
+    double *omega, *q, *nprev, *a, *wstar, *psi, *c, *U, *V, *cross, *R, *T1, *T2, *bcv, *mt;
     double *f, *rhs, *b, *cg_r, *cg_d, *cg_q, *cg_state, *hist, *unit, *mcol;
     // models: base states (linear models; one per phase of the periodic one),
     // the adjoint's Flux x Flux cross product, SFD's filtered state
     std::vector<double*> bq, bw;
     std::vector<bool> base_set;
     double *sff = nullptr, *what = nullptr, *sfd_prev = nullptr;
+    long tstride = 0;             // T1 of every level, this far apart (ibpm_batch::all_levels), or one level's (0)
     double base_mag = 1.0;        // magnitude of the uniform base flow (0: no potential flow)
     int* hist_count;
     double* minv[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -662,8 +730,6 @@ struct Flow {
     // local Helmholtz path of the force solve's A^-1: result and sweep buffer
     // (all levels) and, per level, the box they were last swept over (zero off it)
     double *m1 = nullptr, *m1tmp = nullptr;
-    double* ringsin = nullptr;     // 2 sin(pi l j / ny) at the ring columns (restrict_m2l_pass3)
-    double* sin1 = nullptr;        // 2 sin(pi k / ny), k = 1..ny-1
     std::vector<std::array<int, 4>> hbox;
     // host state
     std::vector<double> px, py, pu, pv;
@@ -695,6 +761,9 @@ struct ibpm_batch {
     double an[4], bn[4], cn[4];
     bool all_stationary = true, any_cg = false, initialized = false, any_ubf = false;
     bool any_periodic = false, any_adjoint = false;
+    // the solves keep T of every level and run passes 1 and 3 over all levels
+    // at once (kAllLevelBytes)
+    bool all_levels = false;
     ibpmg::CrossFFOps* d_cff = nullptr;                // adjoint flows' Flux x Flux cross products
     int cff_n = 0;
     std::vector<ibpmg::CoarsifyJob*> d_cffc;          // their coarsify, per level
@@ -723,8 +792,7 @@ struct ibpm_batch {
     std::vector<int> helm_flow;
     std::vector<double> helm_bytes, helm_cbytes;
     // the L^-1 solve's coarsify chain over its right-hand side's support
-    // (restrict_m2l_pass3), when every pass 1 of that solve is register-held
-    bool m2l_boxed = false;
+    // (restrict_m2l_pass3): d_m2lc and what follows
     int precision = 0;             // ibpm_batch_set_precision
     bool fs32 = false;             // the force solve's solves in FP32
     ibpmg::HelmJob* d_m2lc = nullptr;
@@ -1209,9 +1277,9 @@ static int alloc_flow(ibpm_batch* B, Flow& F) {
     CKR(m.alloc(&F.omega, ns)); CKR(m.alloc(&F.q, nf)); CKR(m.alloc(&F.nprev, ns));
     CKR(m.alloc(&F.a, ns)); CKR(m.alloc(&F.wstar, ns)); CKR(m.alloc(&F.psi, ns));
     CKR(m.alloc(&F.c, ns)); CKR(m.alloc(&F.U, ns)); CKR(m.alloc(&F.V, ns));
-    CKR(m.alloc(&F.cross, nf)); CKR(m.alloc(&F.R, ns)); CKR(m.alloc(&F.T1, (size_t)(F.ny - 1) * t1_ld(F.nx - 1)));
+    CKR(m.alloc(&F.cross, nf)); CKR(m.alloc(&F.R, ns)); CKR(m.alloc(&F.T1, (size_t)(F.nx - 1) * t1_ld(F.ny - 1) * (B->all_levels ? F.L : 1)));
     CKR(m.alloc(&F.T2, (size_t)(F.nx - 1) * t1_ld(F.ny - 1))); CKR(m.alloc(&F.mt, ns));
-    CKR(cos_tables(m, F.nx, &F.cosx)); CKR(cos_tables(m, F.ny, &F.cosy));
+    CKR(m.alloc(&F.bcv, bcv_size(F.nx, F.ny) * F.L));
     const int n = 2 * F.nb + 1;
     CKR(m.alloc(&F.f, n)); CKR(m.alloc(&F.rhs, n)); CKR(m.alloc(&F.b, n));
     CKR(m.alloc(&F.cg_r, n)); CKR(m.alloc(&F.cg_d, n)); CKR(m.alloc(&F.cg_q, n));
@@ -1258,7 +1326,8 @@ static SolveSpec spec_of(const Flow& F, int kind, double alpha, const double* f,
     SolveSpec s{};
     s.nx = F.nx; s.ny = F.ny; s.L = F.L; s.dx = F.dx; s.kind = kind; s.alpha = alpha;
     s.f = f; s.u = u; s.R = F.R; s.T1 = F.T1; s.T2 = F.T2; s.in_scale = in_scale; s.epilogue = epilogue;
-    s.W = W; s.cosx = F.cosx; s.cosy = F.cosy;
+    s.W = W; s.bcv = F.bcv;
+    s.tstride = F.tstride;
     return s;
 }
 
@@ -1380,64 +1449,41 @@ static void mark_nprev_valid(ibpm_batch* B) {
 constexpr int kHelmMaxSweeps = 40;
 
 // The L^-1 solve that follows the local A^-1 runs its passes over part of
-// each level.  Pass 3 writes only the psi that is read afterwards: on level
-// 0, the rows of the regulariser's nodes (and one more on each side), where
-// the interpolation takes Curl psi; on coarser levels, the ring that the next
-// finer level's getBC reads (rows ex and ex + nx/2 whole, columns ey and
-// ey + ny/2 of the rows between).  The solve's other consumers are none: the
-// step's refresh solves psi again.  Pass 1 takes rows off the right-hand
-// side's support in closed form: the support is the local result's box on
-// each level, with coarsify's reach from the finer level inside the central
-// region.  (The LDS passes ignore both restrictions and do the whole level.)
+// each level.  Pass 1 transforms the rows of its right-hand side alone, the
+// local result's box on each level with coarsify's reach from the finer level
+// inside the central region; pass 2 takes the others as 0.  Pass 3 writes only
+// the psi that is read afterwards: on level 0, the rows of the regulariser's
+// nodes (and one more on each side), where the interpolation takes Curl psi.
+// The solve's other consumers are none: the step's refresh solves psi again.
 // Algorithmic bytes of each pass of a job under its restrictions (EllJob's
 // partial-pass fields): 8 B per point read and per point written, counting
 // only the rows a pass reads and writes.
-static void pass_bytes(const EllJob& J, const PassGroup& G, double out[3]) {
+static void pass_bytes(const EllJob& J, bool fp32, double out[3]) {
     const double N1 = J.nx - 1, N2 = J.ny - 1;
-    if (G.fp32) {   // whole level: FP64 in, FP32 T1; FP32 T1 -> T2; FP32 T2, FP64 out
+    if (fp32) {   // whole level: FP64 in, FP32 T; T in and out; FP32 T, FP64 out
         out[0] = 12.0 * N1 * N2;
         out[1] = 8.0 * N1 * N2;
         out[2] = 12.0 * N1 * N2;
         return;
     }
-    const int kG1 = r16_pass_group(1);   // row pairs per workgroup of the register-held pass 1
-    // pass 1: T1 whole; rows read unless their workgroup takes the closed form
-    double read1 = N1;
-    if (J.sin1 && G.regs[0]) {
-        read1 = 0;
-        for (int r0 = 0; r0 < (int)N1; r0 += 2 * kG1) {
-            const int i_first = r0 + 1, i_last = std::min(r0 + 2 * kG1, (int)N1);
-            const bool closed = (i_last < J.sup_lo || i_first > J.sup_hi) && i_first > 1 && i_last < J.nx - 1;
-            if (!closed) read1 += i_last - i_first + 1;
-        }
-    }
-    out[0] = 8.0 * N2 * (read1 + N1);
-    // pass 2: T1 whole in, T2 rows [t2_lo, t2_hi] out
+    // pass 1: the support's rows in and out; pass 2: those in, rows [t2_lo,
+    // t2_hi] out; pass 3: its row pairs in and out
+    const double sup = std::max(0.0, (double)J.sup_hi - J.sup_lo + 1);
+    out[0] = 16.0 * N2 * sup;
     const double w2 = std::max(0.0, std::min((double)J.t2_hi, N1 - 1) - std::max(J.t2_lo, 0) + 1);
-    out[1] = 8.0 * N2 * (N1 + w2);
-    // pass 3: rows of transformed pairs in and out, ring rows in and two values out
-    double full = 0, ring = 0;
-    for (int q = 0; 2 * q < (int)N1; ++q) {
-        const int rows = std::min(2, (int)N1 - 2 * q);
-        const bool f = (q >= J.full_lo && q <= J.full_hi) || q == J.fq0 || q == J.fq1;
-        if (f) {
-            full += rows;
-        } else {
-            for (int h = 0; h < rows; ++h) {
-                const int i = 2 * q + h + 1;
-                if (i >= J.ring_lo && i <= J.ring_hi) ring += 1;
-            }
-        }
-    }
-    out[2] = 8.0 * (N2 * (2 * full + ring) + 2 * ring);
+    out[1] = 8.0 * N2 * (sup + w2);
+    const double p0 = std::max(J.full_lo, 0), p1 = std::min((double)J.full_hi, std::ceil(N1 / 2) - 1);
+    out[2] = 16.0 * N2 * std::max(0.0, std::min(2 * (p1 + 1), N1) - 2 * p0);
 }
 
 // Per-pass bytes of a group's jobs after their restrictions changed.
-static void group_bytes(PassGroup& G) {
+static void group_bytes(PassGroup& G, bool fp32) {
     for (int q = 0; q < 3; ++q) G.bytes[q] = 0;
+    G.p3 = false;
     for (size_t j = 0; j < G.h.size(); ++j) {
         double b[3];
-        pass_bytes(G.h[j], G, b);
+        G.p3 = G.p3 || G.h[j].full_lo <= G.h[j].full_hi;
+        pass_bytes(G.h[j], fp32, b);
         for (int q = 0; q < 3; ++q) {
             G.jbytes[q][j] = b[q];
             G.bytes[q] += b[q];
@@ -1446,12 +1492,12 @@ static void group_bytes(PassGroup& G) {
 }
 
 // Passes 3 and 2 of a Poisson solve whose psi is read only by the
-// interpolation (at the regulariser's nodes, level-0 rows node_lo..node_hi)
-// and by the finer levels' getBC (the coarser levels' rings): see
-// restrict_m2l_pass3.  Register-held pass 3 only.
-static void read_rows_only(EllJob& J, const PassGroup& G, int node_lo, int node_hi, const double* ringsin) {
-    if (!G.regs[2] || J.epilogue != 0 || J.vside) return;
-    const int N1 = J.nx - 1, ex = nx_ext(J.nx), ey = nx_ext(J.ny);
+// interpolation, at the regulariser's nodes (level-0 rows node_lo..node_hi).
+// The coarser levels have no pass 3: the finer levels' boundary values come
+// from T, rows ex .. ex + nx/2 of it.
+static void read_rows_only(EllJob& J, int node_lo, int node_hi) {
+    if (J.epilogue != 0) return;
+    const int N1 = J.nx - 1, ex = nx_ext(J.nx);
     if (J.lev == 0) {
         J.full_lo = std::max(node_lo - 2, 0) / 2;
         J.full_hi = std::min(node_hi, N1 - 1) / 2;
@@ -1459,55 +1505,31 @@ static void read_rows_only(EllJob& J, const PassGroup& G, int node_lo, int node_
         J.t2_hi = 2 * J.full_hi + 1;
     } else {
         J.full_lo = 1; J.full_hi = 0;
-        J.fq0 = (ex - 1) / 2; J.fq1 = (ex + J.nx / 2 - 1) / 2;
-        J.ring_lo = ex + 1; J.ring_hi = ex + J.nx / 2 - 1;
-        J.rj0 = ey; J.rj1 = ey + J.ny / 2;
-        J.ringsin = ringsin;
-        J.t2_lo = 2 * J.fq0;
-        J.t2_hi = 2 * J.fq1 + 1;
+        J.t2_lo = ex - 1;
+        J.t2_hi = ex + J.nx / 2 - 1;
     }
-    if (!G.regs[1]) {   // an LDS pass 2 writes every row
-        J.t2_lo = 0;
-        J.t2_hi = INT_MAX;
-    }
-}
-
-static int ring_tables(ibpm_batch* B) {
-    for (auto& F : B->flows) {
-        if (F.ringsin) continue;
-        const int n = F.ny - 1, ey = nx_ext(F.ny);
-        std::vector<double> t(2 * (size_t)n), s1(n);
-        const double pi = 4. * std::atan(1.);
-        for (int l = 1; l <= n; ++l) {
-            t[l - 1] = 2. * std::sin(pi * l * ey / F.ny);
-            t[n + l - 1] = 2. * std::sin(pi * l * (ey + F.ny / 2) / F.ny);
-            s1[l - 1] = 2. * std::sin(pi * l / F.ny);
-        }
-        CKR(B->mem.alloc(&F.ringsin, t.size()));
-        CKR(upload(F.ringsin, t.data(), sizeof(double) * t.size()));
-        CKR(B->mem.alloc(&F.sin1, s1.size()));
-        CKR(upload(F.sin1, s1.data(), sizeof(double) * s1.size()));
-    }
-    return 0;
 }
 
 // The step's psi = L^-1(-omega*) of substep i feeds only the interpolation of
 // C omega* (the force solve overwrites psi and the refresh solves it again),
 // so its passes 3 and 2 take read_rows_only from the current node rows.
+// (Not where a node lies next to level 0's edge: the interpolation then reads
+// psi of level 1 too.)
 static int restrict_s2(ibpm_batch* B, int i) {
-    CKR(ring_tables(B));
     std::vector<std::array<int, 2>> rows(B->flows.size(), std::array<int, 2>{1, INT_MAX});
     for (size_t k = 0; k < B->flows.size(); ++k) {
         const Flow& F = B->flows[k];
         if (F.reg.node_idx.empty()) continue;
-        int lo = INT_MAX, hi = INT_MIN;
+        int lo = INT_MAX, hi = INT_MIN, jlo = INT_MAX, jhi = INT_MIN;
         for (int idx : F.reg.node_idx) {
-            lo = std::min(lo, idx / (F.ny - 1) + 1);
-            hi = std::max(hi, idx / (F.ny - 1) + 1);
+            const int ii = idx / (F.ny - 1) + 1, jj = idx % (F.ny - 1) + 1;
+            lo = std::min(lo, ii); hi = std::max(hi, ii);
+            jlo = std::min(jlo, jj); jhi = std::max(jhi, jj);
         }
-        rows[k] = {lo, hi};
+        if (lo > 3 && hi < F.nx - 3 && jlo > 3 && jhi < F.ny - 3) rows[k] = {lo, hi};
     }
-    for (auto& step : B->S2[i].steps)
+    SolvePlan& P = B->S2[i];
+    for (auto& step : P.steps)
         for (auto& G : step) {
             bool changed = false;
             for (size_t j = 0; j < G.h.size(); ++j) {
@@ -1515,20 +1537,18 @@ static int restrict_s2(ibpm_batch* B, int i) {
                 const EllJob before = J;
                 whole_level(J);
                 const int k = G.jflow[j];
-                if (B->helm_allowed && rows[k][1] != INT_MAX)
-                    read_rows_only(J, G, rows[k][0], rows[k][1], B->flows[k].ringsin);
+                if (B->helm_allowed && rows[k][1] != INT_MAX) read_rows_only(J, rows[k][0], rows[k][1]);
                 if (std::memcmp(&before, &J, sizeof(EllJob)) != 0) changed = true;
             }
             if (changed) {
                 CKR(up(B, G.d, G.h.data(), sizeof(EllJob) * G.h.size()));
-                group_bytes(G);
+                group_bytes(G, P.fp32);
             }
         }
     return 0;
 }
 
 static int restrict_m2l_pass3(ibpm_batch* B, const std::vector<std::vector<std::array<int, 4>>>& nsup) {
-    CKR(ring_tables(B));
     // per flow and level: rbox, where the coarsify chain puts the right-hand
     // side's R (coarsify's reach from the finer level's support, inside the
     // central region; empty on level 0), and sup, the bounding box of the
@@ -1554,12 +1574,8 @@ static int restrict_m2l_pass3(ibpm_batch* B, const std::vector<std::vector<std::
                               : h;
         }
     }
-    // the boxed coarsify chain needs every pass 1 of the solve to mask R
-    bool all_regs1 = true;
-    for (auto& step : B->M2L.steps)
-        for (auto& G : step) all_regs1 = all_regs1 && G.regs[0];
-    B->m2l_boxed = all_regs1;
-    for (auto& step : B->M2L.steps)
+    SolvePlan& P = B->M2L;
+    for (auto& step : P.steps)
         for (auto& G : step) {
             bool changed = false;
             for (size_t j = 0; j < G.h.size(); ++j) {
@@ -1567,24 +1583,18 @@ static int restrict_m2l_pass3(ibpm_batch* B, const std::vector<std::vector<std::
                 const int k = G.jflow[j];
                 const EllJob before = J;
                 whole_level(J);
-                if (J.epilogue == 0 && !J.vside) {
-                    J.sup_lo = sup[k][J.lev][0];
-                    J.sup_hi = sup[k][J.lev][1];
-                    J.sin1 = B->flows[k].sin1;
-                    if (B->m2l_boxed) {
-                        const std::array<int, 4>& r = rbox[k][J.lev];
-                        J.rb_i0 = r[0]; J.rb_i1 = r[1]; J.rb_j0 = r[2]; J.rb_j1 = r[3];
-                    }
-                }
-                read_rows_only(J, G, nsup[k][0][0], nsup[k][0][1], B->flows[k].ringsin);
+                J.sup_lo = sup[k][J.lev][0];
+                J.sup_hi = sup[k][J.lev][1];
+                const std::array<int, 4>& r = rbox[k][J.lev];
+                J.rb_i0 = r[0]; J.rb_i1 = r[1]; J.rb_j0 = r[2]; J.rb_j1 = r[3];
+                read_rows_only(J, nsup[k][0][0], nsup[k][0][1]);
                 if (std::memcmp(&before, &J, sizeof(EllJob)) != 0) changed = true;
             }
             if (changed) {
                 CKR(up(B, G.d, G.h.data(), sizeof(EllJob) * G.h.size()));
-                group_bytes(G);
+                group_bytes(G, P.fp32);
             }
         }
-    if (!B->m2l_boxed) return 0;
     std::vector<HelmJob> cj;
     B->m2lc_flow.clear();
     B->m2lc_bytes.clear();
@@ -1818,7 +1828,7 @@ static void enqueue_M(ibpm_batch* B, int i, RegOps* smear, hipStream_t s,
         else
             launch_helm_sweeps(B->d_helm, B->helm_n, B->helm_blocks, B->helm_sweeps, s,
                                [&](const std::function<void()>& fn) { timed(pr, K_FSHELM, by / nl, s, fn); });
-        const bool boxed = B->m2l_boxed && !B->M2L.fp32;   // the boxed chain feeds register-held passes only
+        const bool boxed = !B->M2L.fp32;   // the FP32 passes read the whole coarse right-hand side
         if (single_level) {
             run_solve(B->M1L, s, pr, active, false);
         } else if (boxed) {
@@ -2596,9 +2606,8 @@ static int build_inverse(ibpm_batch* B, int i, bool precond) {
         B->m1l_built = true;
     }
     if (single) {
-        // the level-0 solve read as the force solve's: pass 1 in closed form
-        // (zeros: no boundary values) off the local result's rows, passes 3 and
-        // 2 over the node rows only
+        // the level-0 solve read as the force solve's: pass 1 over the local
+        // result's rows, passes 3 and 2 over the node rows only
         for (auto& step : B->M1L.steps)
             for (auto& G : step) {
                 bool changed = false;
@@ -2615,14 +2624,13 @@ static int build_inverse(ibpm_batch* B, int i, bool precond) {
                         }
                         J.sup_lo = F.hbox[0][0];
                         J.sup_hi = F.hbox[0][1];
-                        J.sin1 = F.sin1;
-                        read_rows_only(J, G, lo, hi, F.ringsin);
+                        read_rows_only(J, lo, hi);
                     }
                     if (std::memcmp(&before, &J, sizeof(EllJob)) != 0) changed = true;
                 }
                 if (changed) {
                     CKR(upload(G.d, G.h.data(), sizeof(EllJob) * G.h.size()));
-                    group_bytes(G);
+                    group_bytes(G, B->M1L.fp32);
                 }
             }
     }
@@ -3017,35 +3025,27 @@ static int check_grid(int nx, int ny, int ngrid) {
 }
 
 int ibpm_dst2d(ibpm_ctx* c, int n1, int n2, const double* d_in, double* d_out) {
-    // The 2-D DST is the solve pipeline with unit eigenvalues and no
-    // normalisation: kind Poisson with a scaling table forced to 1 is not
-    // available, so pass 1 and pass 3 are run back to back through T.
+    // The first half of the solve pipeline: pass 1 (rows along j), then pass 2
+    // in its forward-only form (kind 2: the transform along i, to u).
     CKR(check_grid(n1 + 1, n2 + 1, 1));
     DevMem mem;
-    double *T = nullptr, *cosx = nullptr, *cosy = nullptr;
-    CKR(mem.alloc(&T, (size_t)n1 * n2));
-    CKR(cos_tables(mem, n1 + 1, &cosx));
-    CKR(cos_tables(mem, n2 + 1, &cosy));
+    double* T = nullptr;
+    CKR(mem.alloc(&T, (size_t)n1 * t1_ld(n2)));
     EllJob J{};
+    J.nx = n1 + 1; J.ny = n2 + 1; J.lev = 0; J.ngrid = 1; J.kind = 2; J.in_scale = 1.0;
     whole_level(J);
-    J.nx = n1 + 1; J.ny = n2 + 1; J.lev = 0; J.ngrid = 1; J.in_scale = 1.0;
-    J.f = d_in; J.T1 = T; J.T2 = T; J.u = d_out; J.norm = 1.0;
-    J.ld1 = n1; J.ld2 = n2;   // unpadded: the second launch writes the caller's array
+    J.f = d_in; J.T1 = T; J.u = d_out; J.norm = 1.0;
+    J.ld1 = t1_ld(n2);
     CKR(get_plan(&c->c, n2, &J.pj));
     CKR(get_plan(&c->c, n1, &J.pi));
-    // pass 1: rows along j -> T (transposed); a second pass-1 style launch over
-    // the transposed rows transforms along i and transposes back.
-    EllJob J2 = J;
-    J2.nx = n2 + 1; J2.ny = n1 + 1; J2.f = T; J2.T1 = d_out; J2.pj = J.pi;
-    J2.ld1 = n2; J2.ld2 = n1;
     EllJob* d = nullptr;
-    CKR(mem.alloc(&d, 2));
+    CKR(mem.alloc(&d, 1));
     CK(hipMemcpyAsync(d, &J, sizeof(EllJob), hipMemcpyHostToDevice, c->c.stream));
-    CK(hipMemcpyAsync(d + 1, &J2, sizeof(EllJob), hipMemcpyHostToDevice, c->c.stream));
-    const bool r1 = pass_in_registers(J.pj.M, (n1 + 1) / 2), r2 = pass_in_registers(J2.pj.M, (n2 + 1) / 2);
-    launch_ell_pass(1, d, 1, blocks_for_pass(J, 1, r1), lds_for_pass(J, 1, r1), c->c.stream, false, J.pj.M, r1);
-    launch_ell_pass(1, d + 1, 1, blocks_for_pass(J2, 1, r2), lds_for_pass(J2, 1, r2), c->c.stream, false,
-                    J2.pj.M, r2);
+    for (int pass = 1; pass <= 2; ++pass) {
+        const int M = pass == 2 ? J.pi.M : J.pj.M;
+        const bool regs = pass_in_registers(M, ((pass == 2 ? n2 : n1) + 1) / 2);
+        launch_ell_pass(pass, d, 1, blocks_for_pass(J, pass, regs), c->c.stream, M, regs);
+    }
     CK(hipStreamSynchronize(c->c.stream));
     CK(hipGetLastError());
     return 0;
@@ -3057,18 +3057,19 @@ static int solve_common(ibpm_ctx* c, int kind, int nx, int ny, int ngrid, double
     CKR(check_grid(nx, ny, ngrid));
     DevMem mem;
     const long ns = (long)(nx - 1) * (ny - 1);
-    double *R = nullptr, *T1 = nullptr, *T2 = nullptr, *cosx = nullptr, *cosy = nullptr, *fin = nullptr;
+    double *R = nullptr, *T1 = nullptr, *T2 = nullptr, *bcv = nullptr, *fin = nullptr;
+    const long tlev = (long)(nx - 1) * t1_ld(ny - 1);
+    const bool all = 8.0 * tlev * ngrid <= kAllLevelBytes;
     CKR(mem.alloc(&R, ns * ngrid));
-    CKR(mem.alloc(&T1, (size_t)(ny - 1) * t1_ld(nx - 1)));
-    CKR(mem.alloc(&T2, (size_t)(nx - 1) * t1_ld(ny - 1)));
+    CKR(mem.alloc(&T1, tlev * (all ? ngrid : 1)));
+    CKR(mem.alloc(&bcv, bcv_size(nx, ny) * ngrid));
+    if (precision == 2) CKR(mem.alloc(&T2, (size_t)(nx - 1) * t1_ld(ny - 1)));   // the GEMM-DST's second plane pair
     CKR(mem.alloc(&fin, ns * ngrid));
     CK(hipMemcpyAsync(fin, d_f, sizeof(double) * ns * ngrid, hipMemcpyDeviceToDevice, c->c.stream));
-    CKR(cos_tables(mem, nx, &cosx));
-    CKR(cos_tables(mem, ny, &cosy));
     SolveSpec s{};
     s.nx = nx; s.ny = ny; s.L = ngrid; s.dx = dx; s.kind = kind; s.alpha = alpha;
     s.f = fin; s.u = d_u; s.R = R; s.T1 = T1; s.T2 = T2; s.in_scale = in_scale; s.epilogue = 0;
-    s.cosx = cosx; s.cosy = cosy; s.bcring = d_bc;
+    s.bcring = d_bc; s.bcv = bcv; s.tstride = all ? tlev : 0;
     SolvePlan P;
     CKR(build_solve_plan(&c->c, mem, {s}, P));
     if (precision >= 1) set_plan_fp32(P, true);
@@ -3114,8 +3115,8 @@ int ibpm_elliptic_solve_precision(ibpm_ctx* c, int kind, int nx, int ny, int ngr
 // is held until the stream has drained.
 static constexpr int kNoAllocMaxLevels = 16;
 struct NoAllocStage {
-    double cosx[kFftLds / 2], cosy[kFftLds / 2];
     double2 twj[kFftLds], t16j[256], twi[kFftLds], t16i[256];
+    double realj[2 * kFftLds + 16], reali[2 * kFftLds + 16];   // plan_reals of the longest plan
     EllJob ej[kNoAllocMaxLevels];
     CoarsifyJob cj[kNoAllocMaxLevels];
 };
@@ -3139,9 +3140,16 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += (bytes + 255) & ~size_t(255); return o; };
     const size_t o_fin = take(8 * ns * L), o_R = take(8 * ns * L);
-    const size_t o_T1 = take(8 * (size_t)(ny - 1) * t1_ld(nx - 1)), o_T2 = take(8 * (size_t)(nx - 1) * t1_ld(ny - 1));
-    const size_t zero_lo = o_R, zero_hi = off;   // R, T1 and T2 start at zero, as freshly allocated ones
-    const size_t o_cx = take(8 * (size_t)(nx - 1)), o_cy = take(8 * (size_t)(ny - 1));
+    const size_t o_T1 = take(8 * (size_t)(nx - 1) * t1_ld(ny - 1));
+    const size_t zero_lo = o_R, zero_hi = off;   // R and T start at zero, as freshly allocated ones
+    const size_t rows_end = off;
+    const size_t o_bcv = take(8 * bcv_size(nx, ny) * L);
+    const size_t o_rj = take(8 * plan_reals(pj.N)), o_ri = take(8 * plan_reals(pi.N));
+    // the accepted sizes are those of 16 bytes of scratch rows per point; only
+    // small grids need more than that for the boundary values and tables
+    off = std::max(off, rows_end + ((8 * (size_t)(ny - 1) * t1_ld(nx - 1) + 255) & ~size_t(255)));
+    (void)take(8 * (size_t)(nx - 1));
+    (void)take(8 * (size_t)(ny - 1));
     const size_t o_twj = take(16 * (size_t)pj.M), o_t16j = take(16 * 256);
     const size_t o_twi = take(16 * (size_t)pi.M), o_t16i = take(16 * 256);
     const size_t o_ej = take(sizeof(EllJob) * L), o_cj = take(sizeof(CoarsifyJob) * L);
@@ -3156,19 +3164,15 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     double* fin = (double*)(b + o_fin);
     std::lock_guard<std::mutex> lk(g_noalloc_mu);
     NoAllocStage& H = g_noalloc_stage;
-    cos_fill(nx, H.cosx);
-    cos_fill(ny, H.cosy);
-    plan_tables(pj.M, H.twj, H.t16j);
-    plan_tables(pi.M, H.twi, H.t16i);
-    pj.tw = (const double2*)(b + o_twj);
-    pj.tw16 = plan_has_tw16(pj.M) ? (const double2*)(b + o_t16j) : nullptr;
-    pi.tw = (const double2*)(b + o_twi);
-    pi.tw16 = plan_has_tw16(pi.M) ? (const double2*)(b + o_t16i) : nullptr;
+    plan_tables(pj.M, H.twj, H.t16j, H.realj);
+    plan_tables(pi.M, H.twi, H.t16i, H.reali);
+    plan_pointers(pj, (const double2*)(b + o_twj), (const double2*)(b + o_t16j), (const double*)(b + o_rj));
+    plan_pointers(pi, (const double2*)(b + o_twi), (const double2*)(b + o_t16i), (const double*)(b + o_ri));
     SolveSpec sp{};
     sp.nx = nx; sp.ny = ny; sp.L = L; sp.dx = dx; sp.kind = kind; sp.alpha = alpha;
-    sp.f = fin; sp.u = d_u; sp.R = (double*)(b + o_R); sp.T1 = (double*)(b + o_T1); sp.T2 = (double*)(b + o_T2);
+    sp.f = fin; sp.u = d_u; sp.R = (double*)(b + o_R); sp.T1 = (double*)(b + o_T1);
     sp.in_scale = 1.0; sp.epilogue = 0;
-    sp.cosx = (const double*)(b + o_cx); sp.cosy = (const double*)(b + o_cy);
+    sp.bcv = (double*)(b + o_bcv);
     for (int st = 0; st < L; ++st) {   // coarsest level first
         H.ej[st] = EllJob{};
         fill_ell_job(sp, L - 1 - st, H.ej[st]);
@@ -3181,8 +3185,8 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     CoarsifyJob* d_cj = (CoarsifyJob*)(b + o_cj);
     CK(hipMemsetAsync(b + zero_lo, 0, zero_hi - zero_lo, s));
     CK(hipMemcpyAsync(fin, d_f, 8 * ns * L, hipMemcpyDeviceToDevice, s));
-    CK(hipMemcpyAsync(b + o_cx, H.cosx, 8 * (size_t)(nx - 1), hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(b + o_cy, H.cosy, 8 * (size_t)(ny - 1), hipMemcpyHostToDevice, s));
+    CK(hipMemcpyAsync(b + o_rj, H.realj, 8 * plan_reals(pj.N), hipMemcpyHostToDevice, s));
+    CK(hipMemcpyAsync(b + o_ri, H.reali, 8 * plan_reals(pi.N), hipMemcpyHostToDevice, s));
     CK(hipMemcpyAsync(b + o_twj, H.twj, 16 * (size_t)pj.M, hipMemcpyHostToDevice, s));
     CK(hipMemcpyAsync(b + o_t16j, H.t16j, 16 * 256, hipMemcpyHostToDevice, s));
     CK(hipMemcpyAsync(b + o_twi, H.twi, 16 * (size_t)pi.M, hipMemcpyHostToDevice, s));
@@ -3190,14 +3194,14 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     CK(hipMemcpyAsync(d_ej, H.ej, sizeof(EllJob) * L, hipMemcpyHostToDevice, s));
     if (L > 1) CK(hipMemcpyAsync(d_cj, H.cj, sizeof(CoarsifyJob) * (L - 1), hipMemcpyHostToDevice, s));
     for (int lev = 1; lev < L; ++lev) launch_coarsify(d_cj + (lev - 1), 1, nx / 2 - 1, s, false);
-    for (int st = 0; st < L; ++st) {
-        bool regs[3];
-        int maxb[3], lds[3];
-        pass_shape(H.ej[st], regs, maxb, lds);
-        for (int pass = 1; pass <= 3; ++pass)
-            launch_ell_pass(pass, d_ej + st, 1, maxb[pass - 1], lds[pass - 1], s, false,
-                            pass == 2 ? pi.M : pj.M, regs[pass - 1]);
-    }
+    for (int st = 0; st < L; ++st)   // one level's scratch rows: level by level
+        for (int pass : {1, 2, 4, 3}) {
+            const EllJob& J = H.ej[st];
+            if (pass == 4 && !J.bc_out) continue;
+            const int M = pass == 2 ? pi.M : pj.M;
+            const bool regs = pass != 4 && pass_in_registers(M, (pass == 2 ? ny : nx) / 2);
+            launch_ell_pass(pass, d_ej + st, 1, blocks_for_pass(J, pass, regs), s, M, regs);
+        }
     CK(hipGetLastError());
     CK(hipStreamSynchronize(s));
     return 0;
@@ -3780,12 +3784,6 @@ int ibpm_batch_create(ibpm_ctx* ctx, int nflows, const ibpm_flow_params* params,
         if (F.cg) B->any_cg = true;
         if (!F.geom.stationary) B->all_stationary = false;
         if (F.p.cg_tol <= 0) F.p.cg_tol = 1e-7;   // IBSolver.cc:31 default
-        CKR(alloc_flow(B.get(), F));
-        CKR(B->mem.alloc(&F.bf_dev, 4));
-        {
-            const double zero[4] = {0, 0, 0, 0};
-            CKR(upload(F.bf_dev, zero, sizeof zero));
-        }
         B->max_ns_all = std::max(B->max_ns_all, F.ns * F.L);
         B->max_nf = std::max(B->max_nf, F.nf);
         B->max_cells_all = std::max(B->max_cells_all, (long)(F.nx + 1) * (F.ny + 1) * F.L);
@@ -3804,6 +3802,16 @@ int ibpm_batch_create(ibpm_ctx* ctx, int nflows, const ibpm_flow_params* params,
         B->bytes_cross += 8.0 * (2 * F.ns + F.nf) * F.L;
         B->bytes_rhs += 8.0 * (4 + fpn) * (F.p.model == 0 ? nact : (double)F.ns * F.L);
         B->bytes_curlq += 8.0 * (F.ns + F.nf) * F.L;
+    }
+    double tbytes = 0;
+    for (auto& F : B->flows) tbytes += 8.0 * (F.nx - 1) * t1_ld(F.ny - 1) * F.L;
+    B->all_levels = tbytes <= kAllLevelBytes;
+    for (auto& F : B->flows) {
+        F.tstride = B->all_levels ? (long)(F.nx - 1) * t1_ld(F.ny - 1) : 0;
+        CKR(alloc_flow(B.get(), F));
+        CKR(B->mem.alloc(&F.bf_dev, 4));
+        const double zero[4] = {0, 0, 0, 0};
+        CKR(upload(F.bf_dev, zero, sizeof zero));
     }
     if (B->any_cg) {
         for (auto& F : B->flows) F.cg = true;   // one force solver per batch

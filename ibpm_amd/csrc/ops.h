@@ -171,16 +171,16 @@ struct ForceOps {
 };
 
 // Whether a pass launch of FFT length M over row_pairs row pairs (summed
-// over its jobs) uses the register-held transform; the three calls below take
-// that choice.
+// over its jobs) uses the register-held transform; the two calls below take
+// that choice.  Passes 1 to 3, and 4 for the boundary values of the next finer
+// level (dst_passes.h).
 bool pass_in_registers(int M, long row_pairs);
 int blocks_for_pass(const EllJob& J, int pass, bool regs);
-int lds_for_pass(const EllJob& J, int pass, bool regs);
+void launch_ell_pass(int pass, const EllJob* d_jobs, int njobs, int max_blocks, hipStream_t s, int M, bool regs);
+int blocks_for_pass32(const EllJob& J, int pass);
 int lds_for_pass32(const EllJob& J, int pass);
 void launch_ell_pass32(int pass, const EllJob* d_jobs, int njobs, int max_blocks, int lds_bytes, hipStream_t s,
                        bool force_solve, int M);
-void launch_ell_pass(int pass, const EllJob* d_jobs, int njobs, int max_blocks, int lds_bytes, hipStream_t s,
-                     bool force_solve, int M, bool regs);
 void launch_coarsify(const CoarsifyJob* d_jobs, int njobs, int max_rows, hipStream_t s, bool force_solve = false);
 // Split-BF16 GEMM-DST level solve of every job (square levels of n = N = nx - 1
 // <= 511 unknowns per side, planes in the jobs' T1 / T2): Sh, Sl the split sine
@@ -193,8 +193,6 @@ void launch_gemm_dst(const EllJob* d_jobs, int njobs, int n, const __bf16* Sh, c
 // time it).
 int helm_tiles(int h, int w);
 int helm_launches(int nsweeps);   // launches of launch_helm_sweeps for nsweeps sweeps
-// Row pairs per workgroup of register-held pass `pass` (1, 2, 3).
-int r16_pass_group(int pass);
 // eo = ei - out over each job's box; max_blocks: kThreads-point blocks of the
 // largest box.
 void launch_helm_epilogue(const HelmJob* d_jobs, int njobs, int max_blocks, hipStream_t s);
