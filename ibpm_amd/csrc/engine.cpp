@@ -94,6 +94,84 @@ struct Ctx {
     std::map<int, FftPlan> plans;   // by DST length
     std::map<int, std::pair<__bf16*, __bf16*>> sines;   // split sine matrices of the GEMM-DST, by N
     DevMem mem;
+    // Workspace of the stand-alone entry points (OpScope), kept between calls:
+    // device memory, and descriptors with their pinned host image.  A context
+    // is used by one host thread at a time, on one stream.
+    char* ws = nullptr;
+    size_t ws_cap = 0, ws_used = 0;
+    char *desc = nullptr, *h_desc = nullptr;
+    size_t desc_used = 0;
+    ~Ctx() {
+        if (ws) (void)hipFree(ws);
+        if (desc) (void)hipFree(desc);
+        if (h_desc) (void)hipHostFree(h_desc);
+    }
+};
+constexpr size_t kWsMax = size_t(1) << 30;   // most workspace a context keeps; a call that needs more allocates
+constexpr size_t kDescBytes = size_t(1) << 17;
+
+// Device memory and descriptors of one stand-alone call.  What bounds such a
+// call on a small grid is not its kernels (13 us for three passes at 64^2) but
+// allocating, clearing and freeing its buffers and one blocking copy per
+// descriptor (127 us in all): buffers come from the context's workspace, which
+// grows to the largest call so far, and the descriptors go up in one copy.
+// Memory is not cleared.  Scopes nest (a call made of others); the stream must
+// have drained before the scope ends.
+struct OpScope {
+    Ctx* c;
+    size_t base, desc_base, need;
+    std::vector<void*> extra;
+    explicit OpScope(Ctx* ctx) : c(ctx), base(ctx->ws_used), desc_base(ctx->desc_used), need(ctx->ws_used) {}
+    ~OpScope() {
+        if (!extra.empty()) (void)hipStreamSynchronize(c->stream);   // (an error's return may come before)
+        for (void* p : extra) (void)hipFree(p);
+        c->ws_used = base;
+        c->desc_used = desc_base;
+        if (base == 0 && need > c->ws_cap && need <= kWsMax) {
+            if (c->ws) (void)hipFree(c->ws);
+            c->ws_cap = hipMalloc((void**)&c->ws, need) == hipSuccess ? need : 0;
+            if (!c->ws_cap) c->ws = nullptr;
+        }
+    }
+    template <class T>
+    int alloc(T** out, size_t count) {
+        const size_t bytes = (std::max<size_t>(count, 1) * sizeof(T) + 255) & ~size_t(255);
+        need += bytes;
+        if (c->ws_used + bytes <= c->ws_cap) {
+            *out = (T*)(c->ws + c->ws_used);
+            c->ws_used += bytes;
+            return 0;
+        }
+        void* p = nullptr;
+        CK(hipMalloc(&p, bytes));
+        extra.push_back(p);
+        *out = (T*)p;
+        return 0;
+    }
+    // Device address of n descriptors, valid after flush().
+    template <class T>
+    int put(T** out, const T* h, size_t n) {
+        if (!c->desc) {
+            CK(hipMalloc((void**)&c->desc, kDescBytes));
+            CK(hipHostMalloc((void**)&c->h_desc, kDescBytes, hipHostMallocDefault));
+        }
+        const size_t bytes = (n * sizeof(T) + 255) & ~size_t(255);
+        if (c->desc_used + bytes > kDescBytes) { set_error("%zu descriptor bytes exceed the limit", bytes); return -2; }
+        std::memcpy(c->h_desc + c->desc_used, h, n * sizeof(T));
+        *out = (T*)(c->desc + c->desc_used);
+        c->desc_used += bytes;
+        return 0;
+    }
+    int flush() {
+        CK(hipMemcpyAsync(c->desc + desc_base, c->h_desc + desc_base, c->desc_used - desc_base, hipMemcpyHostToDevice,
+                          c->stream));
+        return 0;
+    }
+    int finish() {
+        CK(hipStreamSynchronize(c->stream));
+        CK(hipGetLastError());
+        return 0;
+    }
 };
 
 // Round to nearest even of an FP32 value to bf16 (the device conversion's rule).
@@ -3028,7 +3106,7 @@ int ibpm_dst2d(ibpm_ctx* c, int n1, int n2, const double* d_in, double* d_out) {
     // The first half of the solve pipeline: pass 1 (rows along j), then pass 2
     // in its forward-only form (kind 2: the transform along i, to u).
     CKR(check_grid(n1 + 1, n2 + 1, 1));
-    DevMem mem;
+    OpScope mem(&c->c);
     double* T = nullptr;
     CKR(mem.alloc(&T, (size_t)n1 * t1_ld(n2)));
     EllJob J{};
@@ -3039,15 +3117,75 @@ int ibpm_dst2d(ibpm_ctx* c, int n1, int n2, const double* d_in, double* d_out) {
     CKR(get_plan(&c->c, n2, &J.pj));
     CKR(get_plan(&c->c, n1, &J.pi));
     EllJob* d = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CK(hipMemcpyAsync(d, &J, sizeof(EllJob), hipMemcpyHostToDevice, c->c.stream));
+    CKR(mem.put(&d, &J, 1));
+    CKR(mem.flush());
     for (int pass = 1; pass <= 2; ++pass) {
         const int M = pass == 2 ? J.pi.M : J.pj.M;
         const bool regs = pass_in_registers(M, ((pass == 2 ? n2 : n1) + 1) / 2);
         launch_ell_pass(pass, d, 1, blocks_for_pass(J, pass, regs), c->c.stream, M, regs);
     }
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
+    return mem.finish();
+}
+
+// Launches a stand-alone FP64 solve on the context's stream.  d_f is read in
+// place where the solve allows it: its right-hand side is coarsified before
+// anything is written, and a level of u is written after pass 1 of that level
+// and the coarser ones, so u may be f itself; where the two overlap otherwise,
+// f is copied.
+static int enqueue_solve(Ctx* c, OpScope& mem, int kind, int nx, int ny, int L, double dx, double alpha,
+                         const double* d_f, const double* d_bc, double* d_u, double in_scale) {
+    const long ns = (long)(nx - 1) * (ny - 1), tlev = (long)(nx - 1) * t1_ld(ny - 1);
+    const bool all = 8.0 * tlev * L <= kAllLevelBytes;
+    double *R = nullptr, *T = nullptr, *bcv = nullptr, *fin = nullptr;
+    if (L > 1) CKR(mem.alloc(&R, ns * L));
+    CKR(mem.alloc(&T, tlev * (all ? L : 1)));
+    CKR(mem.alloc(&bcv, bcv_size(nx, ny) * L));
+    if (d_f != d_u && d_f < d_u + ns * L && d_u < d_f + ns * L) {
+        CKR(mem.alloc(&fin, ns * L));
+        CK(hipMemcpyAsync(fin, d_f, sizeof(double) * ns * L, hipMemcpyDeviceToDevice, c->stream));
+        d_f = fin;
+    }
+    SolveSpec s{};
+    s.nx = nx; s.ny = ny; s.L = L; s.dx = dx; s.kind = kind; s.alpha = alpha;
+    s.f = d_f; s.u = d_u; s.R = R; s.T1 = T; s.in_scale = in_scale; s.epilogue = 0;
+    s.bcring = d_bc; s.bcv = bcv; s.tstride = all ? tlev : 0;
+    FftPlan pj{}, pi{};
+    CKR(get_plan(c, ny - 1, &pj));
+    CKR(get_plan(c, nx - 1, &pi));
+    std::vector<EllJob> job(L);   // coarsest level first
+    for (int st = 0; st < L; ++st) {
+        fill_ell_job(s, L - 1 - st, job[st]);
+        job[st].pj = pj;
+        job[st].pi = pi;
+    }
+    std::vector<CoarsifyJob> cj;
+    for (int lev = 1; lev < L; ++lev) cj.push_back(CoarsifyJob{nx, ny, lev, d_f, R, nullptr});
+    EllJob* d = nullptr;
+    CoarsifyJob* dc = nullptr;
+    CKR(mem.put(&d, job.data(), L));
+    if (L > 1) CKR(mem.put(&dc, cj.data(), L - 1));
+    CKR(mem.flush());
+    hipStream_t q = c->stream;
+    for (int lev = 1; lev < L; ++lev) launch_coarsify(dc + (lev - 1), 1, nx / 2 - 1, q, false);
+    bool regs[3];
+    int blocks[4];
+    for (int pass = 1; pass <= 4; ++pass) {
+        const bool r = pass < 4 && pass_in_registers(pass == 2 ? pi.M : pj.M, (pass == 2 ? ny : nx) / 2);
+        if (pass < 4) regs[pass - 1] = r;
+        blocks[pass - 1] = blocks_for_pass(job[0], pass, r);
+    }
+    auto run = [&](int pass, int st, int n) {
+        launch_ell_pass(pass, d + st, n, blocks[pass - 1], q, pass == 2 ? pi.M : pj.M, pass < 4 && regs[pass - 1]);
+    };
+    if (d_bc) run(4, 0, 1);
+    if (all) run(1, 0, L);
+    for (int st = 0; st < L; ++st) {
+        if (!all) run(1, st, 1);
+        run(2, st, 1);
+        if (st + 1 < L) run(4, st, 1);
+        if (!all) run(3, st, 1);
+    }
+    if (all) run(3, 0, L);
     return 0;
 }
 
@@ -3055,24 +3193,27 @@ static int solve_common(ibpm_ctx* c, int kind, int nx, int ny, int ngrid, double
                         const double* d_f, const double* d_bc, double* d_u, double in_scale = 1.0,
                         int precision = 0) {
     CKR(check_grid(nx, ny, ngrid));
+    if (precision == 0) {
+        OpScope mem(&c->c);
+        CKR(enqueue_solve(&c->c, mem, kind, nx, ny, ngrid, dx, alpha, d_f, d_bc, d_u, in_scale));
+        return mem.finish();
+    }
     DevMem mem;
     const long ns = (long)(nx - 1) * (ny - 1);
-    double *R = nullptr, *T1 = nullptr, *T2 = nullptr, *bcv = nullptr, *fin = nullptr;
+    double *R = nullptr, *T1 = nullptr, *T2 = nullptr, *fin = nullptr;
     const long tlev = (long)(nx - 1) * t1_ld(ny - 1);
-    const bool all = 8.0 * tlev * ngrid <= kAllLevelBytes;
     CKR(mem.alloc(&R, ns * ngrid));
-    CKR(mem.alloc(&T1, tlev * (all ? ngrid : 1)));
-    CKR(mem.alloc(&bcv, bcv_size(nx, ny) * ngrid));
-    if (precision == 2) CKR(mem.alloc(&T2, (size_t)(nx - 1) * t1_ld(ny - 1)));   // the GEMM-DST's second plane pair
+    CKR(mem.alloc(&T1, tlev));
+    if (precision == 2) CKR(mem.alloc(&T2, tlev));   // the GEMM-DST's second plane pair
     CKR(mem.alloc(&fin, ns * ngrid));
     CK(hipMemcpyAsync(fin, d_f, sizeof(double) * ns * ngrid, hipMemcpyDeviceToDevice, c->c.stream));
     SolveSpec s{};
     s.nx = nx; s.ny = ny; s.L = ngrid; s.dx = dx; s.kind = kind; s.alpha = alpha;
     s.f = fin; s.u = d_u; s.R = R; s.T1 = T1; s.T2 = T2; s.in_scale = in_scale; s.epilogue = 0;
-    s.bcring = d_bc; s.bcv = bcv; s.tstride = all ? tlev : 0;
+    s.bcring = d_bc;
     SolvePlan P;
     CKR(build_solve_plan(&c->c, mem, {s}, P));
-    if (precision >= 1) set_plan_fp32(P, true);
+    set_plan_fp32(P, true);
     if (precision == 2) {
         CKR(tune_plan_gemm(&c->c, mem, P, 4));
         for (auto& step : P.steps)
@@ -3208,8 +3349,8 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
 }
 
 // Stand-alone stencil entry points run the batch kernels on a one-flow
-// descriptor with scratch buffers.
-static int ops_common(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, FlowOps& o, DevMem& mem) {
+// descriptor with buffers from the context's workspace.
+static int ops_common(int nx, int ny, int ngrid, double dx, FlowOps& o, OpScope& mem) {
     CKR(check_grid(nx, ny, ngrid));
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
     const long nf = (2L * nx * ny + nx + ny) * ngrid;
@@ -3219,113 +3360,116 @@ static int ops_common(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, FlowOps
     if (!o.cross) CKR(mem.alloc(&o.cross, nf));
     if (!o.a) CKR(mem.alloc(&o.a, ns));
     if (!o.nprev) CKR(mem.alloc(&o.nprev, ns));
-    (void)c;
+    return 0;
+}
+
+static int cleared(OpScope& mem, double** out, size_t count) {
+    CKR(mem.alloc(out, count));
+    CK(hipMemsetAsync(*out, 0, sizeof(double) * count, mem.c->stream));
     return 0;
 }
 
 int ibpm_curl_flux(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, const double* d_q, double* d_w) {
     // N = Curl(cross) of the rhs kernel with omega = 0: a = dt * an * N = N.
-    DevMem mem;
+    CKR(check_grid(nx, ny, ngrid));
+    OpScope mem(&c->c);
     FlowOps o{};
-    double* zero = nullptr;
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
-    CKR(mem.alloc(&zero, ns));
+    CKR(cleared(mem, &o.omega, ns));
     o.cross = const_cast<double*>(d_q);
-    o.omega = zero;
     o.a = d_w;
     o.lap_coef = 0; o.an = 1; o.bn = 0; o.dt = 1; o.w_coef = 0;
-    CKR(ops_common(c, nx, ny, ngrid, dx, o, mem));
+    CKR(ops_common(nx, ny, ngrid, dx, o, mem));
     FlowOps* d = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
+    CKR(mem.put(&d, &o, 1));
+    CKR(mem.flush());
     launch_rhs(d, 1, ns, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
-    return 0;
+    return mem.finish();
 }
 
 int ibpm_laplacian(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, const double* d_w, double* d_out) {
     // rhs kernel with a = Lap(omega): lap_coef 1, no nonlinear term, no omega.
-    DevMem mem;
+    CKR(check_grid(nx, ny, ngrid));
+    OpScope mem(&c->c);
     FlowOps o{};
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
     const long nf = (2L * nx * ny + nx + ny) * ngrid;
-    double* zc = nullptr;
-    CKR(mem.alloc(&zc, nf));
-    o.cross = zc;
+    CKR(cleared(mem, &o.cross, nf));
     o.omega = const_cast<double*>(d_w);
     o.a = d_out;
     o.lap_coef = 1; o.an = 0; o.bn = 0; o.dt = 1; o.w_coef = 0;
-    CKR(ops_common(c, nx, ny, ngrid, dx, o, mem));
+    CKR(ops_common(nx, ny, ngrid, dx, o, mem));
     FlowOps* d = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
+    CKR(mem.put(&d, &o, 1));
+    CKR(mem.flush());
     launch_rhs(d, 1, ns, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
+    return mem.finish();
+}
+
+// q = Curl(psi) + q0 into d_q, launched on the context's stream.
+static int enqueue_curl(Ctx* c, OpScope& mem, int nx, int ny, int ngrid, double dx, double u0, double v0,
+                        const double* psi, double* d_q) {
+    FlowOps o{};
+    o.nx = nx; o.ny = ny; o.L = ngrid; o.dx = dx;
+    o.psi = const_cast<double*>(psi);
+    o.q = d_q;
+    o.ubase = u0; o.vbase = v0;
+    FlowOps* d = nullptr;
+    const size_t at = c->desc_used;
+    CKR(mem.put(&d, &o, 1));
+    CK(hipMemcpyAsync(d, c->h_desc + at, sizeof(o), hipMemcpyHostToDevice, c->stream));
+    launch_curl_q(d, 1, (long)(nx + 1) * (ny + 1) * ngrid, c->stream);
     return 0;
 }
 
 int ibpm_curl_scalar(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, double u0, double v0,
                      const double* d_w, double* d_q) {
-    DevMem mem;
-    FlowOps o{};
-    o.psi = const_cast<double*>(d_w);
-    o.q = d_q;
-    o.ubase = u0; o.vbase = v0;
-    CKR(ops_common(c, nx, ny, ngrid, dx, o, mem));
-    FlowOps* d = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
-    launch_curl_q(d, 1, (long)(nx + 1) * (ny + 1) * ngrid, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
-    return 0;
+    CKR(check_grid(nx, ny, ngrid));
+    OpScope mem(&c->c);
+    CKR(enqueue_curl(&c->c, mem, nx, ny, ngrid, dx, u0, v0, d_w, d_q));
+    return mem.finish();
 }
 
 int ibpm_nonlinear(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, const double* d_q,
                    const double* d_w, double* d_n) {
-    DevMem mem;
-    FlowOps o{};
+    CKR(check_grid(nx, ny, ngrid));
+    OpScope mem(&c->c);
+    FlowOps o[2] = {};
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
     const long nf1 = 2L * nx * ny + nx + ny;
     double* zero = nullptr;
-    CKR(mem.alloc(&zero, ns));
-    o.q = const_cast<double*>(d_q);
-    o.omega = const_cast<double*>(d_w);
-    CKR(ops_common(c, nx, ny, ngrid, dx, o, mem));
+    CKR(cleared(mem, &zero, ns));
+    o[0].q = const_cast<double*>(d_q);
+    o[0].omega = const_cast<double*>(d_w);
+    CKR(ops_common(nx, ny, ngrid, dx, o[0], mem));
+    o[1] = o[0];   // curl of cross: rhs kernel with omega = 0, dt = an = 1
+    o[1].omega = zero; o[1].a = d_n; o[1].lap_coef = 0; o[1].an = 1; o[1].bn = 0; o[1].dt = 1; o[1].w_coef = 0;
     FlowOps* d = nullptr;
-    CKR(mem.alloc(&d, 2));
-    FlowOps o2 = o;   // curl of cross: rhs kernel with omega = 0, dt = an = 1
-    o2.omega = zero; o2.a = d_n; o2.lap_coef = 0; o2.an = 1; o2.bn = 0; o2.dt = 1; o2.w_coef = 0;
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
-    CK(hipMemcpyAsync(d + 1, &o2, sizeof(o2), hipMemcpyHostToDevice, c->c.stream));
+    CKR(mem.put(&d, o, 2));
+    CKR(mem.flush());
     launch_vel(d, 1, ns, c->c.stream);
     for (int lev = 0; lev < ngrid; ++lev) launch_cross(d, 1, nf1, lev, c->c.stream);
     launch_rhs(d + 1, 1, ns, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
-    return 0;
+    return mem.finish();
 }
 
 int ibpm_cross_product(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, const double* d_q, const double* d_w,
                        double* d_out) {
-    DevMem mem;
+    CKR(check_grid(nx, ny, ngrid));
+    OpScope mem(&c->c);
     FlowOps o{};
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
     const long nf1 = 2L * nx * ny + nx + ny;
     o.q = const_cast<double*>(d_q);
     o.omega = const_cast<double*>(d_w);
     o.cross = d_out;
-    CKR(ops_common(c, nx, ny, ngrid, dx, o, mem));
+    CKR(ops_common(nx, ny, ngrid, dx, o, mem));
     FlowOps* d = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
+    CKR(mem.put(&d, &o, 1));
+    CKR(mem.flush());
     launch_vel(d, 1, ns, c->c.stream);
     for (int lev = 0; lev < ngrid; ++lev) launch_cross(d, 1, nf1, lev, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
-    return 0;
+    return mem.finish();
 }
 
 // Scalar::coarsify in place over levels 1..ngrid-1, in order (Scalar.cc:46-63):
@@ -3337,27 +3481,25 @@ static void coarsify_in_place(int nx, int ngrid, const CoarsifyJob* d_jobs, hipS
 int ibpm_cross_flux_flux(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, const double* d_q1,
                          const double* d_q2, double* d_out) {
     CKR(check_grid(nx, ny, ngrid));
-    DevMem mem;
+    OpScope mem(&c->c);
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
     CrossFFOps o{nx, ny, ngrid, dx, d_q1, d_q2, d_out};
     std::vector<CoarsifyJob> jobs(ngrid);
     for (int lev = 0; lev < ngrid; ++lev) jobs[lev] = CoarsifyJob{nx, ny, lev, d_out, d_out, nullptr};
     CrossFFOps* d = nullptr;
     CoarsifyJob* dj = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CKR(mem.alloc(&dj, ngrid));
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
-    CK(hipMemcpyAsync(dj, jobs.data(), sizeof(CoarsifyJob) * ngrid, hipMemcpyHostToDevice, c->c.stream));
+    CKR(mem.put(&d, &o, 1));
+    CKR(mem.put(&dj, jobs.data(), ngrid));
+    CKR(mem.flush());
     launch_cross_ff(d, 1, ns, c->c.stream);
     coarsify_in_place(nx, ngrid, dj, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
-    return 0;
+    return mem.finish();
 }
 
 int ibpm_rhs(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, double dt, double nu, double an, double bn,
              const double* d_q, const double* d_w, const double* d_nprev, double* d_a, double* d_n) {
-    DevMem mem;
+    CKR(check_grid(nx, ny, ngrid));
+    OpScope mem(&c->c);
     FlowOps o{};
     const long ns = (long)(nx - 1) * (ny - 1) * ngrid;
     const long nf1 = 2L * nx * ny + nx + ny;
@@ -3368,28 +3510,27 @@ int ibpm_rhs(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, double dt, doubl
     o.lap_coef = 0.5 * nu * (an + bn); o.an = an; o.bn = bn; o.dt = dt; o.w_coef = 1.0;
     o.use_nprev = bn != 0;
     o.nprev_valid = d_nprev != nullptr;   // no N_prev yet: the reference uses N (IBSolver.cc:173-177)
-    CKR(ops_common(c, nx, ny, ngrid, dx, o, mem));
+    CKR(ops_common(nx, ny, ngrid, dx, o, mem));
+    FlowOps* d = nullptr;
+    CKR(mem.put(&d, &o, 1));
+    CKR(mem.flush());
     if (d_nprev && d_nprev != d_n)
         CK(hipMemcpyAsync(d_n, d_nprev, sizeof(double) * ns, hipMemcpyDeviceToDevice, c->c.stream));
-    FlowOps* d = nullptr;
-    CKR(mem.alloc(&d, 1));
-    CK(hipMemcpyAsync(d, &o, sizeof(o), hipMemcpyHostToDevice, c->c.stream));
     launch_vel(d, 1, ns, c->c.stream);
     for (int lev = 0; lev < ngrid; ++lev) launch_cross(d, 1, nf1, lev, c->c.stream);
     launch_rhs(d, 1, ns, c->c.stream);
-    CK(hipStreamSynchronize(c->c.stream));
-    CK(hipGetLastError());
-    return 0;
+    return mem.finish();
 }
 
 int ibpm_flux_from_vorticity(ibpm_ctx* c, int nx, int ny, int ngrid, double dx, double u0, double v0,
                              const double* d_w, double* d_q) {
     CKR(check_grid(nx, ny, ngrid));
-    DevMem mem;
+    OpScope mem(&c->c);
     double* psi = nullptr;
     CKR(mem.alloc(&psi, (size_t)(nx - 1) * (ny - 1) * ngrid));
-    CKR(solve_common(c, 0, nx, ny, ngrid, dx, 0.0, d_w, nullptr, psi, -1.0));   // L psi = -coarsify(omega)
-    return ibpm_curl_scalar(c, nx, ny, ngrid, dx, u0, v0, psi, d_q);
+    CKR(enqueue_solve(&c->c, mem, 0, nx, ny, ngrid, dx, 0.0, d_w, nullptr, psi, -1.0));   // L psi = -coarsify(omega)
+    CKR(enqueue_curl(&c->c, mem, nx, ny, ngrid, dx, u0, v0, psi, d_q));
+    return mem.finish();
 }
 
 }  // extern "C"
