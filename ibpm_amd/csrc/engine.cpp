@@ -753,7 +753,7 @@ struct Flow {
     long ns, nf;
     bool cg = false;
     // device fields
-    double *omega, *q, *nprev, *a, *wstar, *psi, *c, *U, *V, *cross, *R, *T1, *T2, *bcv, *mt;
+    double *omega, *q, *nprev, *a, *wstar, *psi, *c, *R, *T1, *T2, *bcv, *edge, *mt;
     double *f, *rhs, *b, *cg_r, *cg_d, *cg_q, *cg_state, *hist, *unit, *mcol;
     // models: base states (linear models; one per phase of the periodic one),
     // the adjoint's Flux x Flux cross product, SFD's filtered state
@@ -839,6 +839,7 @@ struct ibpm_batch {
     double an[4], bn[4], cn[4];
     bool all_stationary = true, any_cg = false, initialized = false, any_ubf = false;
     bool any_periodic = false, any_adjoint = false;
+    bool any_plain = false, any_other = false;   // flows of the nonlinear model, of others
     // the solves keep T of every level and run passes 1 and 3 over all levels
     // at once (kAllLevelBytes)
     bool all_levels = false;
@@ -888,7 +889,8 @@ struct ibpm_batch {
     bool use_graph = false;
     hipGraphExec_t graph = nullptr;
     ibpmg::Probe* probe = nullptr;
-    double bytes_vel = 0, bytes_cross = 0, bytes_rhs = 0, bytes_curlq = 0;
+    double bytes_rhs = 0, bytes_curlq = 0;
+    int max_advect = 0, max_rim = 0;   // most advect_blocks and advect_rim_blocks of a flow
     int cg_chunk = 4;
     // learned warm start (learn.hip)
     int warm_mode = 1;            // 0 zero, 1 previous force (reference), 2 learned
@@ -1163,9 +1165,10 @@ static int upload_constraint(hipStream_t s, Flow& F, HostStage& st) {
 // u, v, w on the device and the constraint for them.
 static int move_base_flow(ibpm_batch* B, Flow& F, double t) {
     hipStream_t s = B->ctx->c.stream;
+    const double u0 = F.bf.u, v0 = F.bf.v, w0 = F.bf.w;
     F.bf.move(t);
     CKR(stage_begin(s, F.stage));
-    const double uvw[3] = {F.bf.u, F.bf.v, F.bf.w};
+    const double uvw[6] = {F.bf.u, F.bf.v, F.bf.w, u0, v0, w0};   // FlowOps::bf
     CKR(stage_upload(s, F.stage, F.bf_dev, uvw, sizeof uvw));
     return upload_constraint(s, F, F.stage);
 }
@@ -1354,10 +1357,10 @@ static int alloc_flow(ibpm_batch* B, Flow& F) {
     const long ns = F.ns * F.L, nf = F.nf * F.L;
     CKR(m.alloc(&F.omega, ns)); CKR(m.alloc(&F.q, nf)); CKR(m.alloc(&F.nprev, ns));
     CKR(m.alloc(&F.a, ns)); CKR(m.alloc(&F.wstar, ns)); CKR(m.alloc(&F.psi, ns));
-    CKR(m.alloc(&F.c, ns)); CKR(m.alloc(&F.U, ns)); CKR(m.alloc(&F.V, ns));
-    CKR(m.alloc(&F.cross, nf)); CKR(m.alloc(&F.R, ns)); CKR(m.alloc(&F.T1, (size_t)(F.nx - 1) * t1_ld(F.ny - 1) * (B->all_levels ? F.L : 1)));
+    CKR(m.alloc(&F.c, ns)); CKR(m.alloc(&F.R, ns)); CKR(m.alloc(&F.T1, (size_t)(F.nx - 1) * t1_ld(F.ny - 1) * (B->all_levels ? F.L : 1)));
     CKR(m.alloc(&F.T2, (size_t)(F.nx - 1) * t1_ld(F.ny - 1))); CKR(m.alloc(&F.mt, ns));
     CKR(m.alloc(&F.bcv, bcv_size(F.nx, F.ny) * F.L));
+    CKR(m.alloc(&F.edge, advect_edge(F.nx, F.ny, F.L)));
     const int n = 2 * F.nb + 1;
     CKR(m.alloc(&F.f, n)); CKR(m.alloc(&F.rhs, n)); CKR(m.alloc(&F.b, n));
     CKR(m.alloc(&F.cg_r, n)); CKR(m.alloc(&F.cg_d, n)); CKR(m.alloc(&F.cg_q, n));
@@ -1371,7 +1374,7 @@ static int alloc_flow(ibpm_batch* B, Flow& F) {
     CKR(m.alloc(&F.node_idx, 4 * cap)); CKR(m.alloc(&F.old_idx, 4 * cap)); CKR(m.alloc(&F.node_nbr, 4 * cap));
     {   // staging for the lists (capacities above), the constraint and the base flow
         const size_t bytes = sizeof(int) * (n + 1) + (sizeof(int) + sizeof(double)) * 2 * cap + sizeof(int) * (cap + 1) +
-                             sizeof(int) * 8 * cap + sizeof(int4) * 4 * cap + sizeof(double) * (n + 4) +
+                             sizeof(int) * 8 * cap + sizeof(int4) * 4 * cap + sizeof(double) * (n + 7) +
                              sizeof(double) * kESep * n + 13 * 256;
         CK(hipHostMalloc((void**)&F.stage.p, bytes, hipHostMallocDefault));
         F.stage.cap = bytes;
@@ -1449,7 +1452,7 @@ static int build_plans(ibpm_batch* B) {
         for (auto& F : B->flows) {
             FlowOps o{};
             o.nx = F.nx; o.ny = F.ny; o.L = F.L; o.dx = F.dx;
-            o.q = F.q; o.omega = F.omega; o.U = F.U; o.V = F.V; o.cross = F.cross;
+            o.q = F.q; o.omega = F.omega;
             o.a = F.a; o.nprev = F.nprev; o.psi = F.psi;
             const double nu = 1. / F.p.reynolds;   // NavierStokesModel::getAlpha
             o.lap_coef = 0.5 * nu * (B->an[i] + B->bn[i]);
@@ -1467,12 +1470,12 @@ static int build_plans(ibpm_batch* B) {
             o.xc = F.bf.xc; o.yc = F.bf.yc;
             o.xoff = F.p.xoffset; o.yoff = F.p.yoffset;
             o.model = F.p.model;
-            o.skip_central = F.p.model == 0;
             o.q0b = F.bq.empty() ? nullptr : F.bq[0];
             o.w0b = F.bw.empty() ? nullptr : F.bw[0];
             o.sff = F.sff;
             o.what = F.what;
             o.sfd_prev = F.sfd_prev;
+            o.edge = F.edge;
             o.sfd_chi = F.p.sfd_chi;
             o.sfd_inv_delta = F.p.model == 4 ? 1.0 / F.p.sfd_delta : 0.0;   // Array.h:335-340
             B->h_fops[i].push_back(o);
@@ -1931,24 +1934,26 @@ static void enqueue_M(ibpm_batch* B, int i, RegOps* smear, hipStream_t s,
 // Nonlinear term and right-hand side a of substep i (IBSolver.cc:144,169-183).
 static void enqueue_rhs(ibpm_batch* B, int i, hipStream_t s) {
     const int nfl = (int)B->flows.size();
-    int lmax = 0;
-    for (auto& F : B->flows) lmax = std::max(lmax, F.L);
     Probe* pr = B->probe;
     if (B->cff_n) {   // adjoint flows: s = CrossProduct(q0, q), coarsified (VectorOperations.cc:465-486)
         launch_cross_ff(B->d_cff, B->cff_n, B->max_ns_all, s);
         for (size_t lev = 1; lev < B->d_cffc.size(); ++lev)
             if (B->cffc_n[lev]) launch_coarsify(B->d_cffc[lev], B->cffc_n[lev], B->cffc_rows, s);
     }
-    timed(pr, K_VEL, B->bytes_vel, s, [&] { launch_vel(B->d_fops[i], nfl, B->max_ns_all, s); });
-    for (int lev = 0; lev < lmax; ++lev)
-        timed(pr, K_CROSS, B->bytes_cross / lmax, s, [&] { launch_cross(B->d_fops[i], nfl, B->max_nf, lev, s); });
-    timed(pr, K_RHS, B->bytes_rhs, s, [&] { launch_rhs(B->d_fops[i], nfl, B->max_ns_all, s); });
+    timed(pr, K_RHS, B->bytes_rhs, s, [&] { launch_advect(B->d_fops[i], nfl, B->max_advect, B->max_rim, B->any_plain, B->any_other, s); });
 }
 
-static void enqueue_refresh(ibpm_batch* B, hipStream_t s) {
-    run_solve(B->S4, s, B->probe);
+static void enqueue_q(ibpm_batch* B, hipStream_t s) {
     timed(B->probe, K_CURLQ, B->bytes_curlq, s,
           [&] { launch_curl_q(B->d_fops[0], (int)B->flows.size(), B->max_cells_all, s); });
+}
+
+// psi of the new vorticity, which the next substep's right-hand side starts
+// from; q = Curl psi + q0 is formed where it is read: at the end of an advance
+// (enqueue_q), and after every substep for the adjoint model's cross product.
+static void enqueue_refresh(ibpm_batch* B, hipStream_t s) {
+    run_solve(B->S4, s, B->probe);
+    if (B->any_adjoint) enqueue_q(B, s);
 }
 
 // The stationary-body (Cholesky) substep: fixed launch sequence.
@@ -1967,7 +1972,7 @@ static void enqueue_substep_chol(ibpm_batch* B, int i, hipStream_t s) {
     timed(pr, K_SMEAR, pr ? reg_bytes(B, true, false) : 0, s,
           [&] { launch_smear_curl(B->d_smear_f[i], nfl, B->max_nodes, s); });   // c = beta B f
     run_solve(B->S3[i], s, pr);                     // omega = omega* - A^-1 c
-    enqueue_refresh(B, s);                          // q = Curl psi + q0
+    enqueue_refresh(B, s);                          // psi of the new omega
 }
 
 static int enqueue_step_chol(ibpm_batch* B, hipStream_t s) {
@@ -3919,6 +3924,7 @@ int ibpm_batch_create(ibpm_ctx* ctx, int nflows, const ibpm_flow_params* params,
             if (F.p.ubf) { set_error("flow %d: the linear models take no unsteady base flow", k); return -1; }
             F.base_mag = 0.0;
         }
+        (F.p.model == 0 ? B->any_plain : B->any_other) = true;
         if (F.p.model == 3) B->any_periodic = true;
         if (F.p.model == 2) B->any_adjoint = true;
         F.cg = !F.geom.stationary || F.p.force_cg;
@@ -3930,18 +3936,17 @@ int ibpm_batch_create(ibpm_ctx* ctx, int nflows, const ibpm_flow_params* params,
         B->max_cells_all = std::max(B->max_cells_all, (long)(F.nx + 1) * (F.ny + 1) * F.L);
         B->max_comp = std::max(B->max_comp, 2 * F.nb);
         B->max_n = std::max(B->max_n, 2 * F.nb);
-        // algorithmic bytes: vel reads omega + q, writes U, V; cross reads U, V
-        // and writes the cross flux; rhs reads cross, omega, N_prev and writes
-        // a, N; curl_q reads psi and writes q.  vel (and rhs, for the
-        // nonlinear model) pass over the nodes strictly inside the coarse
-        // levels' central regions, so their bytes count the other nodes, each
-        // with its share of the level's fluxes
+        // algorithmic bytes: the right-hand side reads psi, omega and N_prev and
+        // writes a and N (linear models also read their base state, the adjoint
+        // its cross product, SFD its filtered state) outside the coarse levels'
+        // central regions; curl_q reads psi and writes q
         const double ncent = (double)(F.nx / 2 - 1) * (F.ny / 2 - 1) * (F.L - 1);
         const double nact = (double)F.ns * F.L - ncent;
         const double fpn = (double)F.nf / F.ns;
-        B->bytes_vel += 8.0 * (3 + fpn) * nact;
-        B->bytes_cross += 8.0 * (2 * F.ns + F.nf) * F.L;
-        B->bytes_rhs += 8.0 * (4 + fpn) * (F.p.model == 0 ? nact : (double)F.ns * F.L);
+        B->max_advect = std::max(B->max_advect, advect_blocks(F.nx, F.ny, F.L));
+        B->max_rim = std::max(B->max_rim, advect_rim_blocks(F.nx, F.ny, F.L));
+        const bool lin = F.p.model >= 1 && F.p.model <= 3;
+        B->bytes_rhs += 8.0 * (5 + (lin ? 1 + fpn : 0) + (F.p.model == 2 || F.p.model == 4 ? 1 : 0)) * nact;
         B->bytes_curlq += 8.0 * (F.ns + F.nf) * F.L;
     }
     double tbytes = 0;
@@ -3950,9 +3955,7 @@ int ibpm_batch_create(ibpm_ctx* ctx, int nflows, const ibpm_flow_params* params,
     for (auto& F : B->flows) {
         F.tstride = B->all_levels ? (long)(F.nx - 1) * t1_ld(F.ny - 1) : 0;
         CKR(alloc_flow(B.get(), F));
-        CKR(B->mem.alloc(&F.bf_dev, 4));
-        const double zero[4] = {0, 0, 0, 0};
-        CKR(upload(F.bf_dev, zero, sizeof zero));
+        CKR(B->mem.alloc(&F.bf_dev, 6));
     }
     if (B->any_cg) {
         for (auto& F : B->flows) F.cg = true;   // one force solver per batch
@@ -4085,6 +4088,7 @@ int ibpm_batch_init(ibpm_batch* B) {
     for (auto& F : B->flows)                             // updateOperators(t0), ibpm.cc:304
         if (F.ubf) CKR(move_base_flow(B, F, B->time));
     enqueue_refresh(B, s);                               // ibpm.cc:304-305
+    enqueue_q(B, s);
     CK(hipStreamSynchronize(s));
     CK(hipGetLastError());
     B->initialized = true;
@@ -4156,6 +4160,7 @@ int ibpm_batch_advance(ibpm_batch* B, int nsteps) {
             F.alpha_hist.push_back(F.force_alpha);
         }
     }
+    if (nsteps > 0 && !B->any_adjoint) enqueue_q(B, s);
     CK(hipStreamSynchronize(s));
     CK(hipGetLastError());
     return 0;
@@ -4228,6 +4233,7 @@ int ibpm_batch_set_omega(ibpm_batch* B, int k, const double* h) {
     if (!F) return -1;
     CK(hipMemcpy(F->omega, h, sizeof(double) * F->ns * F->L, hipMemcpyHostToDevice));
     enqueue_refresh(B, B->ctx->c.stream);
+    enqueue_q(B, B->ctx->c.stream);
     CK(hipStreamSynchronize(B->ctx->c.stream));
     return 0;
 }
@@ -4255,6 +4261,7 @@ int ibpm_batch_set_state(ibpm_batch* B, int k, const double* h_omega, const doub
         F->force_alpha = F->bf.alpha;
     }
     enqueue_refresh(B, B->ctx->c.stream);
+    enqueue_q(B, B->ctx->c.stream);
     CK(hipStreamSynchronize(B->ctx->c.stream));
     return 0;
 }

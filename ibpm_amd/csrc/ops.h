@@ -16,7 +16,9 @@ struct FlowOps {
     int use_nprev, nprev_valid;
     double ubase, vbase;           // uniform base flow (magnitude 1, angle alpha)
     // unsteady base flow (ubf = 1): bf[0..2] = u, v, w of the current base
-    // flux, X (u - w (y - yc)) d and Y (v + w (x - xc)) d at edge (x, y)
+    // flux, X (u - w (y - yc)) d and Y (v + w (x - xc)) d at edge (x, y);
+    // bf[3..5] those before its last move, which the flux that a substep's N
+    // is formed from was refreshed with
     int ubf;
     const double* bf;
     double xc, yc, xoff, yoff;     // centre of rotation; level-0 grid offsets
@@ -28,12 +30,8 @@ struct FlowOps {
     const double *q0b, *w0b, *sff;
     double *what, *sfd_prev;
     double sfd_chi, sfd_inv_delta;
+    double* edge;                  // U and V past the edges of levels 0..L-2 (k_advect_rim)
     int sfd_valid;                 // what holds the filtered state (else: zero in N, omega at the update)
-    // nonlinear-model flows of a batch: a and N are not formed at the nodes
-    // strictly inside a coarse level's central region, which no kernel reads
-    // (the Helmholtz solve and its coarsify chain read the coarsified
-    // right-hand side there, and N there only feeds the next substep's a there)
-    int skip_central;
 };
 
 // CrossProduct(Flux, Flux) of one flow before its coarsify: out = X(q1) Y(q2)
@@ -207,6 +205,14 @@ void launch_vel(const FlowOps* d, int nflows, long max_pts, hipStream_t s);
 void launch_cross(const FlowOps* d, int nflows, long max_nf, int lev, hipStream_t s);
 void launch_cross_ff(const CrossFFOps* d, int nflows, long max_pts, hipStream_t s);
 void launch_rhs(const FlowOps* d, int nflows, long max_pts, hipStream_t s);
+// A batch substep's N and right-hand side from psi, omega and N_prev;
+// max_blocks, max_rim_blocks: the most advect_blocks and advect_rim_blocks of a
+// flow; plain, other: whether it has flows of the nonlinear and of other models.
+size_t advect_edge(int nx, int ny, int L);   // doubles of FlowOps::edge
+int advect_blocks(int nx, int ny, int L);
+int advect_rim_blocks(int nx, int ny, int L);
+void launch_advect(const FlowOps* d, int nflows, int max_blocks, int max_rim_blocks, bool plain, bool other,
+                   hipStream_t s);
 // max_cells_all: (nx + 1)(ny + 1) L of the largest flow
 void launch_curl_q(const FlowOps* d, int nflows, long max_cells_all, hipStream_t s);
 void launch_interp(const RegOps* d, int nflows, int max_comp, hipStream_t s);

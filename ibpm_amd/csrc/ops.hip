@@ -62,10 +62,36 @@ __device__ inline double curl_y(const Lay& g, const double* F, int lev, int i, i
     return F[g.s(lev, i, j)] - F[g.s(lev, i + 1, j)];
 }
 
+// q0 on the level's X flux (., j) and Y flux (i, .): the uniform base flow
+// (Flux.cc:79-99) or the unsteady one, free stream plus rotation about the body
+// centre at the edge coordinates of each level (Flux.cc:101-129,
+// Grid.cc:104-139), bf its u, v, w.
+__device__ inline double base_x(const FlowOps& F, const double* bf, int lev, int j) {
+    const double d = F.dx * (1 << lev);
+    if (!F.ubf) return F.ubase * d;
+    // level offsets: offset + 0.5 (shift - 1) (2^lev - 1) n dx with shift 0
+    const double y = (F.yoff - 0.5 * ((1 << lev) - 1) * (F.ny * F.dx)) + (j + 0.5) * d;
+    return (bf[0] - bf[2] * (y - F.yc)) * d;
+}
+__device__ inline double base_y(const FlowOps& F, const double* bf, int lev, int i) {
+    const double d = F.dx * (1 << lev);
+    if (!F.ubf) return F.vbase * d;
+    const double x = (F.xoff - 0.5 * ((1 << lev) - 1) * (F.nx * F.dx)) + (i + 0.5) * d;
+    return (bf[1] + bf[2] * (x - F.xc)) * d;
+}
+
+struct FluxField {
+    const Lay& g;
+    const double* q;
+    __device__ double x(int lev, int i, int j) const { return q[g.fx(lev, i, j)]; }
+    __device__ double y(int lev, int i, int j) const { return q[g.fy(lev, i, j)]; }
+};
 // FluxToXVelocity / FluxToYVelocity at one node (VectorOperations.cc:488-665).
 // The central nodes of coarse levels are never read downstream and are 0.
-__device__ inline double xvel(const Lay& g, const double* q, double dx0, int lev, int i, int j) {
-    if (lev == 0) return (q[g.fx(0, i, j)] + q[g.fx(0, i, j - 1)]) * (1. / (2 * dx0));
+// Q gives the fluxes.
+template <class Q>
+__device__ inline double xvel(const Lay& g, const Q& q, double dx0, int lev, int i, int j) {
+    if (lev == 0) return (q.x(0, i, j) + q.x(0, i, j - 1)) * (1. / (2 * dx0));
     const int ilo = nx_ext(g.nx), ihi = g.nx / 2 + nx_ext(g.nx);
     const int jlo = nx_ext(g.ny), jhi = g.ny / 2 + nx_ext(g.ny);
     const double bydx = 1. / (dx0 * (1 << lev));
@@ -75,28 +101,29 @@ __device__ inline double xvel(const Lay& g, const double* q, double dx0, int lev
     const int f = lev - 1;
     if (onI && onJ) {   // corners F
         if (j == jlo) {
-            const double c = (i == ilo) ? q[g.fx(f, 1, 0)] : q[g.fx(f, g.nx - 1, 0)];
-            return (q[g.fx(lev, i, j - 1)] * 8. / 15 + q[g.fx(lev, i, j)] * 6. / 15 + c * 2. / 15) * bydx;
+            const double c = (i == ilo) ? q.x(f, 1, 0) : q.x(f, g.nx - 1, 0);
+            return (q.x(lev, i, j - 1) * 8. / 15 + q.x(lev, i, j) * 6. / 15 + c * 2. / 15) * bydx;
         }
-        const double c = (i == ilo) ? q[g.fx(f, 1, g.ny - 1)] : q[g.fx(f, g.nx - 1, g.ny - 1)];
-        return (q[g.fx(lev, i, j)] * 8. / 15 + q[g.fx(lev, i, j - 1)] * 6. / 15 + c * 2. / 15) * bydx;
+        const double c = (i == ilo) ? q.x(f, 1, g.ny - 1) : q.x(f, g.nx - 1, g.ny - 1);
+        return (q.x(lev, i, j) * 8. / 15 + q.x(lev, i, j - 1) * 6. / 15 + c * 2. / 15) * bydx;
     }
     if (inI && onJ) {   // interfaces E
         const int ii = (i - ilo) * 2;
         if (j == jlo) {
             const int jj = 0;
-            return (q[g.fx(lev, i, jlo - 1)] * 2. / 3 + q[g.fx(f, ii, jj)] * 1. / 3
-                    + (q[g.fx(f, ii - 1, jj)] + q[g.fx(f, ii + 1, jj)]) * 1. / 6) * bydx;
+            return (q.x(lev, i, jlo - 1) * 2. / 3 + q.x(f, ii, jj) * 1. / 3
+                    + (q.x(f, ii - 1, jj) + q.x(f, ii + 1, jj)) * 1. / 6) * bydx;
         }
         const int jj = (jhi - jlo) * 2;
-        return (q[g.fx(lev, i, jhi)] * 2. / 3 + q[g.fx(f, ii, jj - 1)] * 1. / 3
-                + (q[g.fx(f, ii - 1, jj - 1)] + q[g.fx(f, ii + 1, jj - 1)]) * 1. / 6) * bydx;
+        return (q.x(lev, i, jhi) * 2. / 3 + q.x(f, ii, jj - 1) * 1. / 3
+                + (q.x(f, ii - 1, jj - 1) + q.x(f, ii + 1, jj - 1)) * 1. / 6) * bydx;
     }
-    return (q[g.fx(lev, i, j)] + q[g.fx(lev, i, j - 1)]) * 0.5 * bydx;
+    return (q.x(lev, i, j) + q.x(lev, i, j - 1)) * 0.5 * bydx;
 }
 
-__device__ inline double yvel(const Lay& g, const double* q, double dx0, int lev, int i, int j) {
-    if (lev == 0) return (q[g.fy(0, i - 1, j)] + q[g.fy(0, i, j)]) * (1. / (2 * dx0));
+template <class Q>
+__device__ inline double yvel(const Lay& g, const Q& q, double dx0, int lev, int i, int j) {
+    if (lev == 0) return (q.y(0, i - 1, j) + q.y(0, i, j)) * (1. / (2 * dx0));
     const int ilo = nx_ext(g.nx), ihi = g.nx / 2 + nx_ext(g.nx);
     const int jlo = nx_ext(g.ny), jhi = g.ny / 2 + nx_ext(g.ny);
     const double bydx = 1. / (dx0 * (1 << lev));
@@ -106,81 +133,110 @@ __device__ inline double yvel(const Lay& g, const double* q, double dx0, int lev
     const int f = lev - 1;
     if (onI && onJ) {   // corners F
         if (i == ilo) {
-            const double c = (j == jlo) ? q[g.fy(f, 0, 1)] : q[g.fy(f, 0, g.ny - 1)];
-            return (q[g.fy(lev, i - 1, j)] * 8. / 15 + q[g.fy(lev, i, j)] * 6. / 15 + c * 2. / 15) * bydx;
+            const double c = (j == jlo) ? q.y(f, 0, 1) : q.y(f, 0, g.ny - 1);
+            return (q.y(lev, i - 1, j) * 8. / 15 + q.y(lev, i, j) * 6. / 15 + c * 2. / 15) * bydx;
         }
-        const double c = (j == jlo) ? q[g.fy(f, g.nx - 1, 1)] : q[g.fy(f, g.nx - 1, g.ny - 1)];
-        return (q[g.fy(lev, i, j)] * 8. / 15 + q[g.fy(lev, i - 1, j)] * 6. / 15 + c * 2. / 15) * bydx;
+        const double c = (j == jlo) ? q.y(f, g.nx - 1, 1) : q.y(f, g.nx - 1, g.ny - 1);
+        return (q.y(lev, i, j) * 8. / 15 + q.y(lev, i - 1, j) * 6. / 15 + c * 2. / 15) * bydx;
     }
     if (onI && inJ) {   // interfaces E
         const int jj = (j - jlo) * 2;
         if (i == ilo) {
             const int ii = 0;
-            return (q[g.fy(lev, ilo - 1, j)] * 2. / 3 + q[g.fy(f, ii, jj)] * 1. / 3
-                    + (q[g.fy(f, ii, jj - 1)] + q[g.fy(f, ii, jj + 1)]) * 1. / 6) * bydx;
+            return (q.y(lev, ilo - 1, j) * 2. / 3 + q.y(f, ii, jj) * 1. / 3
+                    + (q.y(f, ii, jj - 1) + q.y(f, ii, jj + 1)) * 1. / 6) * bydx;
         }
         const int ii = (ihi - ilo) * 2;
-        return (q[g.fy(lev, ihi, j)] * 2. / 3 + q[g.fy(f, ii - 1, jj)] * 1. / 3
-                + (q[g.fy(f, ii - 1, jj - 1)] + q[g.fy(f, ii - 1, jj + 1)]) * 1. / 6) * bydx;
+        return (q.y(lev, ihi, j) * 2. / 3 + q.y(f, ii - 1, jj) * 1. / 3
+                + (q.y(f, ii - 1, jj - 1) + q.y(f, ii - 1, jj + 1)) * 1. / 6) * bydx;
     }
-    return (q[g.fy(lev, i, j)] + q[g.fy(lev, i - 1, j)]) * 0.5 * bydx;
+    return (q.y(lev, i, j) + q.y(lev, i - 1, j)) * 0.5 * bydx;
+}
+
+// One component of N's cross product at a node, from its own and its base
+// state's velocity (v, v0), vorticity (w, w0) and the sign of the component
+// (-1 for U = -omega u, +1 for V = omega v; CrossProduct,
+// VectorOperations.cc:438-457):
+//   linear and periodic models, LinearizedIBSolver::N (IBSolver.cc:211-216):
+//     CrossProduct(q0, omega) + CrossProduct(q, omega0), summed per node
+//   adjoint, AdjointIBSolver::N (IBSolver.cc:218-222): -CrossProduct(q, omega0),
+//     so that k_rhs's Curl(cross) is the subtracted term
+__device__ inline double cross_node(int model, double sign, double v, double w, double v0, double w0) {
+    if (model == 1 || model == 3) return sign * (v0 * w) + sign * (v * w0);
+    if (model == 2) return -sign * (v * w0);
+    return sign * (v * w);
+}
+__device__ inline bool has_base(int model) { return model >= 1 && model <= 3; }
+
+template <class Q>
+__device__ inline double node_u(const FlowOps& F, const Lay& g, const Q& q, int lev, int i, int j) {
+    const long k = g.s(lev, i, j);
+    const double v = xvel(g, q, F.dx, lev, i, j), w = gin(F.omega)[k];
+    if (!has_base(F.model)) return cross_node(F.model, -1.0, v, w, 0.0, 0.0);
+    const double v0 = F.model == 2 ? 0.0 : xvel(g, FluxField{g, F.q0b}, F.dx, lev, i, j);
+    return cross_node(F.model, -1.0, v, w, v0, gin(F.w0b)[k]);
+}
+template <class Q>
+__device__ inline double node_v(const FlowOps& F, const Lay& g, const Q& q, int lev, int i, int j) {
+    const long k = g.s(lev, i, j);
+    const double v = yvel(g, q, F.dx, lev, i, j), w = gin(F.omega)[k];
+    if (!has_base(F.model)) return cross_node(F.model, 1.0, v, w, 0.0, 0.0);
+    const double v0 = F.model == 2 ? 0.0 : yvel(g, FluxField{g, F.q0b}, F.dx, lev, i, j);
+    return cross_node(F.model, 1.0, v, w, v0, gin(F.w0b)[k]);
 }
 
 // XVelocityToFlux / YVelocityToFlux at one flux of level lev
-// (VectorOperations.cc:669-915).  C holds the already finished finer level of
-// the output, used by the coarse-level region G.
-__device__ inline double xflux_from(const Lay& g, const double* S, const double* C, double dx0,
-                                    int lev, int i, int j) {
+// (VectorOperations.cc:669-915) outside the coarse levels' region G, where the
+// finer level's fluxes are summed.  S gives the node values.
+struct NodeField {
+    const Lay& g;
+    const double* s;
+    __device__ double operator()(int lev, int i, int j) const { return gin(s)[g.s(lev, i, j)]; }
+};
+template <class S>
+__device__ inline double xflux_from(const Lay& g, const S& s, double dx0, int lev, int i, int j) {
     const double dx = dx0 * (1 << lev);
     const int nx2 = nx_ext(g.nx), ny2 = nx_ext(g.ny);
     if (i == 0 || i == g.nx) {   // A
         if (lev == g.L - 1) return 0.0;
         const int ic = (i == 0) ? nx2 : g.nx / 2 + nx2;
         const int jj = j / 2 + ny2;
-        const double a = gin(S)[g.s(lev + 1, ic, jj)], b = gin(S)[g.s(lev + 1, ic, jj + 1)];
+        const double a = s(lev + 1, ic, jj), b = s(lev + 1, ic, jj + 1);
         return (j & 1) ? (0.25 * a + 0.75 * b) * dx : (0.75 * a + 0.25 * b) * dx;
     }
     if (j == 0 || j == g.ny - 1) {   // C
         const int jin = (j == 0) ? 1 : g.ny - 1;
-        const double s0 = gin(S)[g.s(lev, i, jin)];
+        const double s0 = s(lev, i, jin);
         if (lev == g.L - 1) return s0 * 0.5 * dx;
         const int jc = (j == 0) ? ny2 : g.ny / 2 + ny2;
         const int ii = i / 2 + nx2;
-        if ((i & 1) == 0) return (s0 + gin(S)[g.s(lev + 1, ii, jc)]) * 0.5 * dx;
-        return (0.5 * s0 + 0.25 * gin(S)[g.s(lev + 1, ii, jc)] + 0.25 * gin(S)[g.s(lev + 1, ii + 1, jc)]) * dx;
+        if ((i & 1) == 0) return (s0 + s(lev + 1, ii, jc)) * 0.5 * dx;
+        return (0.5 * s0 + 0.25 * s(lev + 1, ii, jc) + 0.25 * s(lev + 1, ii + 1, jc)) * dx;
     }
-    if (lev > 0 && i > nx2 && i < g.nx / 2 + nx2 && j >= ny2 && j < g.ny / 2 + ny2) {   // G
-        const int ii = 2 * (i - nx2), jj = 2 * (j - ny2);
-        return gin(C)[g.fx(lev - 1, ii, jj)] + gin(C)[g.fx(lev - 1, ii, jj + 1)];
-    }
-    return (gin(S)[g.s(lev, i, j)] + gin(S)[g.s(lev, i, j + 1)]) * 0.5 * dx;
+    return (s(lev, i, j) + s(lev, i, j + 1)) * 0.5 * dx;
 }
 
-__device__ inline double yflux_from(const Lay& g, const double* S, const double* C, double dx0,
-                                    int lev, int i, int j) {
+template <class S>
+__device__ inline double yflux_from(const Lay& g, const S& s, double dx0, int lev, int i, int j) {
     const double dx = dx0 * (1 << lev);
     const int nx2 = nx_ext(g.nx), ny2 = nx_ext(g.ny);
     if (j == 0 || j == g.ny) {   // A
         if (lev == g.L - 1) return 0.0;
         const int jc = (j == 0) ? ny2 : g.ny / 2 + ny2;
         const int ii = i / 2 + nx2;
-        const double a = gin(S)[g.s(lev + 1, ii, jc)], b = gin(S)[g.s(lev + 1, ii + 1, jc)];
+        const double a = s(lev + 1, ii, jc), b = s(lev + 1, ii + 1, jc);
         return (i & 1) ? (0.25 * a + 0.75 * b) * dx : (0.75 * a + 0.25 * b) * dx;
     }
     if (i == 0 || i == g.nx - 1) {   // C
         const int iin = (i == 0) ? 1 : g.nx - 1;
-        const double s0 = gin(S)[g.s(lev, iin, j)];
+        const double s0 = s(lev, iin, j);
         if (lev == g.L - 1) return s0 * 0.5 * dx;
         const int ic = (i == 0) ? nx2 : g.nx / 2 + nx2;
         const int jj = j / 2 + ny2;
-        if ((j & 1) == 0) return (s0 + gin(S)[g.s(lev + 1, ic, jj)]) * 0.5 * dx;
-        return (0.5 * s0 + 0.25 * gin(S)[g.s(lev + 1, ic, jj)] + 0.25 * gin(S)[g.s(lev + 1, ic, jj + 1)]) * dx;
+        if ((j & 1) == 0) return (s0 + s(lev + 1, ic, jj)) * 0.5 * dx;
+        return (0.5 * s0 + 0.25 * s(lev + 1, ic, jj) + 0.25 * s(lev + 1, ic, jj + 1)) * dx;
     }
-    if (lev > 0 && j > ny2 && j < g.ny / 2 + ny2 && i >= nx2 && i < g.nx / 2 + nx2) {   // G
-        const int ii = 2 * (i - nx2), jj = 2 * (j - ny2);
-        return gin(C)[g.fy(lev - 1, ii, jj)] + gin(C)[g.fy(lev - 1, ii + 1, jj)];
-    }
-    return (gin(S)[g.s(lev, i, j)] + gin(S)[g.s(lev, i + 1, j)]) * 0.5 * dx;
+    return (s(lev, i, j) + s(lev, i + 1, j)) * 0.5 * dx;
 }
 
 // ------------------------------------------------------------- kernels
@@ -201,40 +257,8 @@ __global__ void __launch_bounds__(kThreads) k_vel(const FlowOps* __restrict__ fl
     if (lev >= 1 && i > nx_ext(g.nx) && i < g.nx / 2 + nx_ext(g.nx) && j > nx_ext(g.ny) &&
         j < g.ny / 2 + nx_ext(g.ny))
         return;
-    const double w = gin(F.omega)[t];
-    double u, v;
-    if (F.model == 1 || F.model == 3) {
-        // LinearizedIBSolver::N (IBSolver.cc:211-216): the velocities of
-        // CrossProduct(q0, omega) + CrossProduct(q, omega0), summed per node
-        const double w0 = gin(F.w0b)[t];
-        double u1 = xvel(g, F.q0b, F.dx, lev, i, j);
-        u1 *= w;
-        u1 *= -1;
-        double u2 = xvel(g, F.q, F.dx, lev, i, j);
-        u2 *= w0;
-        u2 *= -1;
-        double v1 = yvel(g, F.q0b, F.dx, lev, i, j);
-        v1 *= w;
-        double v2 = yvel(g, F.q, F.dx, lev, i, j);
-        v2 *= w0;
-        u = u1 + u2;
-        v = v1 + v2;
-    } else if (F.model == 2) {
-        // AdjointIBSolver::N (IBSolver.cc:218-222): -CrossProduct(q, omega0),
-        // so that k_rhs's Curl(cross) is the subtracted term
-        const double w0 = gin(F.w0b)[t];
-        u = xvel(g, F.q, F.dx, lev, i, j);
-        u *= w0;
-        v = yvel(g, F.q, F.dx, lev, i, j);
-        v *= w0;
-        v *= -1;
-    } else {
-        u = xvel(g, F.q, F.dx, lev, i, j);
-        u *= w;
-        u *= -1;
-        v = yvel(g, F.q, F.dx, lev, i, j);
-        v *= w;
-    }
+    const FluxField q{g, F.q};
+    const double u = node_u(F, g, q, lev, i, j), v = node_v(F, g, q, lev, i, j);
     gout(F.U)[t] = u;
     gout(F.V)[t] = v;
 }
@@ -252,8 +276,9 @@ __global__ void __launch_bounds__(kThreads) k_cross_ff(const CrossFFOps* __restr
     const int lev = (int)((unsigned)t / ns);
     const unsigned r = (unsigned)t - lev * ns;
     const int i = (int)(r / ny1) + 1, j = (int)(r % ny1) + 1;
-    const double a = xvel(g, F.q1, F.dx, lev, i, j) * yvel(g, F.q2, F.dx, lev, i, j);
-    const double b = xvel(g, F.q2, F.dx, lev, i, j) * yvel(g, F.q1, F.dx, lev, i, j);
+    const FluxField q1{g, F.q1}, q2{g, F.q2};
+    const double a = xvel(g, q1, F.dx, lev, i, j) * yvel(g, q2, F.dx, lev, i, j);
+    const double b = xvel(g, q2, F.dx, lev, i, j) * yvel(g, q1, F.dx, lev, i, j);
     gout(F.out)[t] = a - b;
 }
 
@@ -307,8 +332,8 @@ __device__ inline double cross_value(const FlowOps& F, const Lay& g, int lev, co
     const double dx = F.dx * (1 << lev);
     const double sum = x0 + x1, mean = sum * 0.5 * dx;
     const double mc = a.central ? 1.0 : 0.0, md = (a.edge || a.central) ? 0.0 : 1.0;
-    const double edge = a.edge ? (a.xflux ? xflux_from(g, F.V, F.cross, F.dx, lev, a.i, a.j)
-                                          : yflux_from(g, F.U, F.cross, F.dx, lev, a.i, a.j))
+    const double edge = a.edge ? (a.xflux ? xflux_from(g, NodeField{g, F.V}, F.dx, lev, a.i, a.j)
+                                          : yflux_from(g, NodeField{g, F.U}, F.dx, lev, a.i, a.j))
                                : 0.0;
     return (sum * mc + mean * md) + edge;   // exactly one of the three terms is kept
 }
@@ -331,9 +356,49 @@ __global__ void __launch_bounds__(kThreads) k_cross(const FlowOps* __restrict__ 
     if (two) out[t0 + 1] = vb;
 }
 
-// N = Curl(cross) (IBSolver.cc:205-209) and the right-hand side
-// a = omega + dt (c_L Lap(omega) + a_n N + b_n N_prev) (IBSolver.cc:169-183),
-// Lap = -Curl(Curl(.)) (VectorOperations.cc:133-140).  N replaces N_prev.
+// The substep's outputs at node t of level lev, (i, j): N from Curl(cross) and
+// the model's other terms, and the right-hand side a = omega + dt (c_L
+// Lap(omega) + a_n N + b_n N_prev) (IBSolver.cc:169-183), Lap = -Curl(Curl(.))
+// (VectorOperations.cc:133-140).  c: omega; curl: Curl(cross); np: N_prev (read
+// from its always allocated buffer, used where valid), which N replaces.
+__device__ inline void rhs_node(const FlowOps& F, int model, unsigned tu, double c, double curl, double lap_s, double lap,
+                                double np) {
+    double n = curl;
+    if (model == 2) n = lap_s + n;   // AdjointIBSolver::N = Laplacian(s) - Curl(CrossProduct(q, omega0))
+    double sfd_w = 0.0;   // SFD: the filtered vorticity (zero before the first substep)
+    if (model == 4) {   // SFDSolver::N (IBSolver.cc:238-244): N - chi (omega - omega_hat)
+        sfd_w = F.sfd_valid ? gin(F.what)[tu] : 0.0;
+        n -= F.sfd_chi * (c - sfd_w);
+    }
+    double a = lap * F.lap_coef;
+    a += F.an * n;
+    if (F.use_nprev) a += F.bn * (F.nprev_valid ? np : n);
+    a *= F.dt;
+    a += F.w_coef * c;
+    gout(F.a)[tu] = a;
+    gout(F.nprev)[tu] = n;
+}
+
+// SFD: the filtered state's substep (IBSolver.cc:247-279), omega_hat = omega at
+// the first (it holds at every node).
+__device__ inline void sfd_node(const FlowOps& F, unsigned tu, double c) {
+    const double wh = F.sfd_valid ? gin(F.what)[tu] : c;
+    const double rs = (c - wh) * F.sfd_inv_delta;
+    double av = F.an * rs;
+    if (F.bn != 0) av += F.bn * (F.nprev_valid ? gin(F.sfd_prev)[tu] : rs);
+    av *= F.dt;
+    gout(F.what)[tu] = wh + av;
+    gout(F.sfd_prev)[tu] = rs;
+}
+
+// Laplacian of a field at a node from its curls, boundary values included.
+__device__ inline double lap_edge(const Lay& g, const double* f, int lev, int i, int j, double bydx2) {
+    return -((curl_y(g, f, lev, i, j) - curl_y(g, f, lev, i - 1, j) + curl_x(g, f, lev, i, j - 1) -
+              curl_x(g, f, lev, i, j)) * bydx2);
+}
+
+// N = Curl(cross) of a stored cross flux and the right-hand side at every node
+// (stand-alone entry points; a batch's substep is k_advect).
 __global__ void __launch_bounds__(kThreads) k_rhs(const FlowOps* __restrict__ flows) {
     const FlowOps& F = flows[blockIdx.y];
     const Lay g{F.nx, F.ny, F.L};
@@ -344,19 +409,14 @@ __global__ void __launch_bounds__(kThreads) k_rhs(const FlowOps* __restrict__ fl
     const int lev = (int)((unsigned)t / ns);
     const unsigned r = (unsigned)t - lev * ns;
     const int i = (int)(r / ny1) + 1, j = (int)(r % ny1) + 1;
-    if (F.skip_central && lev >= 1 && i > nx_ext(g.nx) && i < g.nx / 2 + nx_ext(g.nx) && j > nx_ext(g.ny) &&
-        j < g.ny / 2 + nx_ext(g.ny))
-        return;
     const double d = F.dx * (1 << lev);
     const double bydx2 = 1. / (d * d);
     const IBPM_GLOBAL double* C = gin(F.cross);
-    const double* W = F.omega;
-    const IBPM_GLOBAL double* Wg = gin(W);
+    const IBPM_GLOBAL double* Wg = gin(F.omega);
     // Away from the level's edge the curls of Lap(omega) are plain differences
     // of the four neighbours (the general expression, term for term and in the
     // same order).  Their offsets fall back to t itself next to the edge, so
-    // all ten loads below are issued before any value is used; N_prev is read
-    // from its buffer (always allocated) and used only when valid.
+    // all ten loads below are issued before any value is used.
     const bool interior = i >= 2 && i <= g.nx - 2 && j >= 2 && j <= g.ny - 2;
     const unsigned tu = (unsigned)t;
     const unsigned te = interior ? tu + ny1 : tu, tw = interior ? tu - ny1 : tu;
@@ -365,50 +425,366 @@ __global__ void __launch_bounds__(kThreads) k_rhs(const FlowOps* __restrict__ fl
     const double cx0 = C[g.fx(lev, i, j - 1)], cx1 = C[g.fx(lev, i, j)];
     const double c = Wg[tu], e = Wg[te], w = Wg[tw], up = Wg[tn], dn = Wg[ts];
     const double np = gin(F.nprev)[tu];
-    double n = (cy1 - cy0 + cx0 - cx1) * bydx2;
-    if (F.model == 2) {   // AdjointIBSolver::N = Laplacian(s) - Curl(CrossProduct(q, omega0))
-        const IBPM_GLOBAL double* Sg = gin(F.sff);
-        const double sc = Sg[tu], se = Sg[te], sw = Sg[tw], su = Sg[tn], sd = Sg[ts];
-        const double sedge = interior ? 0.0
-                                      : (curl_y(g, F.sff, lev, i, j) - curl_y(g, F.sff, lev, i - 1, j)
-                                         + curl_x(g, F.sff, lev, i, j - 1) - curl_x(g, F.sff, lev, i, j)) * bydx2;
-        double lap_s = ((sc - se) - (sw - sc) + (sc - sd) - (su - sc)) * bydx2 * (interior ? 1.0 : 0.0) + sedge;
-        lap_s *= -1;
-        n = lap_s + n;
+    double lap = -(((c - e) - (w - c) + (c - dn) - (up - c)) * bydx2);
+    if (!interior) lap = lap_edge(g, F.omega, lev, i, j, bydx2);
+    rhs_node(F, 0, tu, c, (cy1 - cy0 + cx0 - cx1) * bydx2, 0.0, lap, np);
+}
+
+// ---------------------------------------------------- a substep's stencils
+// N and the right-hand side a of a batch's substep straight from psi, omega and
+// N_prev: the fluxes q = Curl(psi) + q0, the node velocities, the cross product
+// and its flux are formed on the way (k_vel, k_cross and k_rhs hold them in
+// memory).  What bounds it is HBM: psi, omega, N_prev in, N and a out, 40 B per
+// point, against 144 B in the four passes with k_curl_q that it replaces.  16
+// flows of 1024^2 x 6 levels: 2925 us in four passes, 850 in two (714 for the
+// tiles, 4.5 TB/s of the 40 B; a large copy reaches 4.9); one flow of 400^2 x 4:
+// 44 against 16 us.
+//
+// k_advect takes tiles of kAdvI rows by kAdvJ columns of one level (16 rows: 7.1
+// against 5.4 us at 200^2, where they are too few, 732 against 714 on the 16
+// flows; 128 columns: 760; workgroups in launch order over the XCDs: 908): psi and
+// omega of the tile and one node around it (boundary values past the level's
+// edge) go to LDS, 10 loads per thread in flight together, and a node is formed
+// from 9 psi and 5 omega values there.  U and V past the level's edge, which the
+// fluxes next to it average with (VectorOperations.cc:669-915, region C), are
+// those of the coarser level's nodes; k_advect_rim has left them in F.edge.
+// Nodes strictly inside a coarse level's central region are left out: the
+// Helmholtz solve's pass 1 and its coarsify chain read the coarsified
+// right-hand side there, and N there only feeds the next substep's a there.
+//
+// k_advect_rim, before it, also forms the nodes on the rim of a coarse level's
+// central region and the eight next to its corners, whose velocities and fluxes
+// follow the interface rules: as sums of at most 24 node values, one lane each
+// (rim_term), since one lane through all of a node's rules took 68 us on a 400^2
+// grid, nearly all of it latency.
+constexpr int kAdvI = 8, kAdvJ = 64, kRimLanes = 32;
+
+struct AdvShape {
+    int ti, tj, tiles;   // tiles per level
+    int rim, edge;       // rim nodes of a coarse level, edge values of a level below the coarsest
+};
+__host__ __device__ inline AdvShape adv_shape(int nx, int ny) {
+    AdvShape s;
+    s.ti = (nx - 1 + kAdvI - 1) / kAdvI;
+    s.tj = (ny - 1 + kAdvJ - 1) / kAdvJ;
+    s.tiles = s.ti * s.tj;
+    s.edge = 2 * (ny / 2 + 1) + 2 * (nx / 2 + 1);
+    s.rim = nx + ny + 8;
+    return s;
+}
+
+// Rim node m of a coarse level: rows ex and ex + nx/2 from column ey to ey +
+// ny/2, those columns of the rows between, then the two nodes outside each
+// corner.  False for one that is not of the level (small grids).
+__device__ inline bool rim_node(const Lay& g, int m, int& i, int& j) {
+    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
+    const int wide = g.ny / 2 + 1, tall = g.nx / 2 - 1;
+    if (m < 2 * wide) {
+        i = m < wide ? ex : hx;
+        j = ey + m % wide;
+    } else if (m < 2 * wide + 2 * tall) {
+        m -= 2 * wide;
+        j = m < tall ? ey : hy;
+        i = ex + 1 + m % tall;
+    } else {
+        m -= 2 * wide + 2 * tall;   // 0..7: past the corner along i, then along j
+        const bool e = m & 1, n = m & 2;
+        i = (e ? hx : ex) + (m < 4 ? (e ? 1 : -1) : 0);
+        j = (n ? hy : ey) + (m < 4 ? 0 : (n ? 1 : -1));
     }
-    double sfd_w = 0.0;   // SFD: the filtered vorticity (zero before the first substep)
-    if (F.model == 4) {   // SFDSolver::N (IBSolver.cc:238-244): N - chi (omega - omega_hat)
-        sfd_w = F.sfd_valid ? gin(F.what)[tu] : 0.0;
-        n -= F.sfd_chi * (c - sfd_w);
+    return i >= 1 && i <= g.nx - 1 && j >= 1 && j <= g.ny - 1;
+}
+__device__ inline bool is_rim(const Lay& g, int i, int j) {
+    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
+    const bool oni = i == ex || i == hx, onj = j == ey || j == hy;
+    const bool ini = i >= ex && i <= hx, inj = j >= ey && j <= hy;
+    return (oni && inj) || (onj && ini) || ((i == ex - 1 || i == hx + 1) && onj) || ((j == ey - 1 || j == hy + 1) && oni);
+}
+
+// A node value in a flux or at an edge: coef times U (u) or V at (lev, i, j).
+struct NodeTerm {
+    int lev, i, j;
+    bool u;
+    double coef;   // 0: no term
+};
+
+// Term t (0..2) of an X (x) or Y flux outside region G, i in 1..nx-1 of an X
+// flux and j in 1..ny-1 of a Y flux (the rules of xflux_from / yflux_from).
+__device__ inline NodeTerm flux_term(const Lay& g, double dx0, bool x, int lev, int i, int j, int t) {
+    const double dx = dx0 * (1 << lev);
+    const int along = x ? i : j, across = x ? j : i, n = x ? g.ny : g.nx;
+    if (across == 0 || across == n - 1) {   // next to the edge: the node inside, and the coarser level's
+        const int ea = nx_ext(x ? g.nx : g.ny), ec = nx_ext(n);
+        if (t == 0) {
+            const int in = across == 0 ? 1 : n - 1;
+            return NodeTerm{lev, x ? i : in, x ? in : j, !x, 0.5 * dx};
+        }
+        const int a = along / 2 + ea + (t - 1), c = across == 0 ? ec : n / 2 + ec;
+        const double coef = lev == g.L - 1 || (t == 2 && !(along & 1)) ? 0.0 : (along & 1) ? 0.25 * dx : 0.5 * dx;
+        return NodeTerm{lev + 1, x ? a : c, x ? c : a, !x, coef};
     }
-    // the interior difference times 1 plus 0, or times 0 plus the edge value
-    const double edge = interior ? 0.0
-                                 : (curl_y(g, W, lev, i, j) - curl_y(g, W, lev, i - 1, j)
-                                    + curl_x(g, W, lev, i, j - 1) - curl_x(g, W, lev, i, j)) * bydx2;
-    double lap = ((c - e) - (w - c) + (c - dn) - (up - c)) * bydx2 * (interior ? 1.0 : 0.0) + edge;
-    lap *= -1;
-    double a = lap * F.lap_coef;
-    a += F.an * n;
-    if (F.use_nprev) a += F.bn * (F.nprev_valid ? np : n);
-    a *= F.dt;
-    a += F.w_coef * c;
-    gout(F.a)[t] = a;
-    gout(F.nprev)[t] = n;
-    if (F.model == 4) {   // the filtered state's substep (IBSolver.cc:247-279), omega_hat = omega at the first
-        const double wh = F.sfd_valid ? sfd_w : c;
-        const double rs = (c - wh) * F.sfd_inv_delta;
-        double av = F.an * rs;
-        if (F.bn != 0) av += F.bn * (F.nprev_valid ? gin(F.sfd_prev)[tu] : rs);
-        av *= F.dt;
-        gout(F.what)[tu] = wh + av;
-        gout(F.sfd_prev)[tu] = rs;
+    return NodeTerm{lev, x ? i : i + t, x ? j + t : j, !x, t < 2 ? 0.5 * dx : 0.0};
+}
+
+// Term m (0..23) of fy(i, j) - fy(i - 1, j) + fx(i, j - 1) - fx(i, j); a flux of
+// the central region is the sum of two of the finer level, which lie at that
+// level's edge (region G).
+__device__ inline NodeTerm rim_term(const Lay& g, double dx0, int lev, int i, int j, int m) {
+    const int f = m / 6, t = m % 6;
+    const bool x = f >= 2;
+    const int ii = f == 1 ? i - 1 : i, jj = f == 2 ? j - 1 : j;
+    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
+    const bool fine = lev > 0 && (x ? ii > ex && ii < hx && jj >= ey && jj < hy : jj > ey && jj < hy && ii >= ex && ii < hx);
+    NodeTerm r{0, 1, 1, false, 0.0};
+    if (f > 3) return r;
+    if (fine) r = flux_term(g, dx0, x, lev - 1, 2 * (ii - ex) + (x ? 0 : t / 3), 2 * (jj - ey) + (x ? t / 3 : 0), t % 3);
+    else if (t < 3) r = flux_term(g, dx0, x, lev, ii, jj, t);
+    if (f & 1) r.coef = -r.coef;
+    return r;
+}
+
+// Offsets of the two values whose mean a level's field has at (i, j), 0 <= i <=
+// nx, 0 <= j <= ny, off its corners: its own value twice inside, getBC's of the
+// coarser level (Scalar.cc:91-127) on the boundary.  False (offsets of the
+// nearest node): 0 on the coarsest level's boundary.
+__device__ inline bool halo_at(const Lay& g, int lev, int i, int j, unsigned& a, unsigned& b) {
+    const unsigned ny1 = (unsigned)(g.ny - 1), base = (unsigned)(lev * g.ns());
+    const int ci = min(max(i, 1), g.nx - 1), cj = min(max(j, 1), g.ny - 1);
+    a = b = base + (unsigned)(ci - 1) * ny1 + (unsigned)(cj - 1);
+    if (ci == i && cj == j) return true;
+    if (lev == g.L - 1) return false;
+    const bool side = ci != i;   // on left or right, else on bottom or top
+    const int ii = nx_ext(g.nx) + i / 2, jj = nx_ext(g.ny) + j / 2;
+    a = base + (unsigned)g.ns() + (unsigned)(min(max(ii, 1), g.nx - 1) - 1) * ny1 + (unsigned)(min(max(jj, 1), g.ny - 1) - 1);
+    b = a + (side ? (unsigned)(j & 1) : (i & 1) * ny1);
+    return true;
+}
+
+// U (u) or V of the cross product at a node, from psi and the base flow of the
+// last refresh (FlowOps::bf[3..5]), as node_u and node_v give it from q, with
+// every load issued before any is used: the node velocity as a sum of at most
+// four fluxes (the rules of xvel and yvel), each a difference of two psi values.
+__device__ inline double node_value(const FlowOps& F, const Lay& g, const NodeTerm& t) {
+    const int lev = t.lev, na = t.u ? g.nx : g.ny, nc = t.u ? g.ny : g.nx;   // along and across the flux pair
+    const int al = t.u ? t.i : t.j, ac = t.u ? t.j : t.i;
+    const int alo = nx_ext(na), ahi = alo + na / 2, clo = nx_ext(nc), chi = clo + nc / 2;
+    const double bydx = 1. / (F.dx * (1 << lev));
+    const bool rim = lev >= 1 && (ac == clo || ac == chi) && al >= alo && al <= ahi;
+    const bool corner = rim && (al == alo || al == ahi), face = rim && !corner;
+    const int c0 = ac == clo ? ac - 1 : ac, c1 = ac == clo ? ac : ac - 1;   // outside the rim, inside it
+    const int cf = ac == clo ? 0 : nc - 1, af = face ? 2 * (al - alo) : al == alo ? 1 : na - 1;
+    // fluxes (level, along, across) and coefficients
+    const int fl[4] = {lev, (face ? lev - 1 : lev), rim ? lev - 1 : lev, rim ? lev - 1 : lev};
+    const int fa[4] = {al, face ? af : al, face ? af - 1 : corner ? af : al, face ? af + 1 : al};
+    const int fc[4] = {rim ? c0 : ac, face ? cf : corner ? c1 : ac - 1, rim ? cf : ac, rim ? cf : ac};
+    const double co[4] = {face ? 2. / 3 : corner ? 8. / 15 : 0.5, face ? 1. / 3 : corner ? 6. / 15 : 0.5,
+                          face ? 1. / 6 : corner ? 2. / 15 : 0.0, face ? 1. / 6 : 0.0};
+    double v = 0.0, v0 = 0.0;
+    const IBPM_GLOBAL double* P = gin(F.psi);
+    const bool base = has_base(F.model);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int l = max(fl[k], 0), i = t.u ? fa[k] : fc[k], j = t.u ? fc[k] : fa[k];
+        unsigned a0, a1, b0, b1;   // X flux (i, j): psi(i, j + 1) - psi(i, j); Y flux: psi(i, j) - psi(i + 1, j)
+        const bool p = halo_at(g, l, t.u ? i : i + 1, t.u ? j + 1 : j, a0, a1), m = halo_at(g, l, i, j, b0, b1);
+        const double x = (p ? 0.5 : 0.0) * (P[a0] + P[a1]), y = (m ? 0.5 : 0.0) * (P[b0] + P[b1]);
+        v += co[k] * ((t.u ? x - y : y - x) + (t.u ? base_x(F, F.bf + 3, l, j) : base_y(F, F.bf + 3, l, i)));
+        if (base) v0 += co[k] * gin(F.q0b)[t.u ? g.fx(l, i, j) : g.fy(l, i, j)];
+    }
+    const long at = g.s(lev, t.i, t.j);
+    const double w0 = base ? gin(F.w0b)[at] : 0.0;
+    return cross_node(F.model, t.u ? -1.0 : 1.0, v * bydx, gin(F.omega)[at], v0 * bydx, w0);
+}
+
+// Laplacian of a field at a node, the five values read together.
+__device__ inline double lap_at(const Lay& g, const double* f, int lev, int i, int j, double bydx2) {
+    const IBPM_GLOBAL double* P = gin(f);
+    double x[4];
+    const double c = P[g.s(lev, i, j)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        unsigned a, b;
+        const bool in = halo_at(g, lev, i + (k == 0) - (k == 1), j + (k == 2) - (k == 3), a, b);
+        x[k] = (in ? 0.5 : 0.0) * (P[a] + P[b]);
+    }
+    return -(((c - x[0]) - (x[1] - c) + (c - x[3]) - (x[2] - c)) * bydx2);
+}
+
+__global__ void __launch_bounds__(kThreads) k_advect_rim(const FlowOps* __restrict__ flows) {
+    const FlowOps& F = flows[blockIdx.y];
+    const Lay g{F.nx, F.ny, F.L};
+    const AdvShape S = adv_shape(g.nx, g.ny);
+    const int idx = blockIdx.x * kThreads + threadIdx.x, nrim = (g.L - 1) * S.rim * kRimLanes;
+    const bool rim = idx < nrim;
+    int lev = 0, i = 1, j = 1, at = 0;
+    bool node = false;
+    NodeTerm t{0, 1, 1, false, 0.0};
+    if (rim) {
+        const int k = idx / kRimLanes;
+        lev = k / S.rim + 1;
+        node = rim_node(g, k % S.rim, i, j);
+        if (node) t = rim_term(g, F.dx, lev, i, j, idx % kRimLanes);
+    } else {   // U at the coarser level's nodes along left and right, V along bottom and top
+        at = idx - nrim;
+        if (at >= (g.L - 1) * S.edge) return;   // (whole waves: 32 lanes a rim node)
+        const int l = at / S.edge, wide = g.ny / 2 + 1, tall = g.nx / 2 + 1;
+        const int ex = nx_ext(g.nx), ey = nx_ext(g.ny);
+        int m = at % S.edge;
+        const bool u = m < 2 * wide;
+        if (!u) m -= 2 * wide;
+        if (u) t = NodeTerm{l + 1, m < wide ? ex : ex + g.nx / 2, ey + m % wide, true, 1.0};
+        else t = NodeTerm{l + 1, ex + m % tall, m < tall ? ey : ey + g.ny / 2, false, 1.0};
+    }
+    const double d = F.dx * (1 << lev), bydx2 = 1. / (d * d);
+    const unsigned tu = (unsigned)g.s(lev, i, j);
+    const double c = gin(F.omega)[tu], np = gin(F.nprev)[tu];
+    const double lap = lap_at(g, F.omega, lev, i, j, bydx2);
+    const double ls = F.model == 2 ? lap_at(g, F.sff, lev, i, j, bydx2) : 0.0;
+    double v = t.coef != 0.0 ? t.coef * node_value(F, g, t) : 0.0;
+    if (!rim) {
+        gout(F.edge)[at] = v;
+        return;
+    }
+#pragma unroll
+    for (int off = kRimLanes / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (!node || idx % kRimLanes != 0) return;
+    rhs_node(F, F.model, tu, c, v * bydx2, ls, lap, np);
+    if (F.model == 4) sfd_node(F, tu, c);
+}
+
+// PLAIN: the nonlinear model's flows; the others' model terms, in the same
+// kernel, would cost it registers (105 against 80) and so a wave per SIMD.
+template <bool PLAIN>
+__global__ void __launch_bounds__(kThreads) k_advect(const FlowOps* __restrict__ flows) {
+    const FlowOps& F = flows[blockIdx.y];
+    const int model = PLAIN ? 0 : F.model;
+    if ((F.model == 0) != PLAIN) return;
+    const Lay g{F.nx, F.ny, F.L};
+    const AdvShape S = adv_shape(g.nx, g.ny);
+    // workgroups reach the 8 XCDs round-robin (the grid is a multiple of 8 wide):
+    // each takes a run of the flow's tiles, so that the rows and lines that
+    // neighbouring tiles share meet in one L2
+    const int run = (S.tiles * g.L + 7) / 8, bx = blockIdx.x % 8 * run + blockIdx.x / 8;
+    if ((int)blockIdx.x / 8 >= run) return;
+    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny);
+    if (bx >= S.tiles * g.L) return;
+    const int lev = bx / S.tiles, tile = bx % S.tiles;
+    const int i0 = 1 + tile / S.tj * kAdvI, j0 = 1 + tile % S.tj * kAdvJ;   // first node of the tile
+    const int hx = ex + g.nx / 2, hy = ey + g.ny / 2;
+    const bool all_central = lev >= 1 && i0 > ex && i0 + kAdvI - 1 < hx && j0 > ey && j0 + kAdvJ - 1 < hy;
+    if (all_central && model != 4) return;
+    constexpr int W = kAdvJ + 2, H = kAdvI + 2, kIn = (W * H + kThreads - 1) / kThreads;
+    constexpr int kRows = kThreads / kAdvJ, kOut = kAdvI / kRows;   // rows at a time
+    __shared__ double ps[H * W], om[H * W];
+    const unsigned ny1 = (unsigned)(g.ny - 1), base = (unsigned)(lev * g.ns());
+    const int col = threadIdx.x % kAdvJ, row = threadIdx.x / kAdvJ, j = j0 + col;
+    const IBPM_GLOBAL double *P = gin(F.psi), *Om = gin(F.omega);
+    double a[kIn], b[kIn], np[kOut];
+    const bool edge = i0 == 1 || j0 == 1 || i0 + kAdvI > g.nx - 1 || j0 + kAdvJ > g.ny - 1;
+    if (!edge) {
+#pragma unroll
+        for (int q = 0; q < kIn; ++q) {
+            const int idx = min((int)threadIdx.x + q * kThreads, W * H - 1);
+            const unsigned o = base + (unsigned)(i0 - 2 + idx / W) * ny1 + (unsigned)(j0 - 2 + idx % W);
+            a[q] = P[o];
+            b[q] = Om[o];
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < kIn; ++q) {
+            const int idx = min((int)threadIdx.x + q * kThreads, W * H - 1);
+            unsigned o1, o2;   // nodes more than one past the edge are not used
+            const bool in = halo_at(g, lev, min(i0 - 1 + idx / W, g.nx), min(j0 - 1 + idx % W, g.ny), o1, o2);
+            const double keep = in ? 0.5 : 0.0;
+            a[q] = keep * (P[o1] + P[o2]);
+            b[q] = keep * (Om[o1] + Om[o2]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kOut; ++q) {
+        const int i = min(i0 + row + q * kRows, g.nx - 1);
+        np[q] = gin(F.nprev)[base + (unsigned)(i - 1) * ny1 + (unsigned)(min(j, g.ny - 1) - 1)];
+    }
+#pragma unroll
+    for (int q = 0; q < kIn; ++q) {
+        const int idx = threadIdx.x + q * kThreads;
+        if (idx < W * H) {
+            ps[idx] = a[q];
+            om[idx] = b[q];
+        }
+    }
+    __syncthreads();
+    const double d = F.dx * (1 << lev), bydx2 = 1. / (d * d), c2 = 1. / (2 * d), hd = 0.5 * d;
+    const double* bf = F.bf + 3;
+    const double q0x = base_x(F, bf, lev, j), q0m = F.ubf ? base_x(F, bf, lev, j - 1) : q0x;   // X fluxes (., j), (., j - 1)
+    const IBPM_GLOBAL double* E = gin(F.edge) + (long)lev * S.edge;   // (not read on the coarsest level)
+    // U or V past the edge at position k along it, from line m of the edge values
+    auto past = [&](const IBPM_GLOBAL double* e, int k) {
+        return lev == g.L - 1 ? 0.0 : 0.5 * (e[k / 2] + e[k / 2 + (k & 1)]);
+    };
+#pragma unroll
+    for (int q = 0; q < kOut; ++q) {
+        const int r = row + q * kRows, i = i0 + r;
+        if (i > g.nx - 1 || j > g.ny - 1) continue;
+        const unsigned tu = base + (unsigned)(i - 1) * ny1 + (unsigned)(j - 1);
+        const int o = (r + 1) * W + col + 1;
+        const double c = om[o];
+        if (lev >= 1) {
+            if (i > ex && i < hx && j > ey && j < hy) {
+                if (model == 4) sfd_node(F, tu, c);
+                continue;
+            }
+            if (is_rim(g, i, j)) continue;
+        }
+        // node velocities from q = Curl(psi) + q0, U at (i - 1 .. i + 1, j), V at (i, j - 1 .. j + 1)
+        auto xv = [&](int k) { return ((ps[k + 1] - ps[k] + q0x) + (ps[k] - ps[k - 1] + q0m)) * c2; };
+        const double q0y = base_y(F, bf, lev, i), q0n = F.ubf ? base_y(F, bf, lev, i - 1) : q0y;
+        auto yv = [&](int k) { return ((ps[k - W] - ps[k] + q0n) + (ps[k] - ps[k + W] + q0y)) * c2; };
+        double u[3], v[3];
+        if (!has_base(model)) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                u[s] = cross_node(model, -1.0, xv(o + (s - 1) * W), om[o + (s - 1) * W], 0.0, 0.0);
+                v[s] = cross_node(model, 1.0, yv(o + s - 1), om[o + s - 1], 0.0, 0.0);
+            }
+        } else {
+            const IBPM_GLOBAL double *Q = gin(F.q0b), *W0 = gin(F.w0b);
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {   // (past the edge: any node's, replaced below)
+                const int iu = min(max(i + s - 1, 1), g.nx - 1), jv = min(max(j + s - 1, 1), g.ny - 1);
+                const double u0 = (Q[g.fx(lev, iu, j)] + Q[g.fx(lev, iu, j - 1)]) * c2;
+                const double v0 = (Q[g.fy(lev, i - 1, jv)] + Q[g.fy(lev, i, jv)]) * c2;
+                u[s] = cross_node(model, -1.0, xv(o + (s - 1) * W), om[o + (s - 1) * W], u0, W0[g.s(lev, iu, j)]);
+                v[s] = cross_node(model, 1.0, yv(o + s - 1), om[o + s - 1], v0, W0[g.s(lev, i, jv)]);
+            }
+        }
+        if (edge) {
+            const int wide = g.ny / 2 + 1, tall = g.nx / 2 + 1;
+            if (i == 1) u[0] = past(E, j);
+            if (i == g.nx - 1) u[2] = past(E + wide, j);
+            if (j == 1) v[0] = past(E + 2 * wide, i);
+            if (j == g.ny - 1) v[2] = past(E + 2 * wide + tall, i);
+        }
+        const double fy1 = (u[1] + u[2]) * hd, fy0 = (u[0] + u[1]) * hd;
+        const double fx0 = (v[0] + v[1]) * hd, fx1 = (v[1] + v[2]) * hd;
+        const double e = om[o + W], w = om[o - W], up = om[o + 1], dn = om[o - 1];
+        const double lap = -(((c - e) - (w - c) + (c - dn) - (up - c)) * bydx2);
+        double ls = 0.0;
+        if (model == 2) {
+            const IBPM_GLOBAL double* Sg = gin(F.sff);
+            if (i == 1 || i == g.nx - 1 || j == 1 || j == g.ny - 1) {
+                ls = lap_at(g, F.sff, lev, i, j, bydx2);
+            } else {
+                const double sc = Sg[tu];
+                ls = -(((sc - Sg[tu + ny1]) - (Sg[tu - ny1] - sc) + (sc - Sg[tu - 1]) - (Sg[tu + 1] - sc)) * bydx2);
+            }
+        }
+        rhs_node(F, model, tu, c, (fy1 - fy0 + fx0 - fx1) * bydx2, ls, lap, np[q]);
+        if (model == 4) sfd_node(F, tu, c);
     }
 }
 
-// q = Curl(psi) + q0 on every level (NavierStokesModel.cc:121-129): q0 is
-// the uniform base flow (Flux.cc:79-99) or the unsteady one, free stream plus
-// rotation about the body centre at the edge coordinates of each level
-// (Flux.cc:101-129, Grid.cc:104-139).  Thread (lev, i, j) of each level's
+// q = Curl(psi) + q0 on every level (NavierStokesModel.cc:121-129).  Thread (lev, i, j) of each level's
 // (nx + 1) x (ny + 1) cells writes X flux (i, j) (j < ny) and Y flux (i, j)
 // (i < nx), so each psi value is fetched once for both: a cell away from the
 // level's edge reads psi(i, j), psi(i, j + 1) and psi(i + 1, j) and takes
@@ -436,16 +812,7 @@ __global__ void __launch_bounds__(kThreads) k_curl_q(const FlowOps* __restrict__
         cx = j < g.ny ? curl_x(g, F.psi, lev, i, j) : 0.0;
         cy = i < g.nx ? curl_y(g, F.psi, lev, i, j) : 0.0;
     }
-    const double d = F.dx * (1 << lev);
-    // level offsets: offset + 0.5 (shift - 1) (2^lev - 1) n dx with shift 0
-    const double lofs = -0.5 * ((1 << lev) - 1);
-    double qx0 = F.ubase * d, qy0 = F.vbase * d;
-    if (F.ubf) {
-        const double y = (F.yoff + lofs * (F.ny * F.dx)) + (j + 0.5) * d;
-        qx0 = (F.bf[0] - F.bf[2] * (y - F.yc)) * d;
-        const double x = (F.xoff + lofs * (F.nx * F.dx)) + (i + 0.5) * d;
-        qy0 = (F.bf[1] + F.bf[2] * (x - F.xc)) * d;
-    }
+    const double qx0 = base_x(F, F.bf, lev, j), qy0 = base_y(F, F.bf, lev, i);
     IBPM_GLOBAL double* q = gout(F.q) + lev * (unsigned)g.nf();
     if (j < g.ny) q[(unsigned)i * (unsigned)g.ny + (unsigned)j] = cx + qx0;
     if (i < g.nx) q[(unsigned)g.nfx() + (unsigned)i * nyc + (unsigned)j] = cy + qy0;
@@ -940,6 +1307,19 @@ void launch_cross(const FlowOps* d, int nflows, long max_nf, int lev, hipStream_
 }
 void launch_cross_ff(const CrossFFOps* d, int nflows, long max_pts, hipStream_t s) {
     hipLaunchKernelGGL(k_cross_ff, dim3(blocks_for(max_pts), nflows), dim3(kThreads), 0, s, d);
+}
+size_t advect_edge(int nx, int ny, int L) { return (size_t)L * adv_shape(nx, ny).edge; }
+int advect_blocks(int nx, int ny, int L) { return (adv_shape(nx, ny).tiles * L + 7) / 8 * 8; }
+int advect_rim_blocks(int nx, int ny, int L) {
+    const AdvShape S = adv_shape(nx, ny);
+    return (int)(((long)(L - 1) * (S.rim * kRimLanes + S.edge) + kThreads - 1) / kThreads);
+}
+void launch_advect(const FlowOps* d, int nflows, int max_blocks, int max_rim_blocks, bool plain, bool other,
+                   hipStream_t s) {
+    if (max_rim_blocks > 0)   // (one level: no rims, no edge values)
+        hipLaunchKernelGGL(k_advect_rim, dim3(max_rim_blocks, nflows), dim3(kThreads), 0, s, d);
+    if (plain) hipLaunchKernelGGL(k_advect<true>, dim3(max_blocks, nflows), dim3(kThreads), 0, s, d);
+    if (other) hipLaunchKernelGGL(k_advect<false>, dim3(max_blocks, nflows), dim3(kThreads), 0, s, d);
 }
 void launch_rhs(const FlowOps* d, int nflows, long max_pts, hipStream_t s) {
     hipLaunchKernelGGL(k_rhs, dim3(blocks_for(max_pts), nflows), dim3(kThreads), 0, s, d);
