@@ -806,59 +806,81 @@ __global__ void __launch_bounds__(kThreads) k_fs_coarsify(const CoarsifyJob* __r
 // the tile.  Each point's update is the same arithmetic in the same order as
 // a sweep over global memory, so the result does not depend on the blocking.
 // Launches alternate between tmp and out so that the last writes out.
+//
+// Small boxes are bound by latency: a launch's descriptor, one round of loads,
+// a barrier per sweep.  So a thread's few points are loaded all at once and
+// their right-hand side stays in registers.  Plate at 128^2 x 3 (8 to 11
+// sweeps, a box of about 60 by 30 cells): two launches of 12.9 us with 256 threads walking eight
+// points each in turn; unrolled, six sweeps a launch, 8.2 us with 256 threads,
+// 5.9 with 512, 5.1 with 1024; twelve sweeps, 9.3 with 1024 (11.4 with 512),
+// one launch.  16 tandem flows, per step: 698 us before, 273 with six sweeps
+// and 512 threads, 306 as it is.
 #ifndef IBPM_HELM_DEPTH
-#define IBPM_HELM_DEPTH 6
+#define IBPM_HELM_DEPTH 12
 #endif
 constexpr int kHelmTile = 32, kHelmDepth = IBPM_HELM_DEPTH, kHelmReg = kHelmTile + 2 * kHelmDepth;
+constexpr int kHelmThreads = 1024, kHelmPer = (kHelmReg * kHelmReg + kHelmThreads - 1) / kHelmThreads;
 static_assert(kHelmDepth >= 1 && kHelmDepth <= 12, "sweeps per launch: 1..12 (LDS tiles with the halo)");
 
-__global__ void __launch_bounds__(kThreads) k_fs_helm(const HelmJob* __restrict__ jobs, int sweep0, int nsw,
-                                                     bool to_out) {
+__global__ void __launch_bounds__(kHelmThreads) k_fs_helm(const HelmJob* __restrict__ jobs, int sweep0, int nsw,
+                                                          bool to_out) {
     const HelmJob& J = jobs[blockIdx.y];
     if (skipped(J.skip)) return;
-    const int w = J.j1 - J.j0 + 1, h = J.i1 - J.i0 + 1;
+    const int i0 = J.i0, i1 = J.i1, j0 = J.j0, j1 = J.j1, ny = J.ny;
+    const int w = j1 - j0 + 1, h = i1 - i0 + 1;
     if (w <= 0 || h <= 0) return;
     const int tw = (w + kHelmTile - 1) / kHelmTile, th = (h + kHelmTile - 1) / kHelmTile;
     if ((int)blockIdx.x >= tw * th) return;
-    const int ti0 = J.i0 + (blockIdx.x / tw) * kHelmTile - kHelmDepth;   // region origin
-    const int tj0 = J.j0 + (blockIdx.x % tw) * kHelmTile - kHelmDepth;
-    __shared__ double rr[kHelmReg * kHelmReg], ua[kHelmReg * kHelmReg], ub[kHelmReg * kHelmReg];
-    const int ex = nx_ext(J.nx), ey = nx_ext(J.ny);
+    const int bi = (int)blockIdx.x / tw, bj = (int)blockIdx.x - bi * tw;
+    const int ti0 = i0 + bi * kHelmTile - kHelmDepth;   // region origin
+    const int tj0 = j0 + bj * kHelmTile - kHelmDepth;
+    __shared__ double ua[kHelmReg * kHelmReg], ub[kHelmReg * kHelmReg];
+    const int ex = nx_ext(J.nx), ey = nx_ext(ny);
+    const int ci1 = J.lev >= 1 ? J.nx / 2 + ex : 0, cj1 = ny / 2 + ey;   // central region's ends
     const IBPM_GLOBAL double* src = gin(to_out ? J.tmp : J.out);
-    for (int q = threadIdx.x; q < kHelmReg * kHelmReg; q += kThreads) {
+    const IBPM_GLOBAL double* f = gin(J.f);
+    const IBPM_GLOBAL double* Rc = J.lev >= 1 ? gin(J.R) : f;
+    const double in_scale = J.in_scale, inv_diag = J.inv_diag, c = J.c;
+    // a thread's points: all loads issued together, from the box's nearest
+    // point where the point is off the box and the value is not used
+    double r[kHelmPer], u[kHelmPer];
+    bool inbox[kHelmPer];
+#pragma unroll
+    for (int p = 0; p < kHelmPer; ++p) {
+        const int q = threadIdx.x + p * kHelmThreads;
         const int i = ti0 + q / kHelmReg, j = tj0 + q % kHelmReg;
-        const bool inbox = i >= J.i0 && i <= J.i1 && j >= J.j0 && j <= J.j1;
-        double r = 0.0, u = 0.0;
-        if (inbox) {
-            const long k = sidx(J.nx, J.ny, i, j);
-            const bool central = J.lev >= 1 && i > ex && i < J.nx / 2 + ex && j > ey && j < J.ny / 2 + ey;
-            const bool support = i >= J.s0 && i <= J.s1 && j >= J.t0 && j <= J.t1;
-            r = support ? (central ? gin(J.R)[k] : gin(J.f)[k]) * J.in_scale : 0.0;
-            if (sweep0 > 0) u = src[k];
-        }
-        rr[q] = r;
-        ua[q] = u;
+        inbox[p] = i >= i0 && i <= i1 && j >= j0 && j <= j1;
+        const int k = (int)sidx(J.nx, ny, min(max(i, i0), i1), min(max(j, j0), j1));
+        const bool central = i > ex && i < ci1 && j > ey && j < cj1;
+        r[p] = (central ? Rc : f)[k];
+        u[p] = sweep0 > 0 ? src[k] : 0.0;
+    }
+#pragma unroll
+    for (int p = 0; p < kHelmPer; ++p) {
+        const int q = threadIdx.x + p * kHelmThreads;
+        const int i = ti0 + q / kHelmReg, j = tj0 + q % kHelmReg;
+        const bool support = i >= J.s0 && i <= J.s1 && j >= J.t0 && j <= J.t1;
+        r[p] = inbox[p] && support ? r[p] * in_scale : 0.0;
+        if (q < kHelmReg * kHelmReg) ua[q] = inbox[p] ? u[p] : 0.0;
     }
     __syncthreads();
     double* cur = ua;
     double* nxt = ub;
     for (int d = 0; d < nsw; ++d) {
         const int m = d + 1;   // points within m of the region's edge are no longer valid
-        for (int q = threadIdx.x; q < kHelmReg * kHelmReg; q += kThreads) {
+#pragma unroll
+        for (int p = 0; p < kHelmPer; ++p) {
+            const int q = threadIdx.x + p * kHelmThreads;
             const int a = q / kHelmReg, b = q % kHelmReg;
             if (a < m || b < m || a >= kHelmReg - m || b >= kHelmReg - m) continue;
-            const int i = ti0 + a, j = tj0 + b;
-            const bool inbox = i >= J.i0 && i <= J.i1 && j >= J.j0 && j <= J.j1;
             double v = 0.0;
-            if (inbox) {
-                if (sweep0 + d == 0) {
-                    v = rr[q] * J.inv_diag;
-                } else {
-                    const double s4 = (cur[q - kHelmReg] + cur[q + kHelmReg]) + (cur[q - 1] + cur[q + 1]);
-                    v = (rr[q] - J.c * s4) * J.inv_diag;
-                }
+            if (sweep0 + d == 0) {
+                v = r[p] * inv_diag;
+            } else {
+                const double s4 = (cur[q - kHelmReg] + cur[q + kHelmReg]) + (cur[q - 1] + cur[q + 1]);
+                v = (r[p] - c * s4) * inv_diag;
             }
-            nxt[q] = v;
+            nxt[q] = inbox[p] ? v : 0.0;
         }
         __syncthreads();
         double* t = cur;
@@ -866,11 +888,11 @@ __global__ void __launch_bounds__(kThreads) k_fs_helm(const HelmJob* __restrict_
         nxt = t;
     }
     IBPM_GLOBAL double* dst = gout(to_out ? J.out : J.tmp);
-    for (int q = threadIdx.x; q < kHelmTile * kHelmTile; q += kThreads) {
+    for (int q = threadIdx.x; q < kHelmTile * kHelmTile; q += kHelmThreads) {
         const int a = kHelmDepth + q / kHelmTile, b = kHelmDepth + q % kHelmTile;
         const int i = ti0 + a, j = tj0 + b;
-        if (i > J.i1 || j > J.j1) continue;
-        dst[sidx(J.nx, J.ny, i, j)] = cur[a * kHelmReg + b];
+        if (i > i1 || j > j1) continue;
+        dst[sidx(J.nx, ny, i, j)] = cur[a * kHelmReg + b];
     }
 }
 
@@ -1190,7 +1212,7 @@ void launch_helm_sweeps(const HelmJob* d_jobs, int njobs, int max_tiles, int nsw
         const int s0 = n * kHelmDepth, nsw = std::min(kHelmDepth, nsweeps - s0);
         const bool to_out = ((nl - 1 - n) & 1) == 0;
         timed_launch([&] {
-            hipLaunchKernelGGL(k_fs_helm, dim3(max_tiles, njobs), dim3(kThreads), 0, s, d_jobs, s0, nsw, to_out);
+            hipLaunchKernelGGL(k_fs_helm, dim3(max_tiles, njobs), dim3(kHelmThreads), 0, s, d_jobs, s0, nsw, to_out);
         });
     }
 }
