@@ -200,6 +200,12 @@ constexpr long kRegMinPairs = 1024;
 #endif
 __host__ __device__ constexpr int r16_group(int pass) { return pass == 2 ? IBPM_R16_GROUP2 : 1; }
 
+// Waves per SIMD asked of the compiler.  Pass 2 at M = 2048 took 130 registers,
+// which leaves three waves where its LDS has room for four; held to 128, 16
+// tandem flows' levels of 1023 x 1023 take 110 us instead of 116.  The same
+// bound made the compiler take 96 for pass 1, 57 us instead of 52.
+__host__ __device__ constexpr int r16_waves(int pass) { return pass == 2 ? 4 : 1; }
+
 // LDS slot of element e: one pad slot after every 16, so the first stage's
 // writes (16 consecutive elements per lane) spread over the banks, and every
 // access of a stage is a per-lane base plus a compile-time offset.  The
@@ -692,7 +698,7 @@ __device__ __forceinline__ void pass3_r16(const EllJob& J, double2* smem, int bx
 // its force solve does nothing (skipped()).
 #define IBPM_REG_KERNEL(NAME, BODY, PASS)                                        \
     template <int M>                                                             \
-    __global__ void __launch_bounds__(r16_group(PASS) * (M / 16)) NAME(const EllJob* __restrict__ jobs) { \
+    __global__ void __launch_bounds__(r16_group(PASS) * (M / 16), r16_waves(PASS)) NAME(const EllJob* __restrict__ jobs) { \
         extern __shared__ double2 smem[];                                        \
         const int2 blk = xcd_block();                                            \
         const EllJob& J = jobs[blk.y];                                           \
