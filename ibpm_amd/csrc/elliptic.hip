@@ -828,6 +828,67 @@ constexpr int kHelmTile = 32, kHelmDepth = IBPM_HELM_DEPTH, kHelmReg = kHelmTile
 constexpr int kHelmThreads = 1024, kHelmPer = (kHelmReg * kHelmReg + kHelmThreads - 1) / kHelmThreads;
 static_assert(kHelmDepth >= 1 && kHelmDepth <= 12, "sweeps per launch: 1..12 (LDS tiles with the halo)");
 
+constexpr int kHelmChainPts = kHelmReg * kHelmReg;   // the sweeps' LDS tiles hold it
+int helm_chain_points() { return kHelmChainPts; }
+
+// The coarsify chain of the local solves' right-hand side over each job's
+// support: Scalar::coarsify's weights and order (as coarsify_body) with the
+// finer level's value taken as 0 in its central region off its support (R
+// holds other solves' values there) and from f outside the central region.
+// Point p of the support; fineR(fi, fj) is R on the finer level's support.
+template <class FineR>
+__device__ inline double helm_coarse_value(const HelmJob& J, int i, int j, const FineR& fineR) {
+    const int ex = nx_ext(J.nx), ey = nx_ext(J.ny);
+    const int ii = (i - ex) * 2, jj = (j - ey) * 2;   // Grid::c2f
+    const int lf = J.lev - 1;
+    auto fine = [&](int fi, int fj) {
+        const bool central = lf >= 1 && fi > ex && fi < J.nx / 2 + ex && fj > ey && fj < J.ny / 2 + ey;
+        if (!central) return gin(J.f_fine)[sidx(J.nx, J.ny, fi, fj)];
+        const bool sup = fi >= J.fs0 && fi <= J.fs1 && fj >= J.ft0 && fj <= J.ft1;
+        return sup ? fineR(fi, fj) : 0.0;
+    };
+    double x[3][3];   // fine (ii - 1 + d, jj - 1 + c)
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x[d][c] = fine(ii - 1 + d, jj - 1 + c);
+    return 0.25 * x[1][1] + 0.125 * (x[2][1] + x[1][2] + x[0][1] + x[1][0])
+        + 0.0625 * (x[2][2] + x[2][0] + x[0][2] + x[0][0]);
+}
+
+// One level of it in a launch over the whole support.
+__global__ void __launch_bounds__(kThreads) k_fs_helm_coarsify(const HelmJob* __restrict__ jobs, int lev) {
+    const HelmJob& J = jobs[blockIdx.y];
+    if (J.lev != lev || skipped(J.skip)) return;
+    const int w = J.t1 - J.t0 + 1, h = J.s1 - J.s0 + 1;
+    const int p = blockIdx.x * kThreads + threadIdx.x;
+    if (w <= 0 || h <= 0 || p >= w * h) return;
+    const int i = J.s0 + p / w, j = J.t0 + p % w;
+    const double v = helm_coarse_value(J, i, j, [&](int fi, int fj) {
+        return gin(J.R_fine)[sidx(J.nx, J.ny, fi, fj)];
+    });
+    gout(J.R)[sidx(J.nx, J.ny, i, j)] = v;
+}
+
+// Where every level's support fits a workgroup's LDS (kHelmChainPts), one
+// workgroup runs the chain itself, a level's R going to the next through LDS:
+// inside k_fs_helm for its own right-hand side, and in one launch
+// (k_fs_chain) for the L^-1 solve's.  A launch per level costs 3.9 us however
+// small its support is; the whole second chain takes 3.9 us at 128^2 x 3, and
+// 9.9 at 512^2 x 5 where four launches took 4.9 each.  Level J's R into cur, row by row of its support.
+__device__ inline void helm_chain_level(const HelmJob& J, const double* prev, double* cur) {
+    const int w = J.t1 - J.t0 + 1, h = J.s1 - J.s0 + 1, fw = J.ft1 - J.ft0 + 1;
+    if (w > 0 && h > 0)
+        for (int p = threadIdx.x; p < w * h; p += blockDim.x)
+            cur[p] = helm_coarse_value(J, J.s0 + p / w, J.t0 + p % w, [&](int fi, int fj) {
+                return prev[(fi - J.fs0) * fw + (fj - J.ft0)];
+            });
+    __syncthreads();
+}
+
+// CHAIN: the coarse levels' right-hand sides come from the chain run here
+// (jobs hold a flow's levels one after another, level 0 first).
+template <bool CHAIN>
 __global__ void __launch_bounds__(kHelmThreads) k_fs_helm(const HelmJob* __restrict__ jobs, int sweep0, int nsw,
                                                           bool to_out) {
     const HelmJob& J = jobs[blockIdx.y];
@@ -845,7 +906,7 @@ __global__ void __launch_bounds__(kHelmThreads) k_fs_helm(const HelmJob* __restr
     const int ci1 = J.lev >= 1 ? J.nx / 2 + ex : 0, cj1 = ny / 2 + ey;   // central region's ends
     const IBPM_GLOBAL double* src = gin(to_out ? J.tmp : J.out);
     const IBPM_GLOBAL double* f = gin(J.f);
-    const IBPM_GLOBAL double* Rc = J.lev >= 1 ? gin(J.R) : f;
+    const IBPM_GLOBAL double* Rc = !CHAIN && J.lev >= 1 ? gin(J.R) : f;
     const double in_scale = J.in_scale, inv_diag = J.inv_diag, c = J.c;
     // a thread's points: all loads issued together, from the box's nearest
     // point where the point is off the box and the value is not used
@@ -861,12 +922,29 @@ __global__ void __launch_bounds__(kHelmThreads) k_fs_helm(const HelmJob* __restr
         r[p] = (central ? Rc : f)[k];
         u[p] = sweep0 > 0 ? src[k] : 0.0;
     }
+    const double* chain = ua;
+    if (CHAIN) {
+        double *prev = ub, *cur = ua;
+        for (int lev = 1; lev <= J.lev; ++lev) {
+            helm_chain_level(jobs[(int)blockIdx.y - J.lev + lev], prev, cur);
+            chain = cur;
+            cur = prev;
+            prev = (double*)chain;
+        }
+    }
 #pragma unroll
     for (int p = 0; p < kHelmPer; ++p) {
         const int q = threadIdx.x + p * kHelmThreads;
         const int i = ti0 + q / kHelmReg, j = tj0 + q % kHelmReg;
         const bool support = i >= J.s0 && i <= J.s1 && j >= J.t0 && j <= J.t1;
+        const bool central = i > ex && i < ci1 && j > ey && j < cj1;
+        if (CHAIN && support && central) r[p] = chain[(i - J.s0) * (J.t1 - J.t0 + 1) + (j - J.t0)];
         r[p] = inbox[p] && support ? r[p] * in_scale : 0.0;
+    }
+    if (CHAIN) __syncthreads();   // chain is one of the tiles
+#pragma unroll
+    for (int p = 0; p < kHelmPer; ++p) {
+        const int q = threadIdx.x + p * kHelmThreads;
         if (q < kHelmReg * kHelmReg) ua[q] = inbox[p] ? u[p] : 0.0;
     }
     __syncthreads();
@@ -902,6 +980,23 @@ __global__ void __launch_bounds__(kHelmThreads) k_fs_helm(const HelmJob* __restr
     }
 }
 
+// The chain of each flow's jobs, levels 1, 2, ... one after another, in the
+// workgroup of its level-1 job.
+__global__ void __launch_bounds__(kHelmThreads) k_fs_chain(const HelmJob* __restrict__ jobs, int njobs) {
+    __shared__ double buf[2][kHelmChainPts];
+    const int first = blockIdx.x;
+    if (jobs[first].lev != 1 || skipped(jobs[first].skip)) return;
+    for (int q = first; q < njobs && jobs[q].lev == 1 + q - first; ++q) {
+        const HelmJob& J = jobs[q];
+        double* cur = buf[(q - first) & 1];
+        helm_chain_level(J, buf[(q - first + 1) & 1], cur);
+        const int w = J.t1 - J.t0 + 1, h = J.s1 - J.s0 + 1;
+        if (w <= 0 || h <= 0) continue;
+        for (int p = threadIdx.x; p < w * h; p += kHelmThreads)
+            gout(J.R)[sidx(J.nx, J.ny, J.s0 + p / w, J.t0 + p % w)] = cur[p];
+    }
+}
+
 // u = W - v over each job's box, v the local result (J.out): the epilogue of
 // the step's omega = omega* - A^-1 c, whose omega already holds omega* off the
 // boxes (the omega* solve writes both).
@@ -912,38 +1007,6 @@ __global__ void __launch_bounds__(kThreads) k_helm_epilogue(const HelmJob* __res
     if (w <= 0 || h <= 0 || p >= w * h) return;
     const long k = sidx(J.nx, J.ny, J.i0 + p / w, J.j0 + p % w);
     gout(J.eo)[k] = gin(J.ei)[k] - gin(J.out)[k];
-}
-
-// The coarsify chain of the local solves' right-hand side, level lev of every
-// job, over the job's support only: Scalar::coarsify's weights and order (as
-// coarsify_body) with the finer level's value taken as 0 in its central
-// region off its support (R holds other solves' values there) and from f
-// outside the central region.
-__global__ void __launch_bounds__(kThreads) k_fs_helm_coarsify(const HelmJob* __restrict__ jobs, int lev) {
-    const HelmJob& J = jobs[blockIdx.y];
-    if (J.lev != lev || skipped(J.skip)) return;
-    const int w = J.t1 - J.t0 + 1, h = J.s1 - J.s0 + 1;
-    const int p = blockIdx.x * kThreads + threadIdx.x;
-    if (w <= 0 || h <= 0 || p >= w * h) return;
-    const int i = J.s0 + p / w, j = J.t0 + p % w;
-    const int ex = nx_ext(J.nx), ey = nx_ext(J.ny);
-    const int ii = (i - ex) * 2, jj = (j - ey) * 2;   // Grid::c2f
-    const int lf = lev - 1;
-    auto fine = [&](int fi, int fj) {
-        const long k = sidx(J.nx, J.ny, fi, fj);
-        const bool central = lf >= 1 && fi > ex && fi < J.nx / 2 + ex && fj > ey && fj < J.ny / 2 + ey;
-        if (!central) return gin(J.f_fine)[k];
-        const bool sup = fi >= J.fs0 && fi <= J.fs1 && fj >= J.ft0 && fj <= J.ft1;
-        return sup ? gin(J.R_fine)[k] : 0.0;
-    };
-    double x[3][3];   // fine (ii - 1 + d, jj - 1 + c)
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) x[d][c] = fine(ii - 1 + d, jj - 1 + c);
-    const double v = 0.25 * x[1][1] + 0.125 * (x[2][1] + x[1][2] + x[0][1] + x[1][0])
-        + 0.0625 * (x[2][2] + x[2][0] + x[0][2] + x[0][0]);
-    gout(J.R)[sidx(J.nx, J.ny, i, j)] = v;
 }
 
 // ------------------------------------------------ dense sine-matrix GEMM on MFMA
@@ -1211,14 +1274,18 @@ int helm_launches(int nsweeps) { return (nsweeps + kHelmDepth - 1) / kHelmDepth;
 
 int helm_tiles(int h, int w) { return ((h + kHelmTile - 1) / kHelmTile) * ((w + kHelmTile - 1) / kHelmTile); }
 
-void launch_helm_sweeps(const HelmJob* d_jobs, int njobs, int max_tiles, int nsweeps, hipStream_t s,
+void launch_helm_chain(const HelmJob* d_jobs, int njobs, hipStream_t s) {
+    hipLaunchKernelGGL(k_fs_chain, dim3(njobs), dim3(kHelmThreads), 0, s, d_jobs, njobs);
+}
+void launch_helm_sweeps(const HelmJob* d_jobs, int njobs, int max_tiles, int nsweeps, bool chain, hipStream_t s,
                         const std::function<void(const std::function<void()>&)>& timed_launch) {
     const int nl = (nsweeps + kHelmDepth - 1) / kHelmDepth;
     for (int n = 0; n < nl; ++n) {
         const int s0 = n * kHelmDepth, nsw = std::min(kHelmDepth, nsweeps - s0);
         const bool to_out = ((nl - 1 - n) & 1) == 0;
         timed_launch([&] {
-            hipLaunchKernelGGL(k_fs_helm, dim3(max_tiles, njobs), dim3(kHelmThreads), 0, s, d_jobs, s0, nsw, to_out);
+            hipLaunchKernelGGL(chain ? k_fs_helm<true> : k_fs_helm<false>, dim3(max_tiles, njobs), dim3(kHelmThreads), 0, s,
+                               d_jobs, s0, nsw, to_out);
         });
     }
 }

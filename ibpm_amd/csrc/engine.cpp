@@ -876,6 +876,8 @@ struct ibpm_batch {
     bool fs32 = false;             // the force solve's solves in FP32
     ibpmg::HelmJob* d_m2lc = nullptr;
     int m2lc_cap = 0, m2lc_n = 0, m2lc_blocks = 0;
+    // the chains' supports fit a workgroup (helm_chain_points)
+    bool helm_chain = false, m2lc_chain = false;
     std::vector<int> m2lc_flow;
     std::vector<double> m2lc_bytes;
     long st_local_mapps = 0;
@@ -1706,6 +1708,7 @@ static int restrict_m2l_pass3(ibpm_batch* B, const std::vector<std::vector<std::
     CKR(up(B, B->d_m2lc, cj.data(), sizeof(HelmJob) * cj.size()));
     B->m2lc_n = (int)cj.size();
     B->m2lc_blocks = (int)((maxa + kThreads - 1) / kThreads);
+    B->m2lc_chain = B->m2lc_n > 0 && maxa <= helm_chain_points();
     return 0;
 }
 
@@ -1860,6 +1863,12 @@ static int plan_local_helm(ibpm_batch* B, int i) {
     B->helm_n = (int)jobs.size();
     B->helm_blocks = (int)maxarea;   // tiles of the largest box
     B->helm_cblocks = (int)((maxsup + kThreads - 1) / kThreads);
+    // Every tile of the sweeps repeats the chain, so they run it while their
+    // grid is one round of workgroups (two on each of 256 CUs), where it costs
+    // latency only.  Plate 128^2 x 3: sweeps 9.3 -> 10.9 us, two launches of 3.9
+    // saved.  16 tandem flows of 6 levels, per step: 790 us with a launch per level,
+    // 850 with the chain in every tile.
+    B->helm_chain = maxsup <= helm_chain_points() && (long)jobs.size() * maxarea <= 512;
     B->helm_sweeps = sweeps;
     B->helm_flow = jflow;
     B->helm_bytes = jbytes;
@@ -1899,16 +1908,18 @@ static void enqueue_M(ibpm_batch* B, int i, RegOps* smear, hipStream_t s,
                     by += B->helm_bytes[j];
                     cby += B->helm_cbytes[j];
                 }
-        for (int lev = 1; lev < (single_level ? 1 : B->M1[i].nlev); ++lev)
+        for (int lev = 1; lev < (single_level || B->helm_chain ? 1 : B->M1[i].nlev); ++lev)
             timed(pr, K_FSCOARSIFY, cby / std::max(1, B->M1[i].nlev - 1), s,
                   [&] { launch_helm_coarsify(B->d_helm, B->helm_n, B->helm_cblocks, lev, s); });
         const int nl = helm_launches(B->helm_sweeps);
         if (single_level)   // level 0's sweeps alone: the coarser levels' results are not read
-            launch_helm_sweeps(B->d_helm0, B->helm0_n, B->helm0_blocks, B->helm_sweeps, s,
+            launch_helm_sweeps(B->d_helm0, B->helm0_n, B->helm0_blocks, B->helm_sweeps, false, s,
                                [&](const std::function<void()>& fn) { timed(pr, K_FSHELM, B->helm0_bytes / nl, s, fn); });
         else
-            launch_helm_sweeps(B->d_helm, B->helm_n, B->helm_blocks, B->helm_sweeps, s,
-                               [&](const std::function<void()>& fn) { timed(pr, K_FSHELM, by / nl, s, fn); });
+            launch_helm_sweeps(B->d_helm, B->helm_n, B->helm_blocks, B->helm_sweeps, B->helm_chain, s,
+                               [&](const std::function<void()>& fn) {
+                                   timed(pr, K_FSHELM, (by + (B->helm_chain ? cby : 0)) / nl, s, fn);
+                               });
         const bool boxed = !B->M2L.fp32;   // the FP32 passes read the whole coarse right-hand side
         if (single_level) {
             run_solve(B->M1L, s, pr, active, false);
@@ -1917,7 +1928,9 @@ static void enqueue_M(ibpm_batch* B, int i, RegOps* smear, hipStream_t s,
             if (pr)
                 for (size_t j = 0; j < B->m2lc_flow.size(); ++j)
                     if (!active || (*active)[B->m2lc_flow[j]]) cb += B->m2lc_bytes[j];
-            for (int lev = 1; lev < B->M2L.nlev; ++lev)
+            if (B->m2lc_chain)
+                timed(pr, K_FSCOARSIFY, cb, s, [&] { launch_helm_chain(B->d_m2lc, B->m2lc_n, s); });
+            for (int lev = 1; lev < (B->m2lc_chain ? 1 : B->M2L.nlev); ++lev)
                 timed(pr, K_FSCOARSIFY, cb / std::max(1, B->M2L.nlev - 1), s,
                       [&] { launch_helm_coarsify(B->d_m2lc, B->m2lc_n, B->m2lc_blocks, lev, s); });
         }
@@ -2368,12 +2381,12 @@ static int substep_cg(ibpm_batch* B, int i) {
         // omega = omega* - A^-1 c with c = beta B f local like M's right-hand
         // side: the same sweeps (plan_local_helm), then the subtraction over
         // the boxes; off them omega already holds omega* (the S1 solve wrote it)
-        for (int lev = 1; lev < B->S3[i].nlev; ++lev)
+        for (int lev = 1; lev < (B->helm_chain ? 1 : B->S3[i].nlev); ++lev)
             timed(pr, K_HELM, 0, s, [&] { launch_helm_coarsify(B->d_helm3, B->helm_n, B->helm_cblocks, lev, s); });
         const int nl = helm_launches(B->helm_sweeps);
         double by = 0;
         for (double b : B->helm_bytes) by += b;
-        launch_helm_sweeps(B->d_helm3, B->helm_n, B->helm_blocks, B->helm_sweeps, s,
+        launch_helm_sweeps(B->d_helm3, B->helm_n, B->helm_blocks, B->helm_sweeps, B->helm_chain, s,
                            [&](const std::function<void()>& fn) { timed(pr, K_HELM, by / nl, s, fn); });
         timed(pr, K_HELM, 0, s, [&] { launch_helm_epilogue(B->d_helm3, B->helm_n, B->helm_ablocks, s); });
     } else {

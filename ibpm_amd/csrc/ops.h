@@ -196,10 +196,16 @@ int helm_launches(int nsweeps);   // launches of launch_helm_sweeps for nsweeps 
 void launch_helm_epilogue(const HelmJob* d_jobs, int njobs, int max_blocks, hipStream_t s);
 // out = tmp = 0 over each job's box.
 void launch_helm_clear(const HelmJob* d_jobs, int njobs, int max_blocks, hipStream_t s);
-void launch_helm_sweeps(const HelmJob* d_jobs, int njobs, int max_tiles, int nsweeps, hipStream_t s,
+// chain: the sweeps make the coarse levels' right-hand sides themselves (every
+// support of at most helm_chain_points, jobs grouped by flow, level 0 first).
+void launch_helm_sweeps(const HelmJob* d_jobs, int njobs, int max_tiles, int nsweeps, bool chain, hipStream_t s,
                         const std::function<void(const std::function<void()>&)>& timed_launch);
 // The right-hand side's coarsify chain at level lev (>= 1) over each job's
 // support (HelmJob); max_blocks: kThreads-point blocks of the largest support.
+int helm_chain_points();
+// The whole chain, levels 1, 2, ... of each flow (adjacent jobs, level 1
+// first), in one launch where every support has at most helm_chain_points.
+void launch_helm_chain(const HelmJob* d_jobs, int njobs, hipStream_t s);
 void launch_helm_coarsify(const HelmJob* d_jobs, int njobs, int max_blocks, int lev, hipStream_t s);
 void launch_vel(const FlowOps* d, int nflows, long max_pts, hipStream_t s);
 void launch_cross(const FlowOps* d, int nflows, long max_nf, int lev, hipStream_t s);

@@ -42,3 +42,30 @@ def test_sweeps_equal_the_dst_solve(gpu, count, points):
     hl, hd = loc.force_history(), dst.force_history()
     assert np.abs(hl - hd).max() <= 1e-8 * np.abs(hd).max()
     assert np.linalg.norm(loc.omega() - dst.omega()) <= 1e-8 * np.linalg.norm(dst.omega())
+
+
+@pytest.mark.parametrize("levels", [2, 4])
+@pytest.mark.parametrize("reach", [20, 45, 58])
+def test_coarse_right_hand_sides(gpu, reach, levels):
+    """A diagonal plate of 2 reach cells: both coarsify chains within one
+    workgroup's 3136 points on level 1 (reach 20), only the sweeps' own (45),
+    neither (58); two flows, so that the second one's jobs do not start at 0."""
+    n, dx, Re = 256, 8.0 / 256, 196.0
+    print("coarse right-hand sides", reach, levels, flush=True)
+    a, pts = reach * dx, reach + 1
+    geom = ("body Plate\n  line_n %.17g %.17g %.17g %.17g %d\n  center 0 0\n"
+            "  motion pitchplunge 0.1 0.4 0 0.1 0.4 0\nend\n" % (-a, -a + 0.01, a, a + 0.01, pts))
+    small = ("body Plate\n  line_n -0.3 0.01 0.3 0.01 11\n  center 0 0\n"
+             "  motion pitchplunge 0.1 0.4 0 0.1 0.4 0\nend\n")
+    ctx = gpu.Context(0)
+    fl = [gpu.Flow(n, n, levels, 8.0, -4.0, -4.0, Re, DT, g, tol=1e-10) for g in (small, geom)]
+    loc = gpu.Batch(ctx, fl).init()
+    dst = gpu.Batch(ctx, fl).init().set_local_helmholtz(False)
+    loc.advance(2)
+    dst.advance(2)
+    sl = loc.solver_stats()
+    assert sl["local_helmholtz_m_applications"] == sl["m_applications"] > 0
+    for k in range(2):
+        hl, hd = loc.force_history(k), dst.force_history(k)
+        assert np.abs(hl - hd).max() <= 1e-8 * np.abs(hd).max()
+        assert np.linalg.norm(loc.omega(k) - dst.omega(k)) <= 1e-8 * np.linalg.norm(dst.omega(k))
