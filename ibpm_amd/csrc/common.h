@@ -62,6 +62,8 @@ struct EllJob {
     double* T1;              // scratch T: (nx-1) rows of ny-1 values, row stride ld1 = t1_ld(ny-1)
     double* T2;              // the GEMM-DST's second pair of planes (null where it does not run)
     int ld1;
+    double* T1b;             // pass 2 of two solves: the second one's scratch, laid out as T1
+    double scale_b;          // and its right-hand side, this times the first one's solution
     double* u;               // level slice of the solution
     double* u2;              // null, or a second output of the same values (pass 3)
     const double* W;         // epilogue 1 operand (level slice)

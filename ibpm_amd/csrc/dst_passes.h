@@ -298,14 +298,14 @@ IBPM_DST_KERNEL(k_dst_pass1, dst_threads(M)) {
 // One column pair per workgroup, in place.  (Two pairs, 32-byte pieces, measured
 // the same on batches of 400^2 to 1000^2 levels and slower on one flow: 8.2
 // against 7.7 us at 400^2.)
-IBPM_DST_KERNEL(k_dst_pass2, dst_threads(M)) {
+// BOTH: of a Helmholtz solve u = A^-1 f and the Poisson solve L^-1(s u) of its
+// result on the same level, from the one forward transform: u's rows to T1,
+// the other's to T1b (EllJob::T1b).
+template <int M, bool BOTH>
+__device__ __forceinline__ void dst_pass2(const EllJob& J, int bx, double2* lds, double2* y) {
     constexpr int BT = dst_threads(M), N1 = M / 2 - 1;
     typedef LdsFft<M, BT> F;
-    __shared__ double2 lds[F::kSlots], y[M / 2];
-    const int2 blk = xcd_block();
-    const EllJob& J = jobs[blk.y];
-    if (skipped(J.skip)) return;
-    const int N2 = J.ny - 1, la = 2 * blk.x;
+    const int N2 = J.ny - 1, la = 2 * bx;
     if (la >= N2) return;
     typedef double Pair __attribute__((ext_vector_type(2)));
     const long ld = J.ld1;
@@ -347,10 +347,12 @@ IBPM_DST_KERNEL(k_dst_pass2, dst_threads(M)) {
         y[idx + 1] = v;
     }
     __syncthreads();
-    // both transforms by one copy of the code: what bounds a small launch is
+    IBPM_GLOBAL double* Tb = BOTH ? gout(J.T1b) : T;
+    const double sb = BOTH ? J.scale_b : 0.0;
+    // all transforms by one copy of the code: what bounds a small launch is
     // the time a workgroup takes, its instruction fetch among it
 #pragma unroll 1
-    for (int it = 0; it < 2; ++it) {
+    for (int it = 0; it < (BOTH ? 3 : 2); ++it) {
         f.template run<F::Q.n == 1>(lds, [&](int e) {
             const Ext x = ext_at<M>(e);
             const double2 v = y[x.idx + 1];
@@ -365,13 +367,28 @@ IBPM_DST_KERNEL(k_dst_pass2, dst_threads(M)) {
                 gout(J.u)[(long)(k - 1) * N2 + la] = -z.y;
                 if (la + 1 < N2) gout(J.u)[(long)(k - 1) * N2 + la + 1] = z.x;
             } else if (k - 1 >= t2_lo && k - 1 <= t2_hi) {   // rows outside are not read
-                *(IBPM_GLOBAL Pair*)(T + (k - 1) * ld + la) = Pair{-z.y, z.x};
+                *(IBPM_GLOBAL Pair*)((it == 1 ? T : Tb) + (k - 1) * ld + la) = Pair{-z.y, z.x};
+            }
+            if (BOTH && it == 1) {   // (every thread has read y: the transform's barriers lie between)
+                const double l1 = 2. * (cx[slot] + ca - 2.) * bydx2, l2 = 2. * (cx[slot] + cb - 2.) * bydx2;
+                y[k] = make_double2(sb * y[k].x * (1. / l1), sb * y[k].y * (1. / l2));
             }
         });
         if (kind == 2) return;
         __syncthreads();
     }
 }
+
+#define IBPM_DST_PASS2(NAME, BOTH)                                                      \
+    IBPM_DST_KERNEL(NAME, dst_threads(M)) {                                             \
+        __shared__ double2 lds[LdsFft<M, dst_threads(M)>::kSlots], y[M / 2];            \
+        const int2 blk = xcd_block();                                                   \
+        const EllJob& J = jobs[blk.y];                                                  \
+        if (skipped(J.skip)) return;                                                    \
+        dst_pass2<M, BOTH>(J, blk.x, lds, y);                                           \
+    }
+IBPM_DST_PASS2(k_dst_pass2, false)
+IBPM_DST_PASS2(k_dst_pass2_both, true)
 
 // ---------------------------------------------------------------- pass 3
 IBPM_DST_KERNEL(k_dst_pass3, dst_threads(M)) {
@@ -516,7 +533,7 @@ IBPM_DST_KERNEL(k_dst_bc, dst_threads(M)) {
 }
 
 // ------------------------------------------------------------------ host
-// Launches of one pass (4: bc) over jobs of one length; false for a length
+// Launches of one pass (4: bc, 5: pass 2 of two solves) over jobs of one length; false for a length
 // that is not among the instantiated ones (dst_f64_*.hip).
 struct DstLaunch {
     int M, pass, blocks, njobs;
@@ -531,6 +548,7 @@ inline void launch_dst_len(const DstLaunch& L) {
     case 1: hipLaunchKernelGGL(k_dst_pass1<M>, grid, dim3(dst_threads(M)), 0, L.s, L.jobs); break;
     case 2: hipLaunchKernelGGL(k_dst_pass2<M>, grid, dim3(dst_threads(M)), 0, L.s, L.jobs); break;
     case 3: hipLaunchKernelGGL(k_dst_pass3<M>, grid, dim3(dst_threads(M)), 0, L.s, L.jobs); break;
+    case 5: hipLaunchKernelGGL(k_dst_pass2_both<M>, grid, dim3(dst_threads(M)), 0, L.s, L.jobs); break;
     default: hipLaunchKernelGGL(k_dst_bc<M>, grid, dim3(dst_threads(M)), 0, L.s, L.jobs); break;
     }
 }

@@ -1224,12 +1224,12 @@ void launch_ell_pass32(int pass, const EllJob* d_jobs, int njobs, int max_blocks
     }
 }
 
-// Pass 1..3 or bc (4) of jobs of one FFT length M (J.pi.M for pass 2, J.pj.M
-// for the others); regs: pass_in_registers for the launch, with max_blocks
+// Pass 1..3, bc (4) or pass 2 of two solves (5) of jobs of one FFT length M
+// (J.pi.M for passes 2 and 5, J.pj.M for the others); regs: pass_in_registers for the launch, with max_blocks
 // sized for that choice (bc runs the LDS transform at every length).
 void launch_ell_pass(int pass, const EllJob* d_jobs, int njobs, int max_blocks, hipStream_t s, int M, bool regs) {
     const dim3 grid(max_blocks, njobs);
-    if (regs && pass != 4) {
+    if (regs && pass < 4) {
         const int lds = (int)sizeof(double2) * r16_group(pass) * r16_buf(M), bt = r16_group(pass) * (M / 16);
         if (M == 2048) {
             if (pass == 1) hipLaunchKernelGGL(k_reg_pass1<2048>, grid, dim3(bt), lds, s, d_jobs);
