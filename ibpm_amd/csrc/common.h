@@ -65,7 +65,6 @@ struct EllJob {
     double* T1b;             // pass 2 of two solves: the second one's scratch, laid out as T1
     double scale_b;          // and its right-hand side, this times the first one's solution
     double* u;               // level slice of the solution
-    double* u2;              // null, or a second output of the same values (pass 3)
     const double* W;         // epilogue 1 operand (level slice)
     double* vside;           // epilogue solves, levels >= 1: v (before the epilogue) stored at
                              // the points the next finer level's getBC reads (level slice; FP32

@@ -426,10 +426,6 @@ IBPM_DST_KERNEL(k_dst_pass3, dst_threads(M)) {
         const double ua = J.epilogue ? wa[slot] - va : va, ub = J.epilogue ? wb[slot] - vb : vb;
         gout(J.u)[o + k - 1] = ua;
         if (hb) gout(J.u)[o + N2 + k - 1] = ub;
-        if (J.u2) {
-            gout(J.u2)[o + k - 1] = ua;
-            if (hb) gout(J.u2)[o + N2 + k - 1] = ub;
-        }
     });
 }
 

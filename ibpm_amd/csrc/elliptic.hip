@@ -506,7 +506,6 @@ __device__ __forceinline__ void pass3_lds(const EllJob& J, C* smem, int bx) {
             const double v = -(double)z.y * J.norm;
             const double uv = J.epilogue ? gin(J.W)[o] - v : v;
             gout(J.u)[o] = uv;
-            if (J.u2) gout(J.u2)[o] = uv;
             if (J.vside && on_bc_ring(J, ra + 1, k + 1)) gout(J.vside)[o] = v;
         }
         if (rb < N1) {
@@ -514,7 +513,6 @@ __device__ __forceinline__ void pass3_lds(const EllJob& J, C* smem, int bx) {
             const double v = (double)z.x * J.norm;
             const double uv = J.epilogue ? gin(J.W)[o] - v : v;
             gout(J.u)[o] = uv;
-            if (J.u2) gout(J.u2)[o] = uv;
             if (J.vside && on_bc_ring(J, rb + 1, k + 1)) gout(J.vside)[o] = v;
         }
     }
@@ -681,14 +679,12 @@ __device__ __forceinline__ void pass3_r16(const EllJob& J, double2* smem, int bx
             const double val_a = -z.y * J.norm;
             const double ua = J.epilogue ? gin(J.W)[o2] - val_a : val_a;
             gout(J.u)[o2] = ua;
-            if (J.u2) gout(J.u2)[o2] = ua;
         }
         if (hb) {
             const long o2 = (long)rb * N2 + k;
             const double val_b = z.x * J.norm;
             const double ub = J.epilogue ? gin(J.W)[o2] - val_b : val_b;
             gout(J.u)[o2] = ub;
-            if (J.u2) gout(J.u2)[o2] = ub;
         }
     });
 }
@@ -998,8 +994,8 @@ __global__ void __launch_bounds__(kHelmThreads) k_fs_chain(const HelmJob* __rest
 }
 
 // u = W - v over each job's box, v the local result (J.out): the epilogue of
-// the step's omega = omega* - A^-1 c, whose omega already holds omega* off the
-// boxes (the omega* solve writes both).
+// the step's omega = omega* - A^-1 c in place (W and u are one field, which off
+// the boxes holds omega* already).
 __global__ void __launch_bounds__(kThreads) k_helm_epilogue(const HelmJob* __restrict__ jobs) {
     const HelmJob& J = jobs[blockIdx.y];
     const int w = J.j1 - J.j0 + 1, h = J.i1 - J.i0 + 1;
@@ -1131,8 +1127,7 @@ __global__ void __launch_bounds__(64) k_gemm_dst(const EllJob* __restrict__ jobs
                         const double vv = (double)v * J.norm;
                         const double uv = J.epilogue ? gin(J.W)[o] - vv : vv;
                         gout(J.u)[o] = uv;
-                        if (J.u2) gout(J.u2)[o] = uv;
-                        if (J.vside && on_bc_ring(J, r + 1, c + 1)) gout(J.vside)[o] = vv;
+                                    if (J.vside && on_bc_ring(J, r + 1, c + 1)) gout(J.vside)[o] = vv;
                     }
                 } else {
                     if constexpr (STAGE == 2) {   // X2^T[l][k] / eigenvalue (EllipticSolver2d.cc:42-54, 89-93)

@@ -321,7 +321,6 @@ struct SolveSpec {
     const double* bcring;  // single-level explicit boundary values (L == 1 only)
     const double* skip;    // null, or the flow's force-solve flags
     double* vside;         // epilogue solves: side buffer (L levels) for the BC values of v
-    double* u2 = nullptr;  // null, or a second output (L levels) of the same values
 };
 
 // Optional per-launch timing: a HIP event pair around every kernel launch on
@@ -407,7 +406,6 @@ static void fill_ell_job(const SolveSpec& s, int lev, EllJob& J) {
     }
     J.ld1 = t1_ld(s.ny - 1);   // the scratch is sized for the padding
     J.u = s.u + lev * ns;
-    J.u2 = s.u2 ? s.u2 + lev * ns : nullptr;
     J.W = s.W ? s.W + lev * ns : nullptr;
     J.skip = s.skip;
 }
@@ -618,7 +616,7 @@ static int tune_plan_gemm(Ctx* c, DevMem& mem, SolvePlan& P, int mode) {
             EllJob* d = nullptr;
             CKR(mem.alloc(&out, maxns));
             for (auto& J : jobs) {   // write to scratch; no epilogue, side outputs or skip flags
-                J.u = out; J.u2 = nullptr; J.vside = nullptr; J.epilogue = 0; J.W = nullptr; J.skip = nullptr;
+                J.u = out; J.vside = nullptr; J.epilogue = 0; J.W = nullptr; J.skip = nullptr;
             }
             CKR(mem.alloc(&d, jobs.size()));
             CK(hipMemcpy(d, jobs.data(), sizeof(EllJob) * jobs.size(), hipMemcpyHostToDevice));
@@ -1486,7 +1484,13 @@ static int alloc_flow(ibpm_batch* B, Flow& F) {
     DevMem& m = B->mem;
     const long ns = F.ns * F.L, nf = F.nf * F.L;
     CKR(m.alloc(&F.omega, ns)); CKR(m.alloc(&F.q, nf)); CKR(m.alloc(&F.nprev, ns));
-    CKR(m.alloc(&F.a, ns)); CKR(m.alloc(&F.wstar, ns)); CKR(m.alloc(&F.psi, ns));
+    CKR(m.alloc(&F.a, ns)); CKR(m.alloc(&F.psi, ns));
+    // Moving bodies: omega* in omega's own place, so that omega = omega* - A^-1 c
+    // is formed over the boxes of its local form alone (plan_local_helm).  A copy
+    // of omega* beside it was a second output of the omega* solve's pass 3, 134
+    // MB a level of 16 flows of 1024^2.
+    if (B->any_cg) F.wstar = F.omega;
+    else CKR(m.alloc(&F.wstar, ns));
     CKR(m.alloc(&F.c, ns)); CKR(m.alloc(&F.R, ns)); CKR(m.alloc(&F.T1, (size_t)(F.nx - 1) * t1_ld(F.ny - 1) * (B->all_levels ? F.L : 1)));
     CKR(m.alloc(&F.T2, (size_t)(F.nx - 1) * t1_ld(F.ny - 1))); CKR(m.alloc(&F.mt, ns));
     CKR(m.alloc(&F.bcv, bcv_size(F.nx, F.ny) * F.L));
@@ -1552,9 +1556,6 @@ static int build_plans(ibpm_batch* B) {
         for (auto& F : B->flows) {
             const double alpha = -beta_of(B, F, i) / 2. * (1. / F.p.reynolds);   // ProjectionSolver.cc:33
             s1.push_back(spec_of(F, 1, alpha, F.a, F.wstar, 1.0, 0, nullptr));
-            // moving-body batches: omega = omega* too, for the local form of
-            // omega = omega* - A^-1 c (plan_local_helm)
-            if (B->any_cg) s1.back().u2 = F.omega;
             s2.push_back(spec_of(F, 0, 0.0, F.wstar, F.psi, -1.0, 0, nullptr));
             s3.push_back(spec_of(F, 1, alpha, F.c, F.omega, 1.0, 1, F.wstar));
             s3.back().vside = F.mt;   // M-temp is free after the force solve
@@ -2540,7 +2541,7 @@ static int substep_cg(ibpm_batch* B, int i) {
     if (B->helm_on[i]) {
         // omega = omega* - A^-1 c with c = beta B f local like M's right-hand
         // side: the same sweeps (plan_local_helm), then the subtraction over
-        // the boxes; off them omega already holds omega* (the S1 solve wrote it)
+        // the boxes; off them omega holds omega* (the S1 solve wrote it)
         for (int lev = 1; lev < (B->helm_chain ? 1 : B->S3[i].nlev); ++lev)
             timed(pr, K_HELM, 0, s, [&] { launch_helm_coarsify(B->d_helm3, B->helm_n, B->helm_cblocks, lev, s); });
         const int nl = helm_launches(B->helm_sweeps);
