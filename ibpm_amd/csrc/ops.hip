@@ -3,21 +3,11 @@
 // per-flow descriptors and is launched with blockIdx.y = flow, so one launch
 // advances a whole batch of flows of uneven size (blocks past a flow's extent
 // exit at once).
+#include "advect.h"
 #include "geometry.h"
 #include "ops.h"
 
 namespace ibpmg {
-
-// ------------------------------------------------------------ accessors
-struct Lay {
-    int nx, ny, L;
-    __device__ long ns() const { return (long)(nx - 1) * (ny - 1); }
-    __device__ long nf() const { return 2L * nx * ny + nx + ny; }
-    __device__ long nfx() const { return (long)(nx + 1) * ny; }
-    __device__ long s(int lev, int i, int j) const { return lev * ns() + (long)(i - 1) * (ny - 1) + (j - 1); }
-    __device__ long fx(int lev, int i, int j) const { return lev * nf() + (long)i * ny + j; }
-    __device__ long fy(int lev, int i, int j) const { return lev * nf() + nfx() + (long)i * (ny + 1) + j; }
-};
 
 // getBC of level lev from level lev+1 (reference Scalar.cc:91-127); zero on
 // the coarsest level (VectorOperations.cc:74-77).
@@ -456,142 +446,28 @@ __global__ void __launch_bounds__(kThreads) k_rhs(const FlowOps* __restrict__ fl
 // central region and the eight next to its corners, whose velocities and fluxes
 // follow the interface rules: as sums of at most 24 node values, one lane each
 // (rim_term), since one lane through all of a node's rules took 68 us on a 400^2
-// grid, nearly all of it latency.
-constexpr int kAdvI = 8, kAdvJ = 64, kRimLanes = 32;
-
-struct AdvShape {
-    int ti, tj, tiles;   // tiles per level
-    int rim, edge;       // rim nodes of a coarse level, edge values of a level below the coarsest
-};
-__host__ __device__ inline AdvShape adv_shape(int nx, int ny) {
-    AdvShape s;
-    s.ti = (nx - 1 + kAdvI - 1) / kAdvI;
-    s.tj = (ny - 1 + kAdvJ - 1) / kAdvJ;
-    s.tiles = s.ti * s.tj;
-    s.edge = 2 * (ny / 2 + 1) + 2 * (nx / 2 + 1);
-    s.rim = nx + ny + 8;
-    return s;
-}
-
-// Rim node m of a coarse level: rows ex and ex + nx/2 from column ey to ey +
-// ny/2, those columns of the rows between, then the two nodes outside each
-// corner.  False for one that is not of the level (small grids).
-__device__ inline bool rim_node(const Lay& g, int m, int& i, int& j) {
-    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
-    const int wide = g.ny / 2 + 1, tall = g.nx / 2 - 1;
-    if (m < 2 * wide) {
-        i = m < wide ? ex : hx;
-        j = ey + m % wide;
-    } else if (m < 2 * wide + 2 * tall) {
-        m -= 2 * wide;
-        j = m < tall ? ey : hy;
-        i = ex + 1 + m % tall;
-    } else {
-        m -= 2 * wide + 2 * tall;   // 0..7: past the corner along i, then along j
-        const bool e = m & 1, n = m & 2;
-        i = (e ? hx : ex) + (m < 4 ? (e ? 1 : -1) : 0);
-        j = (n ? hy : ey) + (m < 4 ? 0 : (n ? 1 : -1));
-    }
-    return i >= 1 && i <= g.nx - 1 && j >= 1 && j <= g.ny - 1;
-}
-__device__ inline bool is_rim(const Lay& g, int i, int j) {
-    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
-    const bool oni = i == ex || i == hx, onj = j == ey || j == hy;
-    const bool ini = i >= ex && i <= hx, inj = j >= ey && j <= hy;
-    return (oni && inj) || (onj && ini) || ((i == ex - 1 || i == hx + 1) && onj) || ((j == ey - 1 || j == hy + 1) && oni);
-}
-
-// A node value in a flux or at an edge: coef times U (u) or V at (lev, i, j).
-struct NodeTerm {
-    int lev, i, j;
-    bool u;
-    double coef;   // 0: no term
-};
-
-// Term t (0..2) of an X (x) or Y flux outside region G, i in 1..nx-1 of an X
-// flux and j in 1..ny-1 of a Y flux (the rules of xflux_from / yflux_from).
-__device__ inline NodeTerm flux_term(const Lay& g, double dx0, bool x, int lev, int i, int j, int t) {
-    const double dx = dx0 * (1 << lev);
-    const int along = x ? i : j, across = x ? j : i, n = x ? g.ny : g.nx;
-    if (across == 0 || across == n - 1) {   // next to the edge: the node inside, and the coarser level's
-        const int ea = nx_ext(x ? g.nx : g.ny), ec = nx_ext(n);
-        if (t == 0) {
-            const int in = across == 0 ? 1 : n - 1;
-            return NodeTerm{lev, x ? i : in, x ? in : j, !x, 0.5 * dx};
-        }
-        const int a = along / 2 + ea + (t - 1), c = across == 0 ? ec : n / 2 + ec;
-        const double coef = lev == g.L - 1 || (t == 2 && !(along & 1)) ? 0.0 : (along & 1) ? 0.25 * dx : 0.5 * dx;
-        return NodeTerm{lev + 1, x ? a : c, x ? c : a, !x, coef};
-    }
-    return NodeTerm{lev, x ? i : i + t, x ? j + t : j, !x, t < 2 ? 0.5 * dx : 0.0};
-}
-
-// Term m (0..23) of fy(i, j) - fy(i - 1, j) + fx(i, j - 1) - fx(i, j); a flux of
-// the central region is the sum of two of the finer level, which lie at that
-// level's edge (region G).
-__device__ inline NodeTerm rim_term(const Lay& g, double dx0, int lev, int i, int j, int m) {
-    const int f = m / 6, t = m % 6;
-    const bool x = f >= 2;
-    const int ii = f == 1 ? i - 1 : i, jj = f == 2 ? j - 1 : j;
-    const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
-    const bool fine = lev > 0 && (x ? ii > ex && ii < hx && jj >= ey && jj < hy : jj > ey && jj < hy && ii >= ex && ii < hx);
-    NodeTerm r{0, 1, 1, false, 0.0};
-    if (f > 3) return r;
-    if (fine) r = flux_term(g, dx0, x, lev - 1, 2 * (ii - ex) + (x ? 0 : t / 3), 2 * (jj - ey) + (x ? t / 3 : 0), t % 3);
-    else if (t < 3) r = flux_term(g, dx0, x, lev, ii, jj, t);
-    if (f & 1) r.coef = -r.coef;
-    return r;
-}
-
-// Offsets of the two values whose mean a level's field has at (i, j), 0 <= i <=
-// nx, 0 <= j <= ny, off its corners: its own value twice inside, getBC's of the
-// coarser level (Scalar.cc:91-127) on the boundary.  False (offsets of the
-// nearest node): 0 on the coarsest level's boundary.
-__device__ inline bool halo_at(const Lay& g, int lev, int i, int j, unsigned& a, unsigned& b) {
-    const unsigned ny1 = (unsigned)(g.ny - 1), base = (unsigned)(lev * g.ns());
-    const int ci = min(max(i, 1), g.nx - 1), cj = min(max(j, 1), g.ny - 1);
-    a = b = base + (unsigned)(ci - 1) * ny1 + (unsigned)(cj - 1);
-    if (ci == i && cj == j) return true;
-    if (lev == g.L - 1) return false;
-    const bool side = ci != i;   // on left or right, else on bottom or top
-    const int ii = nx_ext(g.nx) + i / 2, jj = nx_ext(g.ny) + j / 2;
-    a = base + (unsigned)g.ns() + (unsigned)(min(max(ii, 1), g.nx - 1) - 1) * ny1 + (unsigned)(min(max(jj, 1), g.ny - 1) - 1);
-    b = a + (side ? (unsigned)(j & 1) : (i & 1) * ny1);
-    return true;
-}
+// grid, nearly all of it latency.  (advect.h has the index rules.)
 
 // U (u) or V of the cross product at a node, from psi and the base flow of the
 // last refresh (FlowOps::bf[3..5]), as node_u and node_v give it from q, with
 // every load issued before any is used: the node velocity as a sum of at most
 // four fluxes (the rules of xvel and yvel), each a difference of two psi values.
 __device__ inline double node_value(const FlowOps& F, const Lay& g, const NodeTerm& t) {
-    const int lev = t.lev, na = t.u ? g.nx : g.ny, nc = t.u ? g.ny : g.nx;   // along and across the flux pair
-    const int al = t.u ? t.i : t.j, ac = t.u ? t.j : t.i;
-    const int alo = nx_ext(na), ahi = alo + na / 2, clo = nx_ext(nc), chi = clo + nc / 2;
-    const double bydx = 1. / (F.dx * (1 << lev));
-    const bool rim = lev >= 1 && (ac == clo || ac == chi) && al >= alo && al <= ahi;
-    const bool corner = rim && (al == alo || al == ahi), face = rim && !corner;
-    const int c0 = ac == clo ? ac - 1 : ac, c1 = ac == clo ? ac : ac - 1;   // outside the rim, inside it
-    const int cf = ac == clo ? 0 : nc - 1, af = face ? 2 * (al - alo) : al == alo ? 1 : na - 1;
-    // fluxes (level, along, across) and coefficients
-    const int fl[4] = {lev, (face ? lev - 1 : lev), rim ? lev - 1 : lev, rim ? lev - 1 : lev};
-    const int fa[4] = {al, face ? af : al, face ? af - 1 : corner ? af : al, face ? af + 1 : al};
-    const int fc[4] = {rim ? c0 : ac, face ? cf : corner ? c1 : ac - 1, rim ? cf : ac, rim ? cf : ac};
-    const double co[4] = {face ? 2. / 3 : corner ? 8. / 15 : 0.5, face ? 1. / 3 : corner ? 6. / 15 : 0.5,
-                          face ? 1. / 6 : corner ? 2. / 15 : 0.0, face ? 1. / 6 : 0.0};
+    const double bydx = 1. / (F.dx * (1 << t.lev));
+    const NodeFluxes f = node_fluxes(g, t);
     double v = 0.0, v0 = 0.0;
     const IBPM_GLOBAL double* P = gin(F.psi);
     const bool base = has_base(F.model);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int l = max(fl[k], 0), i = t.u ? fa[k] : fc[k], j = t.u ? fc[k] : fa[k];
+        const int l = f.lev[k], i = f.i[k], j = f.j[k];
         unsigned a0, a1, b0, b1;   // X flux (i, j): psi(i, j + 1) - psi(i, j); Y flux: psi(i, j) - psi(i + 1, j)
         const bool p = halo_at(g, l, t.u ? i : i + 1, t.u ? j + 1 : j, a0, a1), m = halo_at(g, l, i, j, b0, b1);
         const double x = (p ? 0.5 : 0.0) * (P[a0] + P[a1]), y = (m ? 0.5 : 0.0) * (P[b0] + P[b1]);
-        v += co[k] * ((t.u ? x - y : y - x) + (t.u ? base_x(F, F.bf + 3, l, j) : base_y(F, F.bf + 3, l, i)));
-        if (base) v0 += co[k] * gin(F.q0b)[t.u ? g.fx(l, i, j) : g.fy(l, i, j)];
+        v += f.co[k] * ((t.u ? x - y : y - x) + (t.u ? base_x(F, F.bf + 3, l, j) : base_y(F, F.bf + 3, l, i)));
+        if (base) v0 += f.co[k] * gin(F.q0b)[t.u ? g.fx(l, i, j) : g.fy(l, i, j)];
     }
-    const long at = g.s(lev, t.i, t.j);
+    const long at = g.s(t.lev, t.i, t.j);
     const double w0 = base ? gin(F.w0b)[at] : 0.0;
     return cross_node(F.model, t.u ? -1.0 : 1.0, v * bydx, gin(F.omega)[at], v0 * bydx, w0);
 }
@@ -604,7 +480,7 @@ __device__ inline double lap_at(const Lay& g, const double* f, int lev, int i, i
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         unsigned a, b;
-        const bool in = halo_at(g, lev, i + (k == 0) - (k == 1), j + (k == 2) - (k == 3), a, b);
+        const bool in = neighbour_at(g, lev, i, j, k, a, b);
         x[k] = (in ? 0.5 : 0.0) * (P[a] + P[b]);
     }
     return -(((c - x[0]) - (x[1] - c) + (c - x[3]) - (x[2] - c)) * bydx2);
@@ -613,41 +489,24 @@ __device__ inline double lap_at(const Lay& g, const double* f, int lev, int i, i
 __global__ void __launch_bounds__(kThreads) k_advect_rim(const FlowOps* __restrict__ flows) {
     const FlowOps& F = flows[blockIdx.y];
     const Lay g{F.nx, F.ny, F.L};
-    const AdvShape S = adv_shape(g.nx, g.ny);
-    const int idx = blockIdx.x * kThreads + threadIdx.x, nrim = (g.L - 1) * S.rim * kRimLanes;
-    const bool rim = idx < nrim;
-    int lev = 0, i = 1, j = 1, at = 0;
-    bool node = false;
-    NodeTerm t{0, 1, 1, false, 0.0};
-    if (rim) {
-        const int k = idx / kRimLanes;
-        lev = k / S.rim + 1;
-        node = rim_node(g, k % S.rim, i, j);
-        if (node) t = rim_term(g, F.dx, lev, i, j, idx % kRimLanes);
-    } else {   // U at the coarser level's nodes along left and right, V along bottom and top
-        at = idx - nrim;
-        if (at >= (g.L - 1) * S.edge) return;   // (whole waves: 32 lanes a rim node)
-        const int l = at / S.edge, wide = g.ny / 2 + 1, tall = g.nx / 2 + 1;
-        const int ex = nx_ext(g.nx), ey = nx_ext(g.ny);
-        int m = at % S.edge;
-        const bool u = m < 2 * wide;
-        if (!u) m -= 2 * wide;
-        if (u) t = NodeTerm{l + 1, m < wide ? ex : ex + g.nx / 2, ey + m % wide, true, 1.0};
-        else t = NodeTerm{l + 1, ex + m % tall, m < tall ? ey : ey + g.ny / 2, false, 1.0};
-    }
+    const int idx = blockIdx.x * kThreads + threadIdx.x;
+    const RimLane r = rim_lane(g, adv_shape(g.nx, g.ny), F.dx, idx);
+    if (!r.used) return;   // (whole waves: 32 lanes a rim node)
+    const int lev = r.lev, i = r.i, j = r.j;
+    const NodeTerm& t = r.t;
     const double d = F.dx * (1 << lev), bydx2 = 1. / (d * d);
     const unsigned tu = (unsigned)g.s(lev, i, j);
     const double c = gin(F.omega)[tu], np = gin(F.nprev)[tu];
     const double lap = lap_at(g, F.omega, lev, i, j, bydx2);
     const double ls = F.model == 2 ? lap_at(g, F.sff, lev, i, j, bydx2) : 0.0;
     double v = t.coef != 0.0 ? t.coef * node_value(F, g, t) : 0.0;
-    if (!rim) {
-        gout(F.edge)[at] = v;
+    if (!r.rim) {
+        gout(F.edge)[r.at] = v;
         return;
     }
 #pragma unroll
     for (int off = kRimLanes / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (!node || idx % kRimLanes != 0) return;
+    if (!r.node || idx % kRimLanes != 0) return;
     rhs_node(F, F.model, tu, c, v * bydx2, ls, lap, np);
     if (F.model == 4) sfd_node(F, tu, c);
 }
