@@ -90,19 +90,38 @@ __host__ __device__ inline NodeTerm flux_term(const Lay& g, double dx0, bool x, 
     return NodeTerm{lev, x ? i : i + t, x ? j + t : j, !x, t < 2 ? 0.5 * dx : 0.0};
 }
 
-// Term m (0..23) of fy(i, j) - fy(i - 1, j) + fx(i, j - 1) - fx(i, j); a flux of
-// the central region is the sum of two of the finer level, which lie at that
-// level's edge (region G).
-__host__ __device__ inline NodeTerm rim_term(const Lay& g, double dx0, int lev, int i, int j, int m) {
-    const int f = m / 6, t = m % 6;
-    const bool x = f >= 2;
-    const int ii = f == 1 ? i - 1 : i, jj = f == 2 ? j - 1 : j;
+// Region G of a coarse level: the fluxes that are the sum of two of the finer
+// level, (2 (i - ex), 2 (j - ey) + 0, 1) of an X flux (VectorOperations.cc:669-915).
+__host__ __device__ inline bool flux_central(const Lay& g, bool x, int lev, int i, int j) {
     const int ex = nx_ext(g.nx), ey = nx_ext(g.ny), hx = ex + g.nx / 2, hy = ey + g.ny / 2;
-    const bool fine = lev > 0 && (x ? ii > ex && ii < hx && jj >= ey && jj < hy : jj > ey && jj < hy && ii >= ex && ii < hx);
+    return lev > 0 && (x ? i > ex && i < hx && j >= ey && j < hy : j > ey && j < hy && i >= ex && i < hx);
+}
+
+// Number of terms of a rim node's curl: a flux of region G is two of the finer
+// level, next to that level's edge, three node values each. With four cells
+// across the pair, one of the two lies in the finer level's own region G, so that the
+// pairs go on down to level 0.
+__host__ __device__ inline int rim_terms(const Lay& g, int lev) {
+    return g.nx == 4 || g.ny == 4 ? 12 * (lev + 1) : 24;
+}
+
+// Term m (0 .. rim_terms - 1) of fy(i, j) - fy(i - 1, j) + fx(i, j - 1) - fx(i, j).
+__host__ __device__ inline NodeTerm rim_term(const Lay& g, double dx0, int lev, int i, int j, int m) {
+    const int per = rim_terms(g, lev) / 4, f = m / per, t = m % per;
+    const bool x = f >= 2;
+    int l = lev, ii = f == 1 ? i - 1 : i, jj = f == 2 ? j - 1 : j, d = t / 3;
     NodeTerm r{0, 1, 1, false, 0.0};
     if (f > 3) return r;
-    if (fine) r = flux_term(g, dx0, x, lev - 1, 2 * (ii - ex) + (x ? 0 : t / 3), 2 * (jj - ey) + (x ? t / 3 : 0), t % 3);
-    else if (t < 3) r = flux_term(g, dx0, x, lev, ii, jj, t);
+    // flux d of the chain: a pair's member outside region G, then on with the other
+    for (; flux_central(g, x, l, ii, jj); --d) {
+        ii = 2 * (ii - nx_ext(g.nx));
+        jj = 2 * (jj - nx_ext(g.ny));
+        --l;
+        const bool first = !flux_central(g, x, l, ii, jj);   // the member that the chain ends at
+        if ((d == 0) != first) (x ? jj : ii) += 1;
+        if (d == 0) break;
+    }
+    if (d == 0) r = flux_term(g, dx0, x, l, ii, jj, t % 3);
     if (f & 1) r.coef = -r.coef;
     return r;
 }
@@ -153,24 +172,26 @@ __host__ __device__ inline NodeFluxes node_fluxes(const Lay& g, const NodeTerm& 
     return f;
 }
 
-// Lane idx of k_advect_rim: kRimLanes lanes per rim node, one node value each
-// (t), then one lane per edge value (slot at of FlowOps::edge).  (lev, i, j) is
-// the rim node; every lane's is a node of the grid, since the kernel's loads at
-// it are under no branch.
+// Lane idx of k_advect_rim: kRimLanes lanes per rim node, which share its terms
+// (first, first + kRimLanes, .. below n), then one lane per edge value (slot at of
+// FlowOps::edge, the one term t).  (lev, i, j) is the rim node; every lane's is a
+// node of the grid, since the kernel's loads at it are under no branch.
 struct RimLane {
     bool used, rim, node;   // node: a rim node of the level
     int lev, i, j, at;
+    int first, n;
     NodeTerm t;
 };
-__host__ __device__ inline RimLane rim_lane(const Lay& g, const AdvShape& S, double dx0, int idx) {
-    RimLane r{true, false, false, 0, 1, 1, 0, NodeTerm{0, 1, 1, false, 0.0}};
+__host__ __device__ inline RimLane rim_lane(const Lay& g, const AdvShape& S, int idx) {
+    RimLane r{true, false, false, 0, 1, 1, 0, 0, 1, NodeTerm{0, 1, 1, false, 0.0}};
     const int nrim = (g.L - 1) * S.rim * kRimLanes;
     r.rim = idx < nrim;
     if (r.rim) {
         const int k = idx / kRimLanes;
         r.lev = k / S.rim + 1;
         r.node = rim_node(g, k % S.rim, r.i, r.j);
-        if (r.node) r.t = rim_term(g, dx0, r.lev, r.i, r.j, idx % kRimLanes);
+        r.first = idx % kRimLanes;
+        r.n = r.node ? rim_terms(g, r.lev) : 0;
         return r;
     }
     // U at the coarser level's nodes along left and right, V along bottom and top

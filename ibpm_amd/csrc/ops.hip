@@ -444,8 +444,8 @@ __global__ void __launch_bounds__(kThreads) k_rhs(const FlowOps* __restrict__ fl
 //
 // k_advect_rim, before it, also forms the nodes on the rim of a coarse level's
 // central region and the eight next to its corners, whose velocities and fluxes
-// follow the interface rules: as sums of at most 24 node values, one lane each
-// (rim_term), since one lane through all of a node's rules took 68 us on a 400^2
+// follow the interface rules: as sums of 24 node values at most (more on four cells
+// a side), one lane each (rim_term), since one lane through all of a node's rules took 68 us on a 400^2
 // grid, nearly all of it latency.  (advect.h has the index rules.)
 
 // U (u) or V of the cross product at a node, from psi and the base flow of the
@@ -490,16 +490,19 @@ __global__ void __launch_bounds__(kThreads) k_advect_rim(const FlowOps* __restri
     const FlowOps& F = flows[blockIdx.y];
     const Lay g{F.nx, F.ny, F.L};
     const int idx = blockIdx.x * kThreads + threadIdx.x;
-    const RimLane r = rim_lane(g, adv_shape(g.nx, g.ny), F.dx, idx);
-    if (!r.used) return;   // (whole waves: 32 lanes a rim node)
+    const RimLane r = rim_lane(g, adv_shape(g.nx, g.ny), idx);
+    if (!r.used) return;   // (whole groups of kRimLanes: a rim node's lanes all stay)
     const int lev = r.lev, i = r.i, j = r.j;
-    const NodeTerm& t = r.t;
     const double d = F.dx * (1 << lev), bydx2 = 1. / (d * d);
     const unsigned tu = (unsigned)g.s(lev, i, j);
     const double c = gin(F.omega)[tu], np = gin(F.nprev)[tu];
     const double lap = lap_at(g, F.omega, lev, i, j, bydx2);
     const double ls = F.model == 2 ? lap_at(g, F.sff, lev, i, j, bydx2) : 0.0;
-    double v = t.coef != 0.0 ? t.coef * node_value(F, g, t) : 0.0;
+    double v = 0.0;
+    for (int m = r.first; m < r.n; m += kRimLanes) {   // (once, but on grids of four cells a side)
+        const NodeTerm t = r.rim ? rim_term(g, F.dx, lev, i, j, m) : r.t;
+        if (t.coef != 0.0) v += t.coef * node_value(F, g, t);
+    }
     if (!r.rim) {
         gout(F.edge)[r.at] = v;
         return;

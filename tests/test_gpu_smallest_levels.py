@@ -8,7 +8,9 @@ from tests.helpers import G
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(4, 4, 2), (4, 16, 2), (16, 4, 2), (4, 40, 2), (8, 4, 2)]
+SHAPES = [(4, 4, 2), (4, 16, 2), (16, 4, 2), (4, 40, 2), (8, 4, 2),
+          # fluxes of a central region that go down through the levels between
+          (16, 4, 3), (4, 16, 3), (4, 4, 4), (4, 40, 5)]
 MODELS = ["nonlinear", "linear", "adjoint", "sfd", "ubf"]
 
 
