@@ -963,6 +963,9 @@ struct ibpm_batch {
     int nsub = 3;
     double an[4], bn[4], cn[4];
     bool all_stationary = true, any_cg = false, initialized = false, any_ubf = false;
+    // q is formed from psi at the end of an advance.  psi_fresh: psi (and the
+    // base flow) are those of the last completed substep; q_fresh: q is.
+    bool psi_fresh = false, q_fresh = true;
     bool any_periodic = false, any_adjoint = false;
     bool any_plain = false, any_other = false;   // flows of the nonlinear model, of others
     // the solves keep T of every level and run passes 1 and 3 over all levels
@@ -2099,16 +2102,31 @@ static void enqueue_rhs(ibpm_batch* B, int i, hipStream_t s) {
 }
 
 static void enqueue_q(ibpm_batch* B, hipStream_t s) {
+    B->q_fresh = true;
     timed(B->probe, K_CURLQ, B->bytes_curlq, s,
           [&] { launch_curl_q(B->d_fops[0], (int)B->flows.size(), B->max_cells_all, s); });
 }
 
+// A substep's work is queued: psi is that of the new vorticity, and q too where
+// the substep forms it.
+static void substep_done(ibpm_batch* B) {
+    B->psi_fresh = true;
+    B->q_fresh = B->any_adjoint;
+}
+
 // psi of the new vorticity, which the next substep's right-hand side starts
 // from; q = Curl psi + q0 is formed where it is read: at the end of an advance
-// (enqueue_q), and after every substep for the adjoint model's cross product.
+// (form_q), and after every substep for the adjoint model's cross product.
 static void enqueue_refresh(ibpm_batch* B, hipStream_t s) {
     run_solve(B->S4, s, B->probe);
+    substep_done(B);
     if (B->any_adjoint) enqueue_q(B, s);
+}
+
+// q of the last completed substep, if an advance may still form it (an error
+// inside a substep's solves leaves no psi to form it from).
+static void form_q(ibpm_batch* B, hipStream_t s) {
+    if (!B->q_fresh && B->psi_fresh) enqueue_q(B, s);
 }
 
 // The stationary-body (Cholesky) substep: fixed launch sequence.  br: null, or
@@ -2425,6 +2443,10 @@ static int substep_cg(ibpm_batch* B, int i) {
     hipStream_t s = B->ctx->c.stream;
     const int nfl = (int)B->flows.size();
     const double t_kin = now_s();
+    // building P allocates n x n matrices in the middle of the substep, when psi
+    // is no longer the last one's: should that fail, q is there
+    if (B->pc_mode && !B->pc_broken && !B->pc_valid) form_q(B, s);
+    if (B->any_ubf) B->psi_fresh = false;   // the base flow moves on
     // updateOperators(t + c_n dt), IBSolver.cc:164-166: kinematics and
     // regulariser lists of the moving flows, computed during the previous
     // substep (kinematics_ahead) or here on host threads, then the uploads
@@ -2458,6 +2480,7 @@ static int substep_cg(ibpm_batch* B, int i) {
     // P's refresh at this substep's points, beside the step solves (whose
     // transforms leave CUs idle; the stencils above fill the GPU)
     if (B->pc_mode && !B->pc_broken && B->pc_valid && B->pc_build_levels == 3) CKR(refresh_precond(B, i));
+    B->psi_fresh = false;
     run_solve(B->S1[i], s, pr);
     run_solve(B->S2[i], s, pr);
     timed(pr, K_INTERP, pr ? reg_bytes(B, false, true) : 0, s,
@@ -4293,8 +4316,7 @@ static int select_phase(ibpm_batch* B) {
     return 0;
 }
 
-int ibpm_batch_advance(ibpm_batch* B, int nsteps) {
-    if (!B->initialized) { set_error("ibpm_batch_init not called"); return -1; }
+static int advance_steps(ibpm_batch* B, int nsteps) {
     hipStream_t s = B->ctx->c.stream;
     for (int step = 0; step < nsteps; ++step) {
         if (B->any_periodic) CKR(select_phase(B));
@@ -4324,12 +4346,16 @@ int ibpm_batch_advance(ibpm_batch* B, int nsteps) {
                 track_graph(B, true);
                 CK(hipGraphDestroy(g));
             }
+            B->psi_fresh = false;
             CK(hipGraphLaunch(B->graph, s));
+            substep_done(B);
         } else {
             for (int i = 0; i < B->nsub; ++i) {
+                B->psi_fresh = false;
                 for (auto& F : B->flows)   // updateOperators(t + c_n dt), IBSolver.cc:164-166
                     if (F.ubf) CKR(move_base_flow(B, F, B->time + B->cn[i] * F.p.dt));
                 CKR(enqueue_substep_chol(B, i, s));
+                substep_done(B);
                 if (i == 0 && !B->old_saved) {
                     CK(hipStreamSynchronize(s));
                     mark_nprev_valid(B);
@@ -4347,7 +4373,18 @@ int ibpm_batch_advance(ibpm_batch* B, int nsteps) {
             F.alpha_hist.push_back(F.force_alpha);
         }
     }
-    if (nsteps > 0 && !B->any_adjoint) enqueue_q(B, s);
+    return 0;
+}
+
+int ibpm_batch_advance(ibpm_batch* B, int nsteps) {
+    if (!B->initialized) { set_error("ibpm_batch_init not called"); return -1; }
+    hipStream_t s = B->ctx->c.stream;
+    const int rc = advance_steps(B, nsteps);
+    form_q(B, s);   // also of the steps before one that failed
+    if (rc) {
+        (void)hipStreamSynchronize(s);
+        return rc;
+    }
     CK(hipStreamSynchronize(s));
     CK(hipGetLastError());
     return 0;
@@ -4456,6 +4493,10 @@ int ibpm_batch_set_state(ibpm_batch* B, int k, const double* h_omega, const doub
 int ibpm_batch_get_q(ibpm_batch* B, int k, double* h) {
     Flow* F = flow_of(B, k);
     if (!F) return -1;
+    if (!B->q_fresh) {
+        set_error("no flux: the last advance failed inside a substep (set the vorticity or the state anew)");
+        return -1;
+    }
     CK(hipMemcpy(h, F->q, sizeof(double) * F->nf * F->L, hipMemcpyDeviceToHost));
     return 0;
 }
