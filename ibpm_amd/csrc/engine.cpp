@@ -115,22 +115,32 @@ constexpr size_t kDescBytes = size_t(1) << 17;
 // allocating, clearing and freeing its buffers and one blocking copy per
 // descriptor (127 us in all): buffers come from the context's workspace, which
 // grows to the largest call so far, and the descriptors go up in one copy.
-// Memory is not cleared.  Scopes nest (a call made of others); the stream must
-// have drained before the scope ends.
+// Memory is not cleared.  Scopes nest (a call made of others).  A scope that ends
+// before finish() (an error's return) waits for the stream, whose work reads the
+// workspace and the pinned descriptors.  An error that this call has returned, or
+// a workspace that could not grow, is not left for a later call's hipGetLastError.
 struct OpScope {
     Ctx* c;
     size_t base, desc_base, need;
     std::vector<void*> extra;
+    bool drained = false;
     explicit OpScope(Ctx* ctx) : c(ctx), base(ctx->ws_used), desc_base(ctx->desc_used), need(ctx->ws_used) {}
     ~OpScope() {
-        if (!extra.empty()) (void)hipStreamSynchronize(c->stream);   // (an error's return may come before)
+        if (!drained) {
+            (void)hipStreamSynchronize(c->stream);
+            (void)hipGetLastError();
+        }
         for (void* p : extra) (void)hipFree(p);
         c->ws_used = base;
         c->desc_used = desc_base;
         if (base == 0 && need > c->ws_cap && need <= kWsMax) {
             if (c->ws) (void)hipFree(c->ws);
+            c->ws = nullptr;
             c->ws_cap = hipMalloc((void**)&c->ws, need) == hipSuccess ? need : 0;
-            if (!c->ws_cap) c->ws = nullptr;
+            if (!c->ws_cap) {   // the next call allocates for itself again
+                c->ws = nullptr;
+                (void)hipGetLastError();
+            }
         }
     }
     template <class T>
@@ -151,10 +161,9 @@ struct OpScope {
     // Device address of n descriptors, valid after flush().
     template <class T>
     int put(T** out, const T* h, size_t n) {
-        if (!c->desc) {
-            CK(hipMalloc((void**)&c->desc, kDescBytes));
-            CK(hipHostMalloc((void**)&c->h_desc, kDescBytes, hipHostMallocDefault));
-        }
+        // (each by itself: the first may be there from a call in which the second failed)
+        if (!c->desc) CK(hipMalloc((void**)&c->desc, kDescBytes));
+        if (!c->h_desc) CK(hipHostMalloc((void**)&c->h_desc, kDescBytes, hipHostMallocDefault));
         const size_t bytes = (n * sizeof(T) + 255) & ~size_t(255);
         if (c->desc_used + bytes > kDescBytes) { set_error("%zu descriptor bytes exceed the limit", bytes); return -2; }
         std::memcpy(c->h_desc + c->desc_used, h, n * sizeof(T));
@@ -169,6 +178,7 @@ struct OpScope {
     }
     int finish() {
         CK(hipStreamSynchronize(c->stream));
+        drained = true;
         CK(hipGetLastError());
         return 0;
     }

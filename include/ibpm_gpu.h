@@ -6,8 +6,12 @@
  * the failure (per host thread).  Calls are ordered on the context's single
  * HIP stream; a context is not thread-safe, but batches on different contexts
  * may be driven from different host threads at once (their work then shares
- * the GPU, one stream each).  "d_" pointers are device pointers (allocate
- * them with ibpm_malloc or any HIP allocator on the context's device).
+ * the GPU, one stream each).  A context keeps the device memory that its largest
+ * stand-alone call (the solves and grid operators below) worked in, at most 1 GiB,
+ * for the calls that follow; ibpm_ctx_destroy gives it back.  A call that needs
+ * more allocates for itself and frees it before it returns.  "d_" pointers are
+ * device pointers (allocate them with ibpm_malloc or any HIP allocator on the
+ * context's device).
  *
  * Layouts are the reference's (so a host Scalar/Flux/BoundaryVector buffer
  * copies 1:1):
