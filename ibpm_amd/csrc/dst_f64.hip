@@ -25,7 +25,10 @@ namespace ibpmg {
 
 #define IBPM_DST_NAME2(k) launch_dst_##k
 #define IBPM_DST_NAME(k) IBPM_DST_NAME2(k)
-#define IBPM_CASE(M) case M: launch_dst_len<M>(L); return true;
+#define IBPM_CASE(M)                         \
+    case M:                                  \
+        if (L.njobs) launch_dst_len<M>(L);   \
+        return true;
 
 bool IBPM_DST_NAME(IBPM_DST_PART)(const DstLaunch& L) {
     switch (L.M) {

@@ -529,8 +529,9 @@ IBPM_DST_KERNEL(k_dst_bc, dst_threads(M)) {
 }
 
 // ------------------------------------------------------------------ host
-// Launches of one pass (4: bc, 5: pass 2 of two solves) over jobs of one length; false for a length
-// that is not among the instantiated ones (dst_f64_*.hip).
+// Launches of one pass (4: bc, 5: pass 2 of two solves) over jobs of one length
+// (none without jobs); false for a length that is not among the instantiated
+// ones (dst_f64.hip).
 struct DstLaunch {
     int M, pass, blocks, njobs;
     const EllJob* jobs;

@@ -1174,6 +1174,13 @@ bool launch_dst_5(const DstLaunch& L);
 bool launch_dst_6(const DstLaunch& L);
 bool launch_dst_7(const DstLaunch& L);
 
+static bool launch_dst(const DstLaunch& L) {
+    return launch_dst_0(L) || launch_dst_1(L) || launch_dst_2(L) || launch_dst_3(L) || launch_dst_4(L) ||
+           launch_dst_5(L) || launch_dst_6(L) || launch_dst_7(L);
+}
+
+bool dst_length_built(int M) { return launch_dst(DstLaunch{M, 1, 0, 0, nullptr, nullptr}); }
+
 int blocks_for_pass(const EllJob& J, int pass, bool regs) {
     const int M = pass == 2 ? J.pi.M : J.pj.M, bt = dst_threads(M);
     if (pass == 4) return 1 + (J.bcring ? (J.nx - 1 + bt - 1) / bt : (J.nx / 2 + bt / 64 * kBcRows - 1) / (bt / 64 * kBcRows));
@@ -1237,9 +1244,7 @@ void launch_ell_pass(int pass, const EllJob* d_jobs, int njobs, int max_blocks, 
         }
         return;
     }
-    const DstLaunch L{M, pass, max_blocks, njobs, d_jobs, s};
-    (void)(launch_dst_0(L) || launch_dst_1(L) || launch_dst_2(L) || launch_dst_3(L) || launch_dst_4(L) ||
-           launch_dst_5(L) || launch_dst_6(L) || launch_dst_7(L));
+    (void)launch_dst(DstLaunch{M, pass, max_blocks, njobs, d_jobs, s});   // (plans are of built lengths)
 }
 
 void launch_helm_coarsify(const HelmJob* d_jobs, int njobs, int max_blocks, int lev, hipStream_t s) {

@@ -244,6 +244,7 @@ static int plan_shape(int N, FftPlan* P) {
     while (m % 5 == 0) { P->rad[P->nst++] = 5; m /= 5; }
     while (m % 3 == 0) { P->rad[P->nst++] = 3; m /= 3; }
     if (m != 1) { set_error("DST length %d: 2(N+1) has a prime factor > 5", N); return -2; }
+    if (!dst_length_built(P->M)) { set_error("DST length %d: no transform of length %d is compiled", N, P->M); return -2; }
     P->np = std::max(1, std::min(kFftNpMax, kFftLds / P->M));
     return 0;
 }

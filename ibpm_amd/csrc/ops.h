@@ -173,6 +173,9 @@ struct ForceOps {
 // that choice.  Passes 1 to 3, and 4 for the boundary values of the next finer
 // level (dst_passes.h).
 bool pass_in_registers(int M, long row_pairs);
+// Whether the FP64 passes of FFT length M are compiled (dst_f64.hip); a launch of
+// another length would do nothing, so no plan of one is made.
+bool dst_length_built(int M);
 int blocks_for_pass(const EllJob& J, int pass, bool regs);
 void launch_ell_pass(int pass, const EllJob* d_jobs, int njobs, int max_blocks, hipStream_t s, int M, bool regs);
 int blocks_for_pass32(const EllJob& J, int pass);
