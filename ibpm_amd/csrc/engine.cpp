@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/ibpm_gpu.h"
+#include "dst_tables.h"
 #include "geometry.h"
 #include "learn.h"
 #include "ops.h"
@@ -249,36 +250,7 @@ static int plan_shape(int N, FftPlan* P) {
     return 0;
 }
 
-// Whether a plan of FFT length M has the second-stage table tw16.
-static bool plan_has_tw16(int M) { return M == 1024 || M == 2048; }
-
-// Host values of a plan's tables: tw (M entries), t16 (256 entries, where
-// plan_has_tw16), and the real tables cosn, sin1 (t1_ld(N) each) and ring
-// (2 N) one after another (plan_reals(N) doubles); see FftPlan.
-static size_t plan_reals(int N) { return 2 * (size_t)t1_ld(N) + 2 * (size_t)N; }
-
-static void plan_tables(int M, double2* tw, double2* t16, double* reals) {
-    const double twopi = 8.0 * std::atan(1.0), pi = 4. * std::atan(1.0);
-    for (int k = 0; k < M; ++k) {
-        const double a = -twopi * (double)k / (double)M;
-        tw[k] = make_double2(std::cos(a), std::sin(a));
-    }
-    if (plan_has_tw16(M)) {   // second-stage table of the register-held transforms
-        const int tstep = M / 256;
-        for (int r = 0; r < 16; ++r)
-            for (int jm = 0; jm < 16; ++jm) t16[16 * r + jm] = tw[(tstep * jm * r) % M];
-    }
-    const int n = M / 2, N = n - 1, e = nx_ext(n);
-    double *cosn = reals, *sin1 = cosn + t1_ld(N), *ring = sin1 + t1_ld(N);
-    for (int i = N; i < t1_ld(N); ++i) cosn[i] = sin1[i] = 0.0;
-    for (int i = 1; i < n; ++i) {
-        cosn[i - 1] = std::cos((pi * i) / n);   // EllipticSolver2d.cc:47-48
-        sin1[i - 1] = 2. * std::sin(pi * i / n);
-        ring[i - 1] = 2. * std::sin(pi * i * e / n);
-        ring[N + i - 1] = 2. * std::sin(pi * i * (e + n / 2) / n);
-    }
-}
-
+// (dst_tables.h fills the tables, in this order)
 static void plan_pointers(FftPlan& P, const double2* tw, const double2* t16, const double* reals) {
     P.tw = tw;
     P.tw16 = plan_has_tw16(P.M) ? t16 : nullptr;
@@ -295,7 +267,7 @@ static int get_plan(Ctx* c, int N, FftPlan* out) {
     // tw, t16 and the reals in one upload
     std::vector<double> h(2 * (size_t)P.M + 512 + plan_reals(N));
     double2 *tw = (double2*)h.data(), *t16 = tw + P.M;
-    plan_tables(P.M, tw, t16, (double*)(t16 + 256));
+    plan_tables(P.M, (double*)tw, (double*)t16, (double*)(t16 + 256));
     double* d = nullptr;
     CKR(c->mem.alloc(&d, h.size()));
     CK(hipMemcpy(d, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
@@ -3518,8 +3490,8 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     double* fin = (double*)(b + o_fin);
     std::lock_guard<std::mutex> lk(g_noalloc_mu);
     NoAllocStage& H = g_noalloc_stage;
-    plan_tables(pj.M, H.twj, H.t16j, H.realj);
-    plan_tables(pi.M, H.twi, H.t16i, H.reali);
+    plan_tables(pj.M, (double*)H.twj, (double*)H.t16j, H.realj);
+    plan_tables(pi.M, (double*)H.twi, (double*)H.t16i, H.reali);
     plan_pointers(pj, (const double2*)(b + o_twj), (const double2*)(b + o_t16j), (const double*)(b + o_rj));
     plan_pointers(pi, (const double2*)(b + o_twi), (const double2*)(b + o_t16i), (const double*)(b + o_ri));
     SolveSpec sp{};
