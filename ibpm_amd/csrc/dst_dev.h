@@ -1,31 +1,32 @@
-// dst_dev.h -- device pieces shared by the DST passes: complex arithmetic, the
-// small DFTs, getBC / getRHS at a point, and the workgroup order.
+// dst_dev.h -- device pieces shared by the DST passes: complex arithmetic and the
+// small DFTs (for the host too, where their error is measured), getBC / getRHS at
+// a point, and the workgroup order.
 #pragma once
 #include "ops.h"
 
 namespace ibpmg {
 
-__device__ inline double2 cmul(double2 a, double2 b) {
+__host__ __device__ inline double2 cmul(double2 a, double2 b) {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
-__device__ inline double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ inline double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__host__ __device__ inline double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__host__ __device__ inline double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 // -i * a
-__device__ inline double2 cmi(double2 a) { return make_double2(a.y, -a.x); }
+__host__ __device__ inline double2 cmi(double2 a) { return make_double2(a.y, -a.x); }
 // The same for the FP32 transforms (float2).
-__device__ inline float2 cmul(float2 a, float2 b) {
+__host__ __device__ inline float2 cmul(float2 a, float2 b) {
     return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
-__device__ inline float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ inline float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-__device__ inline float2 cmi(float2 a) { return make_float2(a.y, -a.x); }
+__host__ __device__ inline float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__host__ __device__ inline float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+__host__ __device__ inline float2 cmi(float2 a) { return make_float2(a.y, -a.x); }
 
 // Real type of a complex type, and a complex value from two reals.
 template <class C> struct RealOf;
 template <> struct RealOf<double2> { typedef double T; };
 template <> struct RealOf<float2> { typedef float T; };
 template <class C>
-__device__ inline C cpx(typename RealOf<C>::T x, typename RealOf<C>::T y) {
+__host__ __device__ inline C cpx(typename RealOf<C>::T x, typename RealOf<C>::T y) {
     C r;
     r.x = x;
     r.y = y;
@@ -38,7 +39,7 @@ typedef double DoublePair __attribute__((ext_vector_type(2), aligned(8)));
 // the same operations in the same order for both, constants rounded to the
 // type.
 template <int R, class C>
-__device__ inline void dft(C* v) {
+__host__ __device__ inline void dft(C* v) {
     typedef typename RealOf<C>::T T;
     if constexpr (R == 2) {
         C a = v[0], b = v[1];
@@ -99,7 +100,7 @@ __device__ inline void dft(C* v) {
 
 // 16-point DFT as 4 x 4: X[k1 + 4 k2] = sum_n2 W16^(n2 k1) W4^(n2 k2)
 // sum_n1 x[4 n1 + n2] W4^(n1 k1).
-__device__ inline double2 mul_w16(double2 a, int k) {   // a * exp(-2 pi i k / 16), k in {1,2,3,6,9}
+__host__ __device__ inline double2 mul_w16(double2 a, int k) {   // a * exp(-2 pi i k / 16), k in {1,2,3,6,9}
     const double c1 = 0.92387953251128675613;   // cos(pi / 8)
     const double s1 = 0.38268343236508977173;   // sin(pi / 8)
     const double h = 0.70710678118654752440;    // cos(pi / 4)
@@ -112,7 +113,7 @@ __device__ inline double2 mul_w16(double2 a, int k) {   // a * exp(-2 pi i k / 1
     }
 }
 
-__device__ inline void dft16(double2* v) {
+__host__ __device__ inline void dft16(double2* v) {
     double2 a[4][4];
 #pragma unroll
     for (int n2 = 0; n2 < 4; ++n2) {
@@ -137,7 +138,7 @@ __device__ inline void dft16(double2* v) {
 // Good-Thomas index maps): X[k] = Y[k mod R1][k mod R2], Y the 2-D DFT of
 // x[(R2 n1 + R1 n2) mod R].
 template <int R1, int R2>
-__device__ inline void dft_pfa(double2* v) {
+__host__ __device__ inline void dft_pfa(double2* v) {
     constexpr int R = R1 * R2;
     double2 a[R1][R2];
 #pragma unroll
@@ -160,7 +161,7 @@ __device__ inline void dft_pfa(double2* v) {
 }
 
 // 9-point DFT as 3 x 3, twiddles exp(-2 pi i {1, 2, 4} / 9).
-__device__ inline void dft9(double2* v) {
+__host__ __device__ inline void dft9(double2* v) {
     const double c1 = 0.76604444311897803520, s1 = 0.64278760968653932632;   // 2 pi / 9
     const double c2 = 0.17364817766693034885, s2 = 0.98480775301220805937;   // 4 pi / 9
     const double c4 = -0.93969262078590838405, s4 = 0.34202014332566873304;  // 8 pi / 9
@@ -186,7 +187,7 @@ __device__ inline void dft9(double2* v) {
 
 // DFT of any radix of the compiled FP64 passes.
 template <int R>
-__device__ inline void dft_any(double2* v) {
+__host__ __device__ inline void dft_any(double2* v) {
     if constexpr (R == 6) dft_pfa<2, 3>(v);
     else if constexpr (R == 9) dft9(v);
     else if constexpr (R == 10) dft_pfa<2, 5>(v);

@@ -94,6 +94,35 @@ constexpr Radices radices(int M) {
     return q;
 }
 
+// A butterfly's twiddles w^r, r < R, of stage s >= 1: products of w^1 alone, whose
+// rounding then grows with r (w^7 carries seven times that of w^1), or of the
+// loaded w^1, w^2, w^4, w^8.  Loading costs more than the products: everywhere, the
+// flux at 1000 x 600 x 5 levels takes 212 instead of 188 us, ten steps at 400^2 x 4
+// 10.7 instead of 10.0 ms.  So it is done only where the products leave a larger
+// error than radices 8, 4, 2, 5, 3 from rounded angles had: in transforms of two
+// stages, whose one twiddled stage is half of the work (6 to 36 cells), and at
+// radices 9 and 10.  Error relative to those at 6, 8, 12, 15, 20, 25, 32, 36, 125,
+// 225, 324, 405 cells: 1.16, 1.24, 1.06, 1.08, 1.09, 1.28, 1.08, 1.04, 1.04, 1.04,
+// 1.05, 1.13 from w^1 alone; now 0.95, 0.91, 0.86, 0.73, 0.76, 0.68, 0.67, 0.73,
+// 0.76, 0.74, 0.89, 0.68, and no length above 1.
+constexpr int twiddle_loads(const Radices& q, int s) {
+    if (q.n != 2 && q.r[s] <= 8) return 1;
+    int n = 0;
+    for (int p = 1; p < q.r[s]; p *= 2) ++n;
+    return n;
+}
+// w[1..R-1] from the N loaded powers.
+template <int R, int N>
+__host__ __device__ __forceinline__ void twiddle_powers(const double2* loaded, double2* w) {
+#pragma unroll
+    for (int p = 0; p < N; ++p) w[1 << p] = loaded[p];
+#pragma unroll
+    for (int r = 2; r < R; ++r) {
+        const int h = N == 1 ? r - r / 2 : r < 4 ? 2 : r < 8 ? 4 : 8;   // else the highest loaded power
+        if (r != h) w[r] = cmul(w[r - h], w[h]);
+    }
+}
+
 // FFT of length M in a workgroup of BT threads; element e of a stage is LDS slot
 // e + e / R1 (a pad after every R1 elements where R1 is even, so that the first
 // stage's writes, R1 apart, spread over the banks).
@@ -108,24 +137,27 @@ struct LdsFft {
         return p;
     }
     static constexpr int rounds(int s) { return (M / Q.r[s] + BT - 1) / BT; }
+    static constexpr int loads(int s) { return twiddle_loads(Q, s); }
     static constexpr int first_tw(int s) {
         int p = 0;
-        for (int k = 1; k < s; ++k) p += rounds(k);
+        for (int k = 1; k < s; ++k) p += rounds(k) * loads(k);
         return p;
     }
     static constexpr int kTw = first_tw(Q.n);
-    // w^(jm M / (Ns R)) of every butterfly this thread takes in stages 1..
+    // the loaded powers of w^(jm M / (Ns R)) of every butterfly this thread takes in stages 1..
     double2 tw[kTw > 0 ? kTw : 1];
 
     template <int S = 1>
     __device__ __forceinline__ void load_twiddles(const IBPM_GLOBAL double* g) {
         if constexpr (S < Q.n) {
-            constexpr int Ns = ns(S), R = Q.r[S], step = M / (Ns * R);
+            constexpr int Ns = ns(S), R = Q.r[S], step = M / (Ns * R), n = loads(S), at = first_tw(S);
 #pragma unroll
             for (int b = 0; b < rounds(S); ++b) {
                 const int j = (int)(threadIdx.x + b * BT) % (M / R);
                 const int k = j % Ns * step;
-                tw[first_tw(S) + b] = make_double2(g[2 * k], g[2 * k + 1]);
+#pragma unroll
+                for (int p = 0; p < n; ++p)
+                    tw[at + b * n + p] = make_double2(g[2 * (k << p)], g[2 * (k << p) + 1]);
             }
             load_twiddles<S + 1>(g);
         }
@@ -134,7 +166,7 @@ struct LdsFft {
     // Stage S: v[b][r] is set (stage 0 by load, later stages from LDS).
     template <int S, bool WAIT, class Emit>
     __device__ __forceinline__ void stages(double2* lds, const Emit& emit) {
-        constexpr int R = Q.r[S], MR = M / R;
+        constexpr int R = Q.r[S], MR = M / R, n = loads(S), at = first_tw(S);
         double2 v[rounds(S)][R];
 #pragma unroll
         for (int b = 0; b < rounds(S); ++b) {
@@ -143,9 +175,7 @@ struct LdsFft {
             const double2* in = lds + j + j / R1 * PAD;
             constexpr int step = MR + MR / R1 * PAD;   // MR is a multiple of R1 from stage 1 on
             double2 w[R];
-            w[1] = tw[first_tw(S) + b];
-#pragma unroll
-            for (int r = 2; r < R; ++r) w[r] = cmul(w[r / 2], w[r - r / 2]);
+            twiddle_powers<R, n>(tw + at + b * n, w);
             v[b][0] = in[0];
 #pragma unroll
             for (int r = 1; r < R; ++r) v[b][r] = cmul(in[r * step], w[r]);
