@@ -3434,17 +3434,19 @@ int ibpm_elliptic_solve_precision(ibpm_ctx* c, int kind, int nx, int ny, int ngr
 }
 
 // ibpm_elliptic_solve_noalloc: the multi-domain solve of ibpm_elliptic_solve
-// with every buffer of its own (right-hand-side copy, coarsify buffer,
-// transpose buffers, cosine and twiddle tables, job descriptors) carved from
-// the device's fixed scratch array instead of allocated.  The host values of
-// the tables and descriptors are staged in static memory under a lock, which
-// is held until the stream has drained.
+// with every buffer of its own (right-hand-side copy, coarsify buffer, scratch
+// rows, boundary values, tables, job descriptors) carved from the device's fixed
+// scratch array instead of allocated.  The host values of the tables and
+// descriptors are staged in static memory under a lock, which is held until the
+// stream has drained, and go up in one copy (eight took 40 to 50 us of a call).
 static constexpr int kNoAllocMaxLevels = 16;
+// tables of a plan (FFT length M, N unknowns): tw, t16 where there is one, reals
+static size_t noalloc_t16(int M) { return plan_has_tw16(M) ? 512 : 0; }
+static size_t noalloc_tables(const FftPlan& P) { return 8 * (2 * (size_t)P.M + noalloc_t16(P.M) + plan_reals(P.N)); }
+static constexpr size_t kNoAllocStage = 2 * 8 * (4 * (size_t)kFftLds + 1024) +
+                                        kNoAllocMaxLevels * (sizeof(EllJob) + sizeof(CoarsifyJob)) + 4 * 256;
 struct NoAllocStage {
-    double2 twj[kFftLds], t16j[256], twi[kFftLds], t16i[256];
-    double realj[2 * kFftLds + 16], reali[2 * kFftLds + 16];   // plan_reals of the longest plan
-    EllJob ej[kNoAllocMaxLevels];
-    CoarsifyJob cj[kNoAllocMaxLevels];
+    alignas(256) char bytes[kNoAllocStage];
 };
 static std::mutex g_noalloc_mu;
 static NoAllocStage g_noalloc_stage;
@@ -3464,21 +3466,22 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     const int L = ngrid;
     const long ns = (long)(nx - 1) * (ny - 1);
     size_t off = 0;
-    auto take = [&](size_t bytes) { const size_t o = off; off += (bytes + 255) & ~size_t(255); return o; };
+    auto padded = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
+    auto take = [&](size_t bytes) { const size_t o = off; off += padded(bytes); return o; };
     const size_t o_fin = take(8 * ns * L), o_R = take(8 * ns * L);
     const size_t o_T1 = take(8 * (size_t)(nx - 1) * t1_ld(ny - 1));
     const size_t zero_lo = o_R, zero_hi = off;   // R and T start at zero, as freshly allocated ones
     const size_t rows_end = off;
     const size_t o_bcv = take(8 * bcv_size(nx, ny) * L);
-    const size_t o_rj = take(8 * plan_reals(pj.N)), o_ri = take(8 * plan_reals(pi.N));
-    // the accepted sizes are those of 16 bytes of scratch rows per point; only
-    // small grids need more than that for the boundary values and tables
-    off = std::max(off, rows_end + ((8 * (size_t)(ny - 1) * t1_ld(nx - 1) + 255) & ~size_t(255)));
-    (void)take(8 * (size_t)(nx - 1));
-    (void)take(8 * (size_t)(ny - 1));
-    const size_t o_twj = take(16 * (size_t)pj.M), o_t16j = take(16 * 256);
-    const size_t o_twi = take(16 * (size_t)pi.M), o_t16i = take(16 * 256);
+    const size_t o_stage = off;   // what the host fills, in this order
+    const size_t o_tj = take(noalloc_tables(pj)), o_ti = take(noalloc_tables(pi));
     const size_t o_ej = take(sizeof(EllJob) * L), o_cj = take(sizeof(CoarsifyJob) * L);
+    const size_t stage_bytes = off - o_stage;
+    // the accepted sizes are those of 16 bytes of scratch rows per point, cosine and
+    // twiddle tables and the descriptors; only small grids need more
+    off = std::max(off, rows_end + padded(8 * (size_t)(ny - 1) * t1_ld(nx - 1)) + padded(8 * (size_t)(nx - 1)) +
+                            padded(8 * (size_t)(ny - 1)) + padded(16 * (size_t)pj.M) + padded(16 * (size_t)pi.M) +
+                            2 * 16 * 256 + padded(sizeof(EllJob) * L) + padded(sizeof(CoarsifyJob) * L));
     if (off > kScratchBytes) {
         set_error("ibpm_elliptic_solve_noalloc: a %dx%d grid of %d levels needs %zu bytes of scratch; "
                   "the fixed scratch holds %zu", nx, ny, ngrid, off, kScratchBytes);
@@ -3489,40 +3492,40 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* c, int kind, int nx, int ny, int ngrid
     char* b = (char*)base;
     double* fin = (double*)(b + o_fin);
     std::lock_guard<std::mutex> lk(g_noalloc_mu);
-    NoAllocStage& H = g_noalloc_stage;
-    plan_tables(pj.M, (double*)H.twj, (double*)H.t16j, H.realj);
-    plan_tables(pi.M, (double*)H.twi, (double*)H.t16i, H.reali);
-    plan_pointers(pj, (const double2*)(b + o_twj), (const double2*)(b + o_t16j), (const double*)(b + o_rj));
-    plan_pointers(pi, (const double2*)(b + o_twi), (const double2*)(b + o_t16i), (const double*)(b + o_ri));
+    char* const h = g_noalloc_stage.bytes;
+    if (stage_bytes > kNoAllocStage) { set_error("ibpm_elliptic_solve_noalloc: staging too small"); return -2; }
+    auto tables = [&](FftPlan& P, size_t o) {
+        double* t = (double*)(h + (o - o_stage));
+        plan_tables(P.M, t, t + 2 * P.M, t + 2 * P.M + noalloc_t16(P.M));
+        const double* d = (const double*)(b + o);
+        plan_pointers(P, (const double2*)d, (const double2*)(d + 2 * P.M), d + 2 * P.M + noalloc_t16(P.M));
+    };
+    tables(pj, o_tj);
+    tables(pi, o_ti);
+    EllJob* ej = (EllJob*)(h + (o_ej - o_stage));
+    CoarsifyJob* cj = (CoarsifyJob*)(h + (o_cj - o_stage));
     SolveSpec sp{};
     sp.nx = nx; sp.ny = ny; sp.L = L; sp.dx = dx; sp.kind = kind; sp.alpha = alpha;
     sp.f = fin; sp.u = d_u; sp.R = (double*)(b + o_R); sp.T1 = (double*)(b + o_T1);
     sp.in_scale = 1.0; sp.epilogue = 0;
     sp.bcv = (double*)(b + o_bcv);
     for (int st = 0; st < L; ++st) {   // coarsest level first
-        H.ej[st] = EllJob{};
-        fill_ell_job(sp, L - 1 - st, H.ej[st]);
-        H.ej[st].pj = pj;
-        H.ej[st].pi = pi;
+        ej[st] = EllJob{};
+        fill_ell_job(sp, L - 1 - st, ej[st]);
+        ej[st].pj = pj;
+        ej[st].pi = pi;
     }
-    for (int lev = 1; lev < L; ++lev) H.cj[lev - 1] = CoarsifyJob{nx, ny, lev, sp.f, sp.R, nullptr};
+    for (int lev = 1; lev < L; ++lev) cj[lev - 1] = CoarsifyJob{nx, ny, lev, sp.f, sp.R, nullptr};
     hipStream_t s = c->c.stream;
     EllJob* d_ej = (EllJob*)(b + o_ej);
     CoarsifyJob* d_cj = (CoarsifyJob*)(b + o_cj);
     CK(hipMemsetAsync(b + zero_lo, 0, zero_hi - zero_lo, s));
     CK(hipMemcpyAsync(fin, d_f, 8 * ns * L, hipMemcpyDeviceToDevice, s));
-    CK(hipMemcpyAsync(b + o_rj, H.realj, 8 * plan_reals(pj.N), hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(b + o_ri, H.reali, 8 * plan_reals(pi.N), hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(b + o_twj, H.twj, 16 * (size_t)pj.M, hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(b + o_t16j, H.t16j, 16 * 256, hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(b + o_twi, H.twi, 16 * (size_t)pi.M, hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(b + o_t16i, H.t16i, 16 * 256, hipMemcpyHostToDevice, s));
-    CK(hipMemcpyAsync(d_ej, H.ej, sizeof(EllJob) * L, hipMemcpyHostToDevice, s));
-    if (L > 1) CK(hipMemcpyAsync(d_cj, H.cj, sizeof(CoarsifyJob) * (L - 1), hipMemcpyHostToDevice, s));
+    CK(hipMemcpyAsync(b + o_stage, h, stage_bytes, hipMemcpyHostToDevice, s));
     for (int lev = 1; lev < L; ++lev) launch_coarsify(d_cj + (lev - 1), 1, nx / 2 - 1, s, false);
     for (int st = 0; st < L; ++st)   // one level's scratch rows: level by level
         for (int pass : {1, 2, 4, 3}) {
-            const EllJob& J = H.ej[st];
+            const EllJob& J = ej[st];
             if (pass == 4 && !J.bc_out) continue;
             const int M = pass == 2 ? pi.M : pj.M;
             const bool regs = pass != 4 && pass_in_registers(M, (pass == 2 ? ny : nx) / 2);

@@ -16,6 +16,8 @@ static int pending = 0;   /* launches and copies since the last synchronisation 
 void fake_fail(const char* name, int skip) { fail_name = strdup(name); fail_skip = skip; }
 int fake_failed(void) { return !*fail_name; }
 int fake_pending(void) { return pending; }
+static int uploads = 0;
+int fake_uploads(void) { const int n = uploads; uploads = 0; return n; }   /* host to device copies since the last call */
 
 static Err fails(const char* name, Err e) {
     if (strcmp(name, fail_name) || fail_skip-- > 0) return OK;
@@ -40,8 +42,9 @@ Err hipMemset(void* p, int v, size_t n) { memset(p, v, n); return OK; }
 Err hipMemsetAsync(void* p, int v, size_t n, void* s) { (void)s; memset(p, v, n); ++pending; return OK; }
 Err hipMemcpy(void* d, const void* h, size_t n, int k) { (void)k; memmove(d, h, n); return OK; }
 Err hipMemcpyAsync(void* d, const void* h, size_t n, int k, void* s) {
-    (void)k; (void)s;
+    (void)s;
     MAY_FAIL(INVALID);
+    uploads += k == 1;
     memmove(d, h, n);
     ++pending;
     return OK;
