@@ -191,10 +191,6 @@ __host__ __device__ inline void dft_any(double2* v) {
     if constexpr (R == 6) dft_pfa<2, 3>(v);
     else if constexpr (R == 9) dft9(v);
     else if constexpr (R == 10) dft_pfa<2, 5>(v);
-    else if constexpr (R == 12) dft_pfa<4, 3>(v);
-    else if constexpr (R == 15) dft_pfa<3, 5>(v);
-    else if constexpr (R == 16) dft16(v);
-    else if constexpr (R == 20) dft_pfa<4, 5>(v);
     else dft<R>(v);
 }
 

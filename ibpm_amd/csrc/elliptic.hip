@@ -85,7 +85,7 @@ constexpr bool kSwizzleAll = CM >= 2048;
 // LDS; inputs are staged through registers so the stage runs in place.
 // Twiddles come from the LDS table (see twiddle()).  Template
 // arguments that are 0 are taken from the runtime values.
-template <int R, int CM, int CNP, int CNS, bool SWIN = false, bool SWOUT = false, class C = double2>
+template <int R, int CM, int CNP, int CNS, bool SWIN, bool SWOUT, class C>
 __device__ inline void fft_stage(C* buf, const C* tw, int Mr, int npr, int Nsr) {
     const int M = CM ? CM : Mr;
     const int np = CM ? CNP : npr;

@@ -311,12 +311,11 @@ struct SolveSpec {
 // fs_*: the DST passes and coarsify of the M applications inside the force
 // solve (kernels k_fs_*), counted with the bytes of the flows still iterating.
 // ell32_* / fs32_*: the same passes with FP32 transforms (precision modes).
-enum KClass { K_PASS1, K_PASS2, K_PASS3, K_COARSIFY, K_VEL, K_CROSS, K_RHS, K_CURLQ, K_INTERP,
+enum KClass { K_PASS1, K_PASS2, K_PASS3, K_COARSIFY, K_RHS, K_CURLQ, K_INTERP,
               K_SMEAR, K_MINV, K_CG, K_FORCES, K_CLEAR, K_FSPASS1, K_FSPASS2, K_FSPASS3, K_FSCOARSIFY,
               K_FSHELM, K_HELM, K_PASS32_1, K_PASS32_2, K_PASS32_3, K_FSPASS32_1, K_FSPASS32_2,
               K_FSPASS32_3, K_GEMM, K_PCASM, K_PCNS, K_BC, K_FSBC, K_NCLASS };
-static const char* kclass_names[K_NCLASS] = {"ell_pass1", "ell_pass2", "ell_pass3", "coarsify", "vel",
-                                             "cross", "rhs", "curl_q", "interp", "smear_curl", "minv",
+static const char* kclass_names[K_NCLASS] = {"ell_pass1", "ell_pass2", "ell_pass3", "coarsify", "rhs", "curl_q", "interp", "smear_curl", "minv",
                                              "cg", "forces", "clear_nodes", "fs_pass1", "fs_pass2",
                                              "fs_pass3", "fs_coarsify", "fs_helm", "helm", "ell32_pass1",
                                              "ell32_pass2", "ell32_pass3", "fs32_pass1", "fs32_pass2",

@@ -150,30 +150,13 @@ __device__ inline double yvel(const Lay& g, const Q& q, double dx0, int lev, int
 //   linear and periodic models, LinearizedIBSolver::N (IBSolver.cc:211-216):
 //     CrossProduct(q0, omega) + CrossProduct(q, omega0), summed per node
 //   adjoint, AdjointIBSolver::N (IBSolver.cc:218-222): -CrossProduct(q, omega0),
-//     so that k_rhs's Curl(cross) is the subtracted term
+//     so that rhs_node's Curl(cross) is the subtracted term
 __device__ inline double cross_node(int model, double sign, double v, double w, double v0, double w0) {
     if (model == 1 || model == 3) return sign * (v0 * w) + sign * (v * w0);
     if (model == 2) return -sign * (v * w0);
     return sign * (v * w);
 }
 __device__ inline bool has_base(int model) { return model >= 1 && model <= 3; }
-
-template <class Q>
-__device__ inline double node_u(const FlowOps& F, const Lay& g, const Q& q, int lev, int i, int j) {
-    const long k = g.s(lev, i, j);
-    const double v = xvel(g, q, F.dx, lev, i, j), w = gin(F.omega)[k];
-    if (!has_base(F.model)) return cross_node(F.model, -1.0, v, w, 0.0, 0.0);
-    const double v0 = F.model == 2 ? 0.0 : xvel(g, FluxField{g, F.q0b}, F.dx, lev, i, j);
-    return cross_node(F.model, -1.0, v, w, v0, gin(F.w0b)[k]);
-}
-template <class Q>
-__device__ inline double node_v(const FlowOps& F, const Lay& g, const Q& q, int lev, int i, int j) {
-    const long k = g.s(lev, i, j);
-    const double v = yvel(g, q, F.dx, lev, i, j), w = gin(F.omega)[k];
-    if (!has_base(F.model)) return cross_node(F.model, 1.0, v, w, 0.0, 0.0);
-    const double v0 = F.model == 2 ? 0.0 : yvel(g, FluxField{g, F.q0b}, F.dx, lev, i, j);
-    return cross_node(F.model, 1.0, v, w, v0, gin(F.w0b)[k]);
-}
 
 // XVelocityToFlux / YVelocityToFlux at one flux of level lev
 // (VectorOperations.cc:669-915) outside the coarse levels' region G, where the
@@ -231,7 +214,7 @@ __device__ inline double yflux_from(const Lay& g, const S& s, double dx0, int le
 
 // ------------------------------------------------------------- kernels
 // U = -omega * FluxToX(q), V = omega * FluxToY(q) on every level
-// (CrossProduct, VectorOperations.cc:438-457).
+// (CrossProduct, VectorOperations.cc:438-457), for the stand-alone entry points.
 __global__ void __launch_bounds__(kThreads) k_vel(const FlowOps* __restrict__ flows) {
     const FlowOps& F = flows[blockIdx.y];
     const Lay g{F.nx, F.ny, F.L};
@@ -248,9 +231,10 @@ __global__ void __launch_bounds__(kThreads) k_vel(const FlowOps* __restrict__ fl
         j < g.ny / 2 + nx_ext(g.ny))
         return;
     const FluxField q{g, F.q};
-    const double u = node_u(F, g, q, lev, i, j), v = node_v(F, g, q, lev, i, j);
-    gout(F.U)[t] = u;
-    gout(F.V)[t] = v;
+    const double w = gin(F.omega)[t];
+    const double u = xvel(g, q, F.dx, lev, i, j), v = yvel(g, q, F.dx, lev, i, j);
+    gout(F.U)[t] = -u * w;
+    gout(F.V)[t] = v * w;
 }
 
 // CrossProduct(Flux, Flux) -> Scalar before its coarsify (VectorOperations.cc
@@ -449,7 +433,7 @@ __global__ void __launch_bounds__(kThreads) k_rhs(const FlowOps* __restrict__ fl
 // grid, nearly all of it latency.  (advect.h has the index rules.)
 
 // U (u) or V of the cross product at a node, from psi and the base flow of the
-// last refresh (FlowOps::bf[3..5]), as node_u and node_v give it from q, with
+// last refresh (FlowOps::bf[3..5]), as xvel, yvel and cross_node give it from q, with
 // every load issued before any is used: the node velocity as a sum of at most
 // four fluxes (the rules of xvel and yvel), each a difference of two psi values.
 __device__ inline double node_value(const FlowOps& F, const Lay& g, const NodeTerm& t) {
