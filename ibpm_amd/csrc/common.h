@@ -26,18 +26,18 @@ constexpr int kThreads = 256;          // workgroup size of the stencil kernels 
 #ifndef IBPM_FFT_NP_MAX
 #define IBPM_FFT_NP_MAX 1
 #endif
-constexpr int kFftThreads = IBPM_FFT_THREADS;   // workgroup size of the DST passes
-constexpr int kFftNpMax = IBPM_FFT_NP_MAX;      // most row pairs per DST workgroup
-constexpr int kFftLds = 2048;          // complex doubles staged in LDS per DST block (32 KB)
+constexpr int kFftThreads = IBPM_FFT_THREADS;   // workgroup size of the FP32 DST passes
+constexpr int kFftNpMax = IBPM_FFT_NP_MAX;      // most row pairs per workgroup of theirs
+constexpr int kFftLds = 2048;          // longest transform of a plan; complex values of one in LDS
 constexpr int kMaxStages = 16;
 
 // Plan of one complex FFT of length M = 2(N+1) used for a DST-I of length N.
 struct FftPlan {
     int N;          // DST length
     int M;          // FFT length
-    int np;         // row pairs per workgroup (np * M <= kFftLds)
-    int nst;        // number of Stockham stages
-    int rad[kMaxStages];
+    int np;         // FP32 passes: row pairs per workgroup (np * M <= kFftLds),
+    int nst;        // number of Stockham stages,
+    int rad[kMaxStages];   // their radices
     const double2* tw;   // tw[k] = exp(-2 pi i k / M), k < M
     // tables of n = N + 1 cells: cos(pi i / n) and 2 sin(pi i / n), i = 1..n-1
     // (then zeros to t1_ld(N)), and 2 sin(pi l j / n) at j = n/4 and n/4 + n/2,

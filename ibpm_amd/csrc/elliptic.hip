@@ -1,34 +1,39 @@
-// elliptic.hip -- batched multi-domain DST-I Poisson/Helmholtz solves (FP64).
+// elliptic.hip -- batched multi-domain DST-I Poisson/Helmholtz solves.
 //
 // Replaces EllipticSolver2d::solve (reference EllipticSolver2d.cc:57-185) and
 // the multi-domain driver EllipticSolver::solve (EllipticSolver.cc:47-73).
 //
 // One level solve u = S diag(e) S f * norm (S = DST-I matrix) is three passes,
 // each reading and writing the level once (6 words per grid point):
-//   pass 1: rows of the right-hand side (coarsify select, sign, boundary-value
-//           correction of getRHS fused in) -> DST along j -> rows of T
-//   pass 2: columns of T, two neighbouring ones a pair -> DST along i ->
-//           eigenvalue scaling -> DST along i -> the same columns of T
+//   pass 1: rows of the right-hand side (coarsify select and sign fused in) ->
+//           DST along j -> rows of T
+//   pass 2: columns of T, two neighbouring ones a pair, plus the boundary values'
+//           share (getRHS) -> DST along i -> eigenvalue scaling -> DST along i ->
+//           the same columns of T
 //   pass 3: rows of T -> DST along j -> * 1/(4 nx ny) -> u (or u = W - .)
 // T keeps the level's (i, j) layout throughout, so passes 1 and 3 read and
 // write whole rows and pass 2 works in place.
 // Each DST-I of length N is the imaginary part of a complex FFT of length
 // M = 2(N+1) of the odd extension; two rows share one FFT (real part row a,
-// imaginary part row b).  M = 1024 and 2048 use a radix 16 x 16 x M/256
-// transform held in registers (exchanges through LDS); the other lengths a
-// mixed-radix (2,3,4,5) Stockham transform held in LDS, with each stage
-// staged through registers so one LDS buffer suffices.  Passes may run over
-// part of a level when only part of the result is read (EllJob's partial-pass
-// fields).  The file also holds the coarsify chain and the local Jacobi solves
-// of the force solve's A^-1 (k_fs_helm).
+// imaginary part row b).  The FP64 passes are compiled per length in
+// dst_passes.h, through LDS; here are those of M = 1024 and 2048 as a radix
+// 16 x 16 x M/256 transform held in registers (exchanges through LDS), and the FP32
+// passes: a mixed-radix (2, 3, 4, 5, 8) Stockham transform held in LDS, each
+// stage staged through registers so that one buffer suffices, with lengths that
+// have no compiled plan read from a plan at run time, and the boundary values in
+// pass 1, level by level.  Passes may run over part of a level when only part of
+// the result is read (EllJob's partial-pass fields; not the FP32 ones).  The file
+// also holds the coarsify chain and the local Jacobi solves of the force solve's
+// A^-1 (k_fs_helm).
 #include "dst_passes.h"
 
 #include <algorithm>
 
 namespace ibpmg {
 
-// FFT lengths with a compiled plan (M = 2(N+1) for N = 199, 255, 383, 399,
-// 511, 1023: the configured grids); any other length uses the runtime plan.
+// FFT lengths whose FP32 passes have a compiled plan (M = 2(N+1) for N = 199, 255,
+// 383, 399, 511, 1023: the configured grids); any other length uses the runtime
+// plan.
 __host__ __device__ constexpr bool compiled_len(int M) {
     return M == 400 || M == 512 || M == 768 || M == 800 || M == 1024 || M == 2048;
 }
@@ -190,7 +195,12 @@ __device__ inline void fft_any(C* buf, const C* tw, const FftPlan& P) {
 // A launch at M = 1024 runs only a quarter wave per CU when it holds few rows
 // (one 511-row level: 256 workgroups of one wave), where the LDS passes'
 // larger workgroups hide latency better; it takes the register-held
-// transform from kRegMinPairs row pairs on.  M = 2048 always takes it.
+// transform from kRegMinPairs row pairs on.  The pairs are those of one level,
+// summed over the flows that share its length, as they were when a launch was
+// one level: a small batch's passes 1 and 3 over all levels at once hold more (five
+// levels of one 512^2 flow: 1280 pairs) and stay with the LDS passes, as its pass 2
+// does.  The line has not been measured again for those launches.  M = 2048
+// always takes the register-held transform.
 constexpr long kRegMinPairs = 1024;
 
 // Row pairs per workgroup of the register-held passes: pass 2 reads and writes
@@ -348,7 +358,7 @@ __device__ __forceinline__ void fft_regs(double2* v, double* bd, int t, const IB
     }
 }
 
-// The three passes are written once over a template length CM (0: runtime
+// The FP32 passes are written once over a template length CM (0: runtime
 // plan).  Row length N, FFT length M and rows per block follow from the plan,
 // so with CM != 0 every index computation folds to constants.
 template <int CM, class C>
@@ -359,9 +369,8 @@ __device__ inline void load_twiddles(C* tw, const FftPlan& P) {
     for (int k = threadIdx.x; k < M; k += kFftThreads) tw[k] = cpx<C>(T(g[2 * k]), T(g[2 * k + 1]));
 }
 
-// The LDS passes are also instanced over C = float2: FP32 transforms and
-// scratch T, with the right-hand side, boundary terms, eigenvalue
-// scaling and output in FP64.
+// Instanced over C = float2: FP32 transforms and scratch T, with the right-hand
+// side, boundary terms, eigenvalue scaling and output in FP64.
 template <int CM, class C>
 __device__ __forceinline__ void pass1_lds(const EllJob& J, C* smem, int bx) {
     typedef typename RealOf<C>::T T;
@@ -518,8 +527,8 @@ __device__ __forceinline__ void pass3_lds(const EllJob& J, C* smem, int bx) {
     }
 }
 
-// The three passes for M = 1024, 2048 (N = M/2 - 1), the same arithmetic as the
-// LDS passes above around a register-held transform.  Passes 1 and 3 run one
+// The three passes for M = 1024, 2048 (N = M/2 - 1), the same arithmetic as those
+// of dst_passes.h around a register-held transform.  Passes 1 and 3 run one
 // row pair per workgroup of T = M/16 threads, pass 2 G = r16_group(2) column
 // pairs (see pass2_r16).
 

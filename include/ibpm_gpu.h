@@ -62,11 +62,11 @@ int ibpm_elliptic_solve(ibpm_ctx* ctx, int kind, int nx, int ny, int ngrid, doub
 /* The multi-domain solve of ibpm_elliptic_solve without any allocation.  No
    counterpart in the reference: it is for callers that cannot allocate device
    memory (code under HIP graph capture, tight serving loops, harnesses that
-   forbid hipMalloc).  Its own buffers (right-hand-side copy, coarsify and
-   transpose buffers, tables, job descriptors) live in a fixed 32 MiB device
+   forbid hipMalloc).  Its own buffers (right-hand-side copy, coarsify buffer,
+   scratch rows, tables, job descriptors) live in a fixed 32 MiB device
    array that every GPU the library runs on holds until the process ends; a
    grid needs 16 (nx-1)(ny-1) ngrid bytes plus about 16 (nx-1)(ny-1) for the
-   transposes, so e.g. 512 x 512 with 5 levels fits and 1024 x 1024 with 6 does
+   scratch rows, so e.g. 512 x 512 with 5 levels fits and 1024 x 1024 with 6 does
    not: sizes beyond the array, or more than 16 levels, return -2 with a
    message.  The caller passes d_f and d_u (which may alias).  Calls on one GPU
    share its array, so calls that overlap on one GPU (other threads, other
@@ -76,7 +76,7 @@ int ibpm_elliptic_solve_noalloc(ibpm_ctx* ctx, int kind, int nx, int ny, int ngr
 
 /* ibpm_elliptic_solve with a choice of transform precision: 0 FP64 (the
    reference's arithmetic; ibpm_elliptic_solve), 1 FP32 transforms and
-   transposed intermediates with the right-hand side, boundary terms,
+   scratch rows with the right-hand side, boundary terms,
    eigenvalue scaling and output in FP64.  No counterpart in the reference
    (whose solve is FP64 FFTW, src/EllipticSolver2d.cc:57-104); for measuring
    the reduced-precision path's error per solve.  2: the split-BF16 GEMM-DST
@@ -384,7 +384,7 @@ int ibpm_batch_set_local_helmholtz(ibpm_batch* b, int on);
 /* Transform precision of the batch's elliptic solves (no counterpart in the
    reference, whose solves are FP64): 0 (the default) FP64 everywhere; 1 the
    step's own solves (A^-1 a, L^-1 omega*, A^-1 c, the refresh's L^-1) run FP32
-   transforms and transposed intermediates, with FP64 right-hand sides, boundary
+   transforms and scratch rows, with FP64 right-hand sides, boundary
    terms, eigenvalue scaling and fields, so omega, psi and q stay FP64; 2 also
    the solves inside the force solve's M applications (CG's vectors, its
    residual test and the Cholesky factor stay FP64).  Each reduced-precision
